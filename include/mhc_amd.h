@@ -444,6 +444,42 @@ int mhc_sinkhorn_bwd_max_iters(int n);
 int mhc_sinkhorn_bwd(const void* m_in, int in_dtype, const void* g_out, int g_dtype, void* g_in,
                      int gi_dtype, int64_t batch, int n, int iters, float eps, hipStream_t stream);
 
+/* ------------------------------------------------- attention (inference)
+ * The model's attention layer between its projections
+ * (model/model_minimind.py:180-245): 16-bit tensors (bf16 or fp16) of one
+ * dtype, head_dim 64, 96 or 128, heads a multiple of kv_heads.  All data
+ * pointers are 16-byte aligned.
+ */
+
+/* Causal attention over a sequence's own positions.  q [B, T, heads *
+ * head_dim], k, v [B, T, kv_heads * head_dim]: the raw projections; q and k get
+ * their per-head RMSNorm (gains [head_dim]) and the rotary embedding (cos, sin
+ * [T, head_dim]).  k_out: the normed and rotated k (the cache's content); out
+ * [B, T, heads * head_dim]. */
+int mhc_attn_prefill_fwd(const void* q, const void* k, const void* v, const void* q_gain,
+                         const void* k_gain, const void* cos, const void* sin, void* k_out,
+                         void* out, int64_t B, int T, int heads, int kv_heads, int head_dim,
+                         int dtype, float q_eps, float k_eps, hipStream_t stream);
+
+/* Bytes of workspace mhc_attn_decode_fwd needs (0: none), or -1 for a shape it
+ * does not take (heads / kv_heads > 4, another head_dim, S < 1). */
+int64_t mhc_attn_decode_workspace_bytes(int64_t B, int S, int heads, int kv_heads, int head_dim);
+
+/* One decode step.  q, k, v: the raw projections of one new token per sequence
+ * ([B, heads * head_dim], [B, kv_heads * head_dim]); normed and rotated here
+ * (cos, sin [head_dim] of the new position).  k_past, v_past: S cached
+ * positions [B, S, kv_heads, head_dim], head elements contiguous, the other
+ * strides given in elements (multiples of 8).  out [B, heads * head_dim].
+ * k_out, v_out (both or neither): the caches grown by the new position,
+ * contiguous [B, S + 1, kv_heads, head_dim]. */
+int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void* q_gain,
+                        const void* k_gain, const void* cos, const void* sin, const void* k_past,
+                        int64_t k_stride_b, int64_t k_stride_s, int64_t k_stride_h,
+                        const void* v_past, int64_t v_stride_b, int64_t v_stride_s,
+                        int64_t v_stride_h, void* k_out, void* v_out, void* out, void* workspace,
+                        int64_t workspace_bytes, int64_t B, int S, int heads, int kv_heads,
+                        int head_dim, int dtype, float q_eps, float k_eps, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -628,4 +628,78 @@ int mhc_sinkhorn_bwd(const void* m_in, int in_dtype, const void* g_out, int g_dt
                                              iters, eps, stream), fn);
 }
 
+// ------------------------------------------------------ attention (inference)
+
+static int check_attn(int64_t rows, int heads, int kv_heads, int head_dim, int dtype, const char* fn) {
+  if (rows < 0 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0)
+    return fail(hipErrorInvalidValue, "%s: bad shape (rows=%lld heads=%d kv_heads=%d)", fn, (long long)rows, heads, kv_heads);
+  if (head_dim != 64 && head_dim != 96 && head_dim != 128)
+    return fail(hipErrorInvalidValue, "%s: head_dim must be 64, 96 or 128 (got %d)", fn, head_dim);
+  if (dtype != mhc::kBF16 && dtype != mhc::kF16) return fail(hipErrorInvalidValue, "%s: dtype must be bf16 or fp16 (got %d)", fn, dtype);
+  if (rows * heads * head_dim > (int64_t(1) << 38)) return fail(hipErrorInvalidValue, "%s: too large", fn);
+  return 0;
+}
+
+int mhc_attn_prefill_fwd(const void* q, const void* k, const void* v, const void* q_gain,
+                         const void* k_gain, const void* cos, const void* sin, void* k_out,
+                         void* out, int64_t B, int T, int heads, int kv_heads, int head_dim,
+                         int dtype, float q_eps, float k_eps, hipStream_t stream) {
+  const char* fn = "mhc_attn_prefill_fwd";
+  if (B < 0 || B > kMaxBlocks || T < 0) return fail(hipErrorInvalidValue, "%s: bad shape (B=%lld T=%d)", fn, (long long)B, T);
+  if (int rc = check_attn(B * T, heads, kv_heads, head_dim, dtype, fn)) return rc;
+  if (B * ((T + 63) / 64) * heads > kMaxBlocks || B * T * kv_heads / 32 > kMaxBlocks - 1)
+    return fail(hipErrorInvalidValue, "%s: too large", fn);
+  if (B * T == 0) return 0;
+  for (const void* p : {q, k, v, q_gain, k_gain, cos, sin, (const void*)k_out, (const void*)out})
+    if (!p || !aligned16(p)) return fail(hipErrorInvalidValue, "%s: null or unaligned pointer", fn);
+  const bool f16 = dtype == mhc::kF16;
+  const mhc::KRopeArgs r{k, k_gain, cos, sin, k_out, B * T, T, kv_heads, head_dim, f16, k_eps};
+  if (int rc = hip_status(mhc::launch_k_norm_rope(r, stream), fn)) return rc;
+  const mhc::AttnPrefillArgs a{q, q_gain, cos, sin, k_out, v, out, (int)B, T, heads, kv_heads, head_dim, 0, 0,
+                               f16, q_eps};
+  return hip_status(mhc::launch_attn_prefill(a, stream), fn);
+}
+
+int64_t mhc_attn_decode_workspace_bytes(int64_t B, int S, int heads, int kv_heads, int head_dim) {
+  if (B < 0 || S < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || heads / kv_heads > 4) return -1;
+  if (head_dim != 64 && head_dim != 96 && head_dim != 128) return -1;
+  if (B == 0) return 0;
+  int per = 0;
+  const int splits = mhc::attn_decode_splits(B, S, kv_heads, &per);
+  return splits == 1 ? 0 : B * heads * splits * (head_dim + 2) * 4;
+}
+
+int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void* q_gain,
+                        const void* k_gain, const void* cos, const void* sin, const void* k_past,
+                        int64_t k_stride_b, int64_t k_stride_s, int64_t k_stride_h,
+                        const void* v_past, int64_t v_stride_b, int64_t v_stride_s,
+                        int64_t v_stride_h, void* k_out, void* v_out, void* out, void* workspace,
+                        int64_t workspace_bytes, int64_t B, int S, int heads, int kv_heads,
+                        int head_dim, int dtype, float q_eps, float k_eps, hipStream_t stream) {
+  const char* fn = "mhc_attn_decode_fwd";
+  if (int rc = check_attn(B, heads, kv_heads, head_dim, dtype, fn)) return rc;
+  const int64_t need = mhc_attn_decode_workspace_bytes(B, S, heads, kv_heads, head_dim);
+  if (need < 0) return fail(hipErrorInvalidValue, "%s: needs S >= 1 and heads / kv_heads <= 4 (S=%d heads=%d kv_heads=%d)", fn, S, heads, kv_heads);
+  if (S > (1 << 30) || B * kv_heads > (1 << 20)) return fail(hipErrorInvalidValue, "%s: too large", fn);
+  if (B == 0) return 0;
+  for (const void* p : {q, k, v, q_gain, k_gain, cos, sin, k_past, v_past, (const void*)out})
+    if (!p || !aligned16(p)) return fail(hipErrorInvalidValue, "%s: null or unaligned pointer", fn);
+  if (!k_out != !v_out || !aligned16(k_out) || !aligned16(v_out))
+    return fail(hipErrorInvalidValue, "%s: k_out and v_out are both given, 16-byte aligned, or neither", fn);
+  for (int64_t st : {k_stride_b, k_stride_s, k_stride_h, v_stride_b, v_stride_s, v_stride_h})
+    if (st % 8 != 0) return fail(hipErrorInvalidValue, "%s: cache strides must be multiples of 8 elements", fn);
+  if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace)))
+    return fail(hipErrorInvalidValue, "%s: workspace of %lld bytes needed (got %lld)", fn, (long long)need, (long long)workspace_bytes);
+  mhc::AttnDecodeArgs a{};
+  a.q = q; a.k = k; a.v = v; a.q_gain = q_gain; a.k_gain = k_gain; a.cos = cos; a.sin = sin;
+  a.k_past = k_past; a.v_past = v_past; a.k_out = k_out; a.v_out = v_out; a.out = out;
+  a.work = static_cast<float*>(workspace);
+  a.ks_b = k_stride_b; a.ks_s = k_stride_s; a.ks_h = k_stride_h;
+  a.vs_b = v_stride_b; a.vs_s = v_stride_s; a.vs_h = v_stride_h;
+  a.B = B; a.S = S; a.heads = heads; a.kv_heads = kv_heads; a.head_dim = head_dim;
+  a.splits = mhc::attn_decode_splits(B, S, kv_heads, &a.tiles_per_split);
+  a.f16 = dtype == mhc::kF16; a.q_eps = q_eps; a.k_eps = k_eps;
+  return hip_status(mhc::launch_attn_decode(a, stream), fn);
+}
+
 }  // extern "C"

@@ -222,4 +222,64 @@ constexpr int kMfmaMaxColBlocks = 32;
 int64_t mfma_packed_bytes(int n, int C, int mode);
 bool mfma_supported(int x_dtype, int phi_dtype, int n, int C, int mode);
 
+// Attention of the model's sublayer (inference, 16-bit tensors, head_dim 64, 96 or
+// 128).  q [M, heads * head_dim], k and v [M, kv_heads * head_dim] are the raw
+// projections; gains [head_dim], cos / sin [T, head_dim], all in the same type.
+struct KRopeArgs {
+  const void* k;
+  const void* gain;
+  const void* cos;
+  const void* sin;
+  void* out;
+  int64_t M;
+  int T, kv_heads, head_dim;
+  bool f16;
+  float eps;
+};
+hipError_t launch_k_norm_rope(const KRopeArgs& a, hipStream_t s);
+
+// One decode step: B query tokens over S >= 1 cached positions and the new one.
+// k_past / v_past: [B, S, kv_heads, head_dim] with the given element strides (a
+// head's elements contiguous).  k_out / v_out (optional): the grown caches,
+// contiguous [B, S + 1, kv_heads, head_dim].  work: attn_decode_work_floats.
+struct AttnDecodeArgs {
+  const void* q;
+  const void* k;
+  const void* v;
+  const void* q_gain;
+  const void* k_gain;
+  const void* cos;  // [head_dim], the new position's
+  const void* sin;
+  const void* k_past;
+  const void* v_past;
+  void* k_out;
+  void* v_out;
+  void* out;  // [B, heads * head_dim]
+  float* work;
+  int64_t ks_b, ks_s, ks_h, vs_b, vs_s, vs_h;
+  int64_t B;
+  int S, heads, kv_heads, head_dim;
+  int splits, tiles_per_split;
+  bool f16;
+  float q_eps, k_eps;
+};
+int attn_decode_splits(int64_t B, int S, int kv_heads, int* tiles_per_split);
+hipError_t launch_attn_decode(const AttnDecodeArgs& a, hipStream_t s);
+
+// Causal attention of B sequences of T positions: q raw (normed and rotated
+// here), k already normed and rotated, v; contiguous [B, T, (kv_)heads, head_dim].
+struct AttnPrefillArgs {
+  const void* q;
+  const void* q_gain;
+  const void* cos;
+  const void* sin;
+  const void* k;
+  const void* v;
+  void* out;
+  int B, T, heads, kv_heads, head_dim, qtiles, cus;
+  bool f16;
+  float q_eps;
+};
+hipError_t launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t s);
+
 }  // namespace mhc

@@ -587,3 +587,121 @@ def sinkhorn_bwd(m: torch.Tensor, g: torch.Tensor, iters: int, eps: float,
                                    float(eps), H.stream(dev))
     H.check(rc, "mhc_sinkhorn_bwd")
     return out
+
+
+# ------------------------------------------- the model's sublayers, inference
+# Kernels in place of the torch ops of the sublayers.  They record no autograd
+# graph and see only data pointers, so a call takes them only when nothing but
+# the numbers could tell: no grad mode, no forward-mode level, no functorch
+# transform, no tracing or compiling, no dispatch mode, no autocast, and
+# submodules that nobody has hooked or patched.
+
+def plain_call() -> bool:
+    """Whether nothing is recording, transforming or tracing torch ops here."""
+    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda")
+                or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._len_torch_dispatch_stack() > 0
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.compiler.is_compiling() or torch.jit.is_tracing())
+
+
+_GLOBAL_HOOKS = torch.nn.modules.module
+
+
+def plain_module(m: torch.nn.Module, kind: type) -> bool:
+    """Whether m is exactly a `kind` whose call is its class's forward: no hooks
+    on it or on all modules, no forward of its own."""
+    return (type(m) is kind and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks)
+            and not (_GLOBAL_HOOKS._global_forward_hooks
+                     or _GLOBAL_HOOKS._global_forward_pre_hooks))
+
+
+def plain_tensors(dtype: torch.dtype, dev: torch.device, *ts) -> bool:
+    """Whether every tensor is a plain one of that dtype on that device, its data
+    16-byte aligned."""
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == dtype
+               and t.device == dev and t.data_ptr() % 16 == 0 for t in ts)
+
+
+ATTN_HEAD_DIMS = (64, 96, 128)
+
+
+def attn_route(m, q, k, v, position_embeddings, past) -> Optional[str]:
+    """Which kernel serves this call of the attention layer m between its
+    projections (q, k, v): "prefill", "decode", or None (the torch ops).
+    q [B, T, heads * head_dim]; k, v [B, T, kv_heads * head_dim]."""
+    H_, KV, hd = m.n_local_heads, m.n_local_kv_heads, m.head_dim
+    if (not q.is_cuda or q.dtype not in (torch.bfloat16, torch.float16) or hd not in ATTN_HEAD_DIMS
+            or q.dim() != 3 or H_ % KV != 0 or not plain_call()):
+        return None
+    B, T, _ = q.shape
+    if B * T == 0 or (m.training and m.dropout > 0) or (T > 1 and not m.is_causal):
+        return None
+    if not (plain_module(m.q_norm, torch.nn.RMSNorm) and plain_module(m.k_norm, torch.nn.RMSNorm)):
+        return None
+    cos, sin = position_embeddings
+    gq, gk = m.q_norm.weight, m.k_norm.weight
+    if gq is None or gk is None or not plain_tensors(q.dtype, q.device, q, k, v, gq, gk, cos, sin):
+        return None
+    if not (q.shape == (B, T, H_ * hd) and k.shape == v.shape == (B, T, KV * hd)
+            and gq.shape == gk.shape == (hd,) and cos.shape == sin.shape == (T, hd)
+            and all(t.is_contiguous() for t in (q, k, v, gq, gk, cos, sin))):
+        return None
+    if past is None:
+        return "prefill"
+    pk, pv = past[0], past[1]
+    if (T != 1 or H_ // KV > 4 or not plain_tensors(q.dtype, q.device, pk, pv)
+            or pk.dim() != 4 or pk.shape != pv.shape
+            or pk.shape[0] != B or pk.shape[1] < 1 or tuple(pk.shape[2:]) != (KV, hd)):
+        return None
+    for t in (pk, pv):
+        if t.stride(3) != 1 or any(s % 8 for s in t.stride()[:3]):
+            return None
+    return "decode"
+
+
+def _rms_eps(norm, dtype) -> float:
+    return float(norm.eps) if norm.eps is not None else float(torch.finfo(dtype).eps)
+
+
+def attn_prefill(m, q, k, v, position_embeddings):
+    """(attention output [B, T, heads * head_dim], normed and rotated k); the
+    call is one attn_route calls "prefill"."""
+    B, T, _ = q.shape
+    H_, KV, hd = m.n_local_heads, m.n_local_kv_heads, m.head_dim
+    cos, sin = position_embeddings
+    kr, out = torch.empty_like(k), torch.empty_like(q)
+    H.check(H.load().mhc_attn_prefill_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), m.q_norm.weight.data_ptr(),
+        m.k_norm.weight.data_ptr(), cos.data_ptr(), sin.data_ptr(), kr.data_ptr(), out.data_ptr(),
+        B, T, H_, KV, hd, H.dtype_tag(q), _rms_eps(m.q_norm, q.dtype), _rms_eps(m.k_norm, q.dtype),
+        H.stream(q.device)), "mhc_attn_prefill_fwd")
+    return out, kr
+
+
+def attn_decode(m, q, k, v, position_embeddings, past, use_cache: bool):
+    """(attention output [B, 1, heads * head_dim], grown (k, v) caches or None);
+    the call is one attn_route calls "decode"."""
+    B = q.shape[0]
+    H_, KV, hd = m.n_local_heads, m.n_local_kv_heads, m.head_dim
+    cos, sin = position_embeddings
+    pk, pv = past[0], past[1]
+    S = pk.shape[1]
+    lib = H.load()
+    out = torch.empty_like(q)
+    grown = None
+    if use_cache:
+        grown = tuple(torch.empty(B, S + 1, KV, hd, dtype=q.dtype, device=q.device)
+                      for _ in range(2))
+    nbytes = lib.mhc_attn_decode_workspace_bytes(B, S, H_, KV, hd)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes > 0 else None
+    H.check(lib.mhc_attn_decode_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), m.q_norm.weight.data_ptr(),
+        m.k_norm.weight.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+        pk.data_ptr(), *pk.stride()[:3], pv.data_ptr(), *pv.stride()[:3],
+        grown[0].data_ptr() if grown else None, grown[1].data_ptr() if grown else None,
+        out.data_ptr(), H.ptr(ws), max(nbytes, 0), B, S, H_, KV, hd, H.dtype_tag(q),
+        _rms_eps(m.q_norm, q.dtype), _rms_eps(m.k_norm, q.dtype), H.stream(q.device)),
+        "mhc_attn_decode_fwd")
+    return out, grown

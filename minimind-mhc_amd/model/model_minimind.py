@@ -33,6 +33,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from . import _ops
 from ._ops import StreamChain
 from .mhc_common import MHCHead, StreamExpand
 from .mhc_fused import MHCConnection_Fused
@@ -123,7 +124,10 @@ def repeat_kv(x: torch.Tensor, n_rep: int) -> torch.Tensor:
 
 class Attention(nn.Module):
     """GQA attention with q/k RMSNorm, RoPE and a (k, v) cache
-    (model/model_minimind.py:161-256), evaluated with torch SDPA."""
+    (model/model_minimind.py:161-256).  Inference on 16-bit tensors without a
+    mask runs between the projections on HIP kernels, for a prefill from an
+    empty cache and for one-token steps (_ops.attn_route says when); everything
+    else on torch ops and SDPA."""
 
     def __init__(self, config: MiniMindConfig):
         super().__init__()
@@ -145,9 +149,20 @@ class Attention(nn.Module):
     def forward(self, x, position_embeddings, past_key_value=None, use_cache=False,
                 attention_mask=None):
         bsz, seq_len, _ = x.shape
-        xq = self.q_proj(x).view(bsz, seq_len, self.n_local_heads, self.head_dim)
-        xk = self.k_proj(x).view(bsz, seq_len, self.n_local_kv_heads, self.head_dim)
-        xv = self.v_proj(x).view(bsz, seq_len, self.n_local_kv_heads, self.head_dim)
+        xq, xk, xv = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        route = None if attention_mask is not None else _ops.attn_route(
+            self, xq, xk, xv, position_embeddings, past_key_value)
+        if route == "decode":
+            out, past_kv = _ops.attn_decode(self, xq, xk, xv, position_embeddings,
+                                            past_key_value, use_cache)
+            return self.o_proj(out), past_kv
+        if route == "prefill":
+            out, xk = _ops.attn_prefill(self, xq, xk, xv, position_embeddings)
+            kv_shape = (bsz, seq_len, self.n_local_kv_heads, self.head_dim)
+            return self.o_proj(out), ((xk.view(kv_shape), xv.view(kv_shape)) if use_cache else None)
+        xq = xq.view(bsz, seq_len, self.n_local_heads, self.head_dim)
+        xk = xk.view(bsz, seq_len, self.n_local_kv_heads, self.head_dim)
+        xv = xv.view(bsz, seq_len, self.n_local_kv_heads, self.head_dim)
         xq, xk = self.q_norm(xq), self.k_norm(xk)
         cos, sin = position_embeddings
         xq, xk = apply_rotary_pos_emb(xq, xk, cos, sin)
