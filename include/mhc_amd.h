@@ -480,6 +480,27 @@ int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void*
                         int64_t workspace_bytes, int64_t B, int S, int heads, int kv_heads,
                         int head_dim, int dtype, float q_eps, float k_eps, hipStream_t stream);
 
+/* ------------------------------------- routed-expert layer (inference)
+ * SwiGLU experts with top-k routing (model/model_minimind.py:270-298); 16-bit
+ * tensors (bf16 or fp16) of one dtype.
+ */
+
+/* Bytes of workspace mhc_moe_fwd needs, or -1 for a shape it does not take:
+ * hidden and inter multiples of 32, 1 <= topk <= 8, topk <= experts <= 32,
+ * M <= 262144. */
+int64_t mhc_moe_workspace_bytes(int64_t M, int hidden, int inter, int experts, int topk);
+
+/* out [M, hidden] = sum over a token's topk experts of weight * expert(x).
+ * probs [M, experts]: the router's softmax; the topk largest are taken (the
+ * lower index where two are equal) and, with norm_topk, divided by their sum.
+ * gate_w, up_w, down_w: host arrays of `experts` device pointers to
+ * [inter, hidden], [inter, hidden] and [hidden, inter].  Device pointers are
+ * 16-byte aligned. */
+int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
+                const void* const* up_w, const void* const* down_w, void* out, void* workspace,
+                int64_t workspace_bytes, int64_t M, int hidden, int inter, int experts, int topk,
+                int norm_topk, int dtype, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -702,4 +702,41 @@ int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void*
   return hip_status(mhc::launch_attn_decode(a, stream), fn);
 }
 
+// ------------------------------------------- routed-expert layer (inference)
+
+int64_t mhc_moe_workspace_bytes(int64_t M, int hidden, int inter, int experts, int topk) {
+  if (M < 0 || M > 262144 || hidden < 32 || hidden % 32 != 0 || inter < 32 || inter % 32 != 0) return -1;
+  if (experts < 1 || experts > mhc::kMoeMaxExperts || topk < 1 || topk > mhc::kMoeMaxTopk || topk > experts) return -1;
+  mhc::MoeArgs a{};
+  a.M = M; a.hidden = hidden; a.inter = inter; a.experts = experts; a.topk = topk;
+  return mhc::moe_workspace(a, nullptr);
+}
+
+int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
+                const void* const* up_w, const void* const* down_w, void* out, void* workspace,
+                int64_t workspace_bytes, int64_t M, int hidden, int inter, int experts, int topk,
+                int norm_topk, int dtype, hipStream_t stream) {
+  const char* fn = "mhc_moe_fwd";
+  const int64_t need = mhc_moe_workspace_bytes(M, hidden, inter, experts, topk);
+  if (need < 0)
+    return fail(hipErrorInvalidValue, "%s: bad shape (M=%lld hidden=%d inter=%d experts=%d topk=%d)", fn, (long long)M, hidden, inter, experts, topk);
+  if (dtype != mhc::kBF16 && dtype != mhc::kF16) return fail(hipErrorInvalidValue, "%s: dtype must be bf16 or fp16 (got %d)", fn, dtype);
+  if (M == 0) return 0;
+  if (!x || !probs || !gate_w || !up_w || !down_w || !out || !aligned16(x) || !aligned16(out))
+    return fail(hipErrorInvalidValue, "%s: null or unaligned pointer", fn);
+  if (!workspace || workspace_bytes < need || !aligned16(workspace))
+    return fail(hipErrorInvalidValue, "%s: workspace of %lld bytes needed (got %lld)", fn, (long long)need, (long long)workspace_bytes);
+  mhc::MoeArgs a{};
+  for (int e = 0; e < experts; ++e) {
+    for (const void* w : {gate_w[e], up_w[e], down_w[e]})
+      if (!w || !aligned16(w)) return fail(hipErrorInvalidValue, "%s: null or unaligned weight of expert %d", fn, e);
+    a.gate_w[e] = gate_w[e]; a.up_w[e] = up_w[e]; a.down_w[e] = down_w[e];
+  }
+  a.x = x; a.probs = probs; a.out = out;
+  a.M = M; a.hidden = hidden; a.inter = inter; a.experts = experts; a.topk = topk;
+  a.norm_topk = norm_topk != 0; a.f16 = dtype == mhc::kF16;
+  mhc::moe_workspace(a, static_cast<char*>(workspace));
+  return hip_status(mhc::launch_moe(a, stream), fn);
+}
+
 }  // extern "C"

@@ -282,4 +282,34 @@ struct AttnPrefillArgs {
 };
 hipError_t launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t s);
 
+// Routed-expert SwiGLU layer (inference, 16-bit tensors).  x, out [M, hidden];
+// probs [M, experts] (the router's softmax); gate_w / up_w [inter, hidden] and
+// down_w [hidden, inter] per expert.  hidden and inter are multiples of 32.
+constexpr int kMoeMaxExperts = 32;
+constexpr int kMoeMaxTopk = 8;
+struct MoeArgs {
+  const void* x;
+  const void* probs;
+  void* out;
+  const void* gate_w[kMoeMaxExperts];
+  const void* up_w[kMoeMaxExperts];
+  const void* down_w[kMoeMaxExperts];
+  int64_t M;
+  int hidden, inter, experts, topk;
+  bool norm_topk, f16;
+  // workspace (moe_workspace)
+  int* counts;    // [workgroups][experts] of the grouping launches
+  int* offsets;   // [experts + 1] first row of each expert
+  int* pick;      // [M, topk] expert, and its weight
+  float* pick_w;
+  int* slot_of;   // [M, topk] row of the pair
+  int* row_tok;   // [M * topk] a row's token, and its weight
+  float* row_w;
+  void* h;        // [M * topk, inter]
+  void* y;        // [M * topk, hidden]
+};
+// Lays the workspace out at base (null: only its size) and returns its bytes.
+int64_t moe_workspace(MoeArgs& a, char* base);
+hipError_t launch_moe(const MoeArgs& a, hipStream_t s);
+
 }  // namespace mhc

@@ -89,6 +89,9 @@ _SIGNATURES = {
                                          _I64, _I, _I, _I, _P]),
     "mhc_sinkhorn_bwd": (_I, [_P, _I, _P, _I, _P, _I, _I64, _I, _I, _F, _P]),
     "mhc_sinkhorn_bwd_max_iters": (_I, [_I]),
+    "mhc_moe_workspace_bytes": (_I64, [_I64, _I, _I, _I, _I]),
+    "mhc_moe_fwd": (_I, [_P, _P, _P, _P, _P, _P,          # x, probs, gate_w, up_w, down_w, out
+                         _P, _I64, _I64, _I, _I, _I, _I, _I, _I, _P]),
     "mhc_attn_prefill_fwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P,  # q, k, v, gains, cos, sin, k_out, out
                                   _I64, _I, _I, _I, _I, _I, _F, _F, _P]),
     "mhc_attn_decode_workspace_bytes": (_I64, [_I64, _I, _I, _I, _I]),

@@ -7,6 +7,7 @@ current stream.  Inputs are made contiguous, as the reference's Functions do
 """
 from __future__ import annotations
 
+import ctypes
 import threading
 import weakref
 from typing import Optional
@@ -705,3 +706,39 @@ def attn_decode(m, q, k, v, position_embeddings, past, use_cache: bool):
         _rms_eps(m.q_norm, q.dtype), _rms_eps(m.k_norm, q.dtype), H.stream(q.device)),
         "mhc_attn_decode_fwd")
     return out, grown
+
+
+def moe_experts(experts, x: torch.Tensor, probs: torch.Tensor, topk: int, norm_topk: bool):
+    """The routed experts' weighted sum for x [M, hidden] on the HIP kernels, or
+    None for a call they do not take.  experts: modules with gate_proj, up_proj
+    and down_proj (plain nn.Linear without bias) and SiLU between them; probs
+    [M, experts], the router's softmax."""
+    if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or not plain_call()
+            or x.dim() != 2 or x.shape[0] == 0 or not x.is_contiguous()
+            or probs.shape != (x.shape[0], len(experts)) or not probs.is_contiguous()):
+        return None
+    M, D = x.shape
+    kind, ws = type(experts[0]), ([], [], [])
+    for e in experts:
+        if not plain_module(e, kind):
+            return None
+        for lin, w in zip((e.gate_proj, e.up_proj, e.down_proj), ws):
+            if not plain_module(lin, torch.nn.Linear) or lin.bias is not None:
+                return None
+            w.append(lin.weight)
+    inter = ws[0][0].shape[0]
+    if (any(t.shape != (inter, D) or not t.is_contiguous() for t in ws[0] + ws[1])
+            or any(t.shape != (D, inter) or not t.is_contiguous() for t in ws[2])
+            or not plain_tensors(x.dtype, x.device, x, probs, *ws[0], *ws[1], *ws[2])):
+        return None
+    lib = H.load()
+    nbytes = lib.mhc_moe_workspace_bytes(M, D, inter, len(experts), topk)
+    if nbytes < 0:
+        return None
+    out = torch.empty_like(x)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    ptrs = [(ctypes.c_void_p * len(w))(*[t.data_ptr() for t in w]) for w in ws]
+    H.check(lib.mhc_moe_fwd(x.data_ptr(), probs.data_ptr(), *ptrs, out.data_ptr(),
+                            work.data_ptr(), nbytes, M, D, inter, len(experts), topk,
+                            int(norm_topk), H.dtype_tag(x), H.stream(x.device)), "mhc_moe_fwd")
+    return out

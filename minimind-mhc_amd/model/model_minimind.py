@@ -210,7 +210,9 @@ class FeedForward(nn.Module):
 
 
 class MOEFeedForward(nn.Module):
-    """Top-k softmax-routed experts (model/model_minimind.py:270-298), inference path."""
+    """Top-k softmax-routed experts (model/model_minimind.py:270-298).  Inference on
+    16-bit tensors runs the experts on HIP kernels with no host synchronisation
+    (_ops.moe_experts says when); everything else loops over the experts."""
 
     def __init__(self, config: MiniMindConfig):
         super().__init__()
@@ -224,6 +226,12 @@ class MOEFeedForward(nn.Module):
         b, l, d = x.shape
         xf = x.view(-1, d)
         scores = F.softmax(self.gate(xf), dim=-1)
+        if not self.training:
+            y = _ops.moe_experts(self.experts, xf, scores, self.config.num_experts_per_tok,
+                                 self.config.norm_topk_prob)
+            if y is not None:
+                self.aux_loss = scores.new_zeros(1).squeeze()
+                return y.view(b, l, d)
         w, idx = torch.topk(scores, k=self.config.num_experts_per_tok, dim=-1, sorted=False)
         if self.config.norm_topk_prob:
             w = w / (w.sum(dim=-1, keepdim=True) + 1e-20)
