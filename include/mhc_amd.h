@@ -85,6 +85,15 @@ int mhc_phi_pack(const void* phi, int phi_dtype, void* packed, int n, int C, int
                  hipStream_t stream);
 
 /*
+ * The same image of an fp16 phi (mhc_phi_packed_bytes bytes; n in {2, 4, 8, 16}),
+ * for fp16 streams.  A pre-phase call that passes it as phi_packed says so with
+ * phi_dtype = MHC_DTYPE_F16 | MHC_PHI_F16_IMAGE; with plain MHC_DTYPE_F16
+ * phi_packed is ignored and the VALU kernel runs.
+ */
+#define MHC_PHI_F16_IMAGE 0x100
+int mhc_phi_pack_f16(const void* phi, void* packed, int n, int C, int mode, hipStream_t stream);
+
+/*
  * Size in bytes of the split-operand image of an fp32 phi for (n, C, mode), or
  * 0 when that shape has no fp32 MFMA kernel.  Shapes with one: n in {1,2,4}
  * with C <= 1024 (16-column tiles of hi | lo pairs, one-workgroup-per-tile

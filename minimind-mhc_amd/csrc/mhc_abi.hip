@@ -66,6 +66,10 @@ int check_pre(const mhc::PreArgs& a, const char* fn) {
 }
 
 int run_pre(mhc::PreArgs& a, hipStream_t stream, const char* fn) {
+  // MHC_PHI_F16_IMAGE says that phi_packed is there as an fp16 image; without it
+  // an fp16 call ignores phi_packed
+  const bool f16_image = a.phi_dtype == (mhc::kF16 | MHC_PHI_F16_IMAGE);
+  if (f16_image) a.phi_dtype = mhc::kF16;
   if (int rc = check_pre(a, fn)) return rc;
   if (a.M == 0) return 0;
   const bool packed_ok = a.phi_packed && a.mode != mhc::kRms && aligned16(a.x) && aligned16(a.sub_in) &&
@@ -73,10 +77,11 @@ int run_pre(mhc::PreArgs& a, hipStream_t stream, const char* fn) {
   const bool mfma = packed_ok && mhc::mfma_supported(a.x_dtype, a.phi_dtype, a.n, a.C, a.mode);
   const bool split = packed_ok && !a.norm_w && mhc::split_supported(a.x_dtype, a.phi_dtype, a.n, a.C, a.mode);
   const bool ks32 = packed_ok && mhc::ks32_supported(a.x_dtype, a.phi_dtype, a.n, a.C, a.mode);
-  if (!mfma && !split && !ks32) a.phi_packed = nullptr;
+  const bool f16 = packed_ok && f16_image && mhc::f16_supported(a.x_dtype, a.phi_dtype, a.n, a.C, a.mode);
+  if (!mfma && !split && !ks32 && !f16) a.phi_packed = nullptr;
   if (!mfma || !mhc::ssq_used(a.n, a.C)) a.x_ssq = nullptr;
   if (split) return hip_status(mhc::launch_pre_split(a, mhc::device_cus(), stream), fn);
-  if (ks32) return hip_status(mhc::launch_pre_kstream_f32(a, stream), fn);
+  if (ks32 || f16) return hip_status(mhc::launch_pre_kstream(a, stream), fn);
   return hip_status(mfma ? mhc::launch_pre_mfma(a, stream) : mhc::launch_pre_generic(a, stream), fn);
 }
 
@@ -196,6 +201,13 @@ int mhc_phi_pack(const void* phi, int phi_dtype, void* packed, int n, int C, int
   if (phi_dtype != mhc::kBF16) return fail(hipErrorInvalidValue, "mhc_phi_pack: phi must be bf16");
   if (!phi || !packed) return fail(hipErrorInvalidValue, "mhc_phi_pack: null pointer");
   return hip_status(mhc::launch_phi_pack(phi, phi_dtype, packed, n, C, mode, stream), "mhc_phi_pack");
+}
+
+int mhc_phi_pack_f16(const void* phi, void* packed, int n, int C, int mode, hipStream_t stream) {
+  if (!mhc::f16_supported(mhc::kF16, mhc::kF16, n, C, mode))
+    return fail(hipErrorInvalidValue, "mhc_phi_pack_f16: no fp16 layout for n=%d C=%d mode=%d", n, C, mode);
+  if (!phi || !packed) return fail(hipErrorInvalidValue, "mhc_phi_pack_f16: null pointer");
+  return hip_status(mhc::launch_phi_pack(phi, mhc::kF16, packed, n, C, mode, stream), "mhc_phi_pack_f16");
 }
 
 int64_t mhc_phi_split_bytes(int n, int C, int mode) {

@@ -7,33 +7,7 @@
 namespace mhc {
 namespace {
 
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
-
-template <bool F16>
-__device__ __forceinline__ float elem_lo(uint32_t u) {
-  if constexpr (F16) return f16_bits_to_f32((uint16_t)(u & 0xffffu));
-  else return bf16lo(u);
-}
-template <bool F16>
-__device__ __forceinline__ float elem_hi(uint32_t u) {
-  if constexpr (F16) return f16_bits_to_f32((uint16_t)(u >> 16));
-  else return bf16hi(u);
-}
-template <bool F16>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  if constexpr (F16) return (uint32_t)f32_to_f16_bits(a) | ((uint32_t)f32_to_f16_bits(b) << 16);
-  else return pack_bf16x2(a, b);
-}
-template <bool F16>
-__device__ __forceinline__ f32x4_t mfma16(const U32x4& a, const U32x4& b, const f32x4_t& c) {
-  if constexpr (F16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
-                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
 
 __device__ __forceinline__ U32x4 ld16(const void* p) { return *static_cast<const U32x4*>(p); }
 

@@ -241,6 +241,35 @@ __device__ __forceinline__ float affine_rn(float s, float alpha, float beta) {
   return __fadd_rn(mul_nc(s, alpha), beta);
 }
 
+// ------------------------------------------------- packed 16-bit pairs, either type
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+
+template <bool F16>
+__device__ __forceinline__ float elem_lo(uint32_t u) {
+  if constexpr (F16) return f16_bits_to_f32((uint16_t)(u & 0xffffu));
+  else return bf16lo(u);
+}
+template <bool F16>
+__device__ __forceinline__ float elem_hi(uint32_t u) {
+  if constexpr (F16) return f16_bits_to_f32((uint16_t)(u >> 16));
+  else return bf16hi(u);
+}
+template <bool F16>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  if constexpr (F16) return (uint32_t)f32_to_f16_bits(a) | ((uint32_t)f32_to_f16_bits(b) << 16);
+  else return pack_bf16x2(a, b);
+}
+template <bool F16>
+__device__ __forceinline__ f32x4_t mfma16(const U32x4& a, const U32x4& b, const f32x4_t& c) {
+  if constexpr (F16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
+                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
 // ---------------------------------------------- reference rounding points
 // The reference's PyTorch path evaluates the gates as separate torch ops on
 // tensors of the stream dtype (model/mhc_fused.py:846-854): the projection
@@ -274,10 +303,11 @@ __device__ __forceinline__ float gate_res(float m, float alpha, float bias, int 
 // bf16(x * inv) for the 8 columns of one 16-byte chunk: the fp32 product
 // rounded to bf16, as the reference's x_norm = (x.float() * inv_rms).to(x.dtype)
 // (model/mhc_fused.py:845) rounds it.
+template <bool F16 = false>
 __device__ __forceinline__ U32x4 x_norm_chunk(const U32x4& v, float inv) {
   U32x4 o;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) o.v[j] = pack_bf16x2(bf16lo(v.v[j]) * inv, bf16hi(v.v[j]) * inv);
+  for (int j = 0; j < 4; ++j) o.v[j] = pack2<F16>(elem_lo<F16>(v.v[j]) * inv, elem_hi<F16>(v.v[j]) * inv);
   return o;
 }
 
@@ -334,6 +364,39 @@ __device__ __forceinline__ U32x4 preagg_chunk(const U32x4 (&x)[N], const uint32_
 #pragma unroll
     for (int i = 0; i < N; ++i) xj[i] = x[i].v[j];
     out.v[j] = preagg_pair<N>(xj, hlo, hhi);
+  }
+  return out;
+}
+
+// c + lo^2 + hi^2 of a packed pair.
+template <bool F16>
+__device__ __forceinline__ float sumsq2(uint32_t v, float c) {
+  if constexpr (F16) {
+    const float lo = elem_lo<true>(v), hi = elem_hi<true>(v);
+    return fmaf(hi, hi, fmaf(lo, lo, c));
+  } else {
+    return dot2_bf16(v, v, c);
+  }
+}
+
+// preagg_chunk on fp16 streams: two products a v_pk_mul_f16, each rounded to fp16
+// by the multiply itself, summed in fp32 in stream order.  (No dot2 with a zero
+// partner here: an infinite neighbour, which fp16 streams do reach, would make
+// the column NaN.)
+template <int N>
+__device__ __forceinline__ U32x4 preagg_chunk_f16(const U32x4 (&x)[N], const float (&h)[N]) {
+  U32x4 out;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float lo = 0.f, hi = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const _Float16 hh = (_Float16)h[i];
+      const f16x2_t p = __builtin_bit_cast(f16x2_t, x[i].v[j]) * f16x2_t{hh, hh};
+      lo += (float)p.x;
+      hi += (float)p.y;
+    }
+    out.v[j] = pack2<true>(lo, hi);
   }
   return out;
 }

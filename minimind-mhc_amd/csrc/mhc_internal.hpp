@@ -194,7 +194,11 @@ int64_t ks32_packed_bytes(int n, int C, int mode);
 bool ks32_supported(int x_dtype, int phi_dtype, int n, int C, int mode);
 hipError_t launch_phi_pack_ks32(const void* phi, int phi_dtype, void* packed, int n, int C, int mode,
                                 hipStream_t s);
-hipError_t launch_pre_kstream_f32(const PreArgs& a, hipStream_t s);
+// fp16 stream and phi on the K-streamed kernel (n in {2, 4, 8, 16}, any C % 8 ==
+// 0): image as packed bf16, with fp16 values (mhc_phi_pack_f16).
+bool f16_supported(int x_dtype, int phi_dtype, int n, int C, int mode);
+// The K-streamed kernel of a.x_dtype for a.n.
+hipError_t launch_pre_kstream(const PreArgs& a, hipStream_t s);
 
 // Per-row sums of squares handed from the kernel that writes a stream to the
 // pre kernel that reads it: one fp32 partial per kSsqCols columns of C (for

@@ -1,7 +1,7 @@
 // Pre phase: MFMA dispatch, phi packing, and the generic VALU kernel.
 //
 // The generic kernel serves every (dtype, n, C) the MFMA instances do not:
-// fp16 streams, mixed stream / phi dtypes, fp32 outside the split kernel's
+// mixed stream / phi dtypes, fp16 at n = 1 or without an image, fp32 outside the split kernel's
 // shapes (n <= 4, C <= 1024), C % 8 != 0, and the n == 1 MHCHead (plain
 // RMSNorm) at C > 1024.  One 256-thread workgroup per token; it is a
 // correctness path, not a tuned one.  x_norm = x * inv_rms is rounded to the
@@ -20,11 +20,12 @@ namespace mhc {
 // so that lane `lane` of the wave reading column block cb of stream i finds its
 // MFMA B operand (8 consecutive k for output column lane%16) as one 16-byte load.
 // lo: the image of phi - bf16(phi) instead (the low half of an fp32 phi split
-// into bf16 hi + lo operands for the fp32 K-streamed kernel).
+// into bf16 hi + lo operands for the fp32 K-streamed kernel).  f16: phi's fp16
+// bits (the fp16 K-streamed kernel).
 __global__ __launch_bounds__(256) void phi_pack_kernel(const void* __restrict__ phi, int dt,
                                                        uint16_t* __restrict__ packed, int C,
                                                        int FD, int NCB, int NT, int64_t total,
-                                                       int lo) {
+                                                       int lo, int f16) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= total) return;
   const int s = (int)(idx & 7);
@@ -38,6 +39,10 @@ __global__ __launch_bounds__(256) void phi_pack_kernel(const void* __restrict__ 
   const int f = nt * 16 + (lane & 15);
   float v = 0.f;
   if (c < C && f < FD) v = ld_any(phi, ((int64_t)i * C + c) * FD + f, dt);
+  if (f16) {
+    packed[idx] = f32_to_f16_bits(v);
+    return;
+  }
   const uint16_t hi = f32_to_bf16_bits(v);
   packed[idx] = lo ? f32_to_bf16_bits(v - bf16_bits_to_f32(hi)) : hi;
 }
@@ -64,6 +69,21 @@ static bool pre_wide(int n, int C) {
   return n == 16 || (C + kCBlock - 1) / kCBlock > kMfmaMaxColBlocks;
 }
 
+// fp16 stream and phi on the K-streamed kernel, any C it takes.
+bool f16_supported(int x_dtype, int phi_dtype, int n, int C, int mode) {
+  return x_dtype == kF16 && phi_dtype == kF16 && n >= 2 && mfma_packed_bytes(n, C, mode) > 0;
+}
+
+hipError_t launch_pre_kstream(const PreArgs& a, hipStream_t s) {
+  switch (a.n) {
+    case 2: return launch_pre_kstream_n2(a, s);
+    case 4: return launch_pre_kstream_n4(a, s);
+    case 8: return launch_pre_kstream_n8(a, s);
+    case 16: return launch_pre_kstream_n16(a, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 bool mfma_supported(int x_dtype, int phi_dtype, int n, int C, int mode) {
   return x_dtype == kBF16 && phi_dtype == kBF16 && mfma_packed_bytes(n, C, mode) > 0;
 }
@@ -76,7 +96,7 @@ hipError_t launch_phi_pack(const void* phi, int phi_dtype, void* packed, int n, 
   const int64_t total = (int64_t)n * ncb * nt * 64 * 8;
   const int64_t blocks = (total + 255) / 256;
   hipLaunchKernelGGL(phi_pack_kernel, dim3((unsigned)blocks), dim3(256), 0, s, phi, phi_dtype,
-                     static_cast<uint16_t*>(packed), C, fd, ncb, nt, total, lo);
+                     static_cast<uint16_t*>(packed), C, fd, ncb, nt, total, lo, (int)(phi_dtype == kF16));
   return hipGetLastError();
 }
 
@@ -100,15 +120,6 @@ hipError_t launch_phi_pack_ks32(const void* phi, int phi_dtype, void* packed, in
   if (e != hipSuccess) return e;
   return launch_phi_pack(phi, phi_dtype, static_cast<unsigned char*>(packed) + mfma_packed_bytes(n, C, mode),
                          n, C, mode, s, 1);
-}
-
-hipError_t launch_pre_kstream_f32(const PreArgs& a, hipStream_t s) {
-  switch (a.n) {
-    case 2: return launch_pre_kstream_n2(a, s);
-    case 4: return launch_pre_kstream_n4(a, s);
-    case 8: return launch_pre_kstream_n8(a, s);
-    default: return hipErrorInvalidValue;
-  }
 }
 
 // ------------------------------------------------------ process-wide settings
@@ -149,15 +160,7 @@ int device_cus() {
 hipError_t launch_pre_mfma(const PreArgs& a, hipStream_t s) {
   const int cus = device_cus();
   // n = 16, C > 1024: phi streams from L2 through the K-split MFMA loop.
-  if (pre_wide(a.n, a.C)) {
-    switch (a.n) {
-      case 2: return launch_pre_kstream_n2(a, s);
-      case 4: return launch_pre_kstream_n4(a, s);
-      case 8: return launch_pre_kstream_n8(a, s);
-      case 16: return launch_pre_kstream_n16(a, s);
-      default: return hipErrorInvalidValue;
-    }
-  }
+  if (pre_wide(a.n, a.C)) return launch_pre_kstream(a, s);
   // Decode-size batches: one workgroup per group of up to 16 tokens.
   if (a.M <= pre_token_max_m() && a.phi_packed) {
     switch (a.n) {

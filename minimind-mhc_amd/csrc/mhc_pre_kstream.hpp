@@ -44,6 +44,8 @@
 // model/mhc_fused_no_hres.py:48-145; model/mhc_common.py:128-195.
 #pragma once
 
+#include <type_traits>
+
 #include "mhc_pre_persist.hpp"
 
 namespace mhc {
@@ -197,13 +199,18 @@ constexpr bool ks_regroup_in_slot() {
 // squares handed over) 48.6 -> 43.3 us; the 64-token n = 8 group projection,
 // which must follow the order, 12.7 -> 13.9 us (one box).  Wave kq taking a
 // contiguous range of pairs instead measured the same at C5, slower at 64.
-template <int N, int MODE, bool NORM, bool F32 = false, bool PAIRS = false>
+// F16: fp16 stream and phi (phi_packed is then the fp16 image): the same
+// schedule with fp16 operands, products and roundings.  4055 tokens, n = 4,
+// C = 768 with the norm: VALU kernel 387 us, here 24.4; n = 8 at 4096 tokens 6485 -> 44,
+// at 64 tokens 371 -> 33 (ahead of it at every batch size from 1 on).
+template <int N, int MODE, bool NORM, bool F32 = false, bool PAIRS = false, bool F16 = false>
 __global__ __launch_bounds__(kKsWaves * 64) void pre_kstream_kernel(PreArgs a) {
   using P = KsPlan<N, MODE>;
   using GP = GateParams<N>;
   using NS = KsNorm<N, MODE, NORM>;
+  static_assert(!(F32 && F16), "one stream type");
   static_assert(!(F32 && NORM), "fp32 streams: the norm runs as a second launch");
-  static_assert(!PAIRS || (!F32 && ks_pairs<N, MODE>() && P::NH == 1), "chunk pairs: bf16, n in {2, 4, 8}");
+  static_assert(!PAIRS || (!F32 && ks_pairs<N, MODE>() && P::NH == 1), "chunk pairs: 16-bit, n in {2, 4, 8}");
   constexpr int FD = P::FD;
   constexpr int NT = P::NT;
   constexpr int NTW = P::NTW;
@@ -211,7 +218,7 @@ __global__ __launch_bounds__(kKsWaves * 64) void pre_kstream_kernel(PreArgs a) {
   constexpr int D = F32 ? 2 : P::D;      // chunks in flight (fp32: hi and lo phi operands)
   constexpr int XQ = F32 ? 2 : 1;        // 16-byte loads per 8 columns of a row
   constexpr uint32_t ES = F32 ? 4u : 2u; // bytes per stream element
-  constexpr int XDT = F32 ? kF32 : kBF16;
+  constexpr int XDT = F32 ? kF32 : F16 ? kF16 : kBF16;
   constexpr int LPT = P::LPT;
   constexpr int SKV = P::SKV;
   constexpr int T = P::WAVES * 64;
@@ -466,7 +473,7 @@ __global__ __launch_bounds__(kKsWaves * 64) void pre_kstream_kernel(PreArgs a) {
 #pragma unroll
             for (int m = 0; m < P::MB; ++m)
 #pragma unroll
-              for (int q = 0; q < 4; ++q) ss[m] = dot2_bf16(ov[h][m].v[q], ov[h][m].v[q], ss[m]);
+              for (int q = 0; q < 4; ++q) ss[m] = sumsq2<F16>(ov[h][m].v[q], ss[m]);
         }
       }
 #pragma unroll
@@ -501,7 +508,7 @@ __global__ __launch_bounds__(kKsWaves * 64) void pre_kstream_kernel(PreArgs a) {
                   const float f = __uint_as_float(v[d][m][xq].v[q]);
                   ss[m] = fmaf(f, f, ss[m]);
                 } else {
-                  ss[m] = dot2_bf16(v[d][m][xq].v[q], v[d][m][xq].v[q], ss[m]);
+                  ss[m] = sumsq2<F16>(v[d][m][xq].v[q], ss[m]);
                 }
               }
       }
@@ -540,11 +547,9 @@ __global__ __launch_bounds__(kKsWaves * 64) void pre_kstream_kernel(PreArgs a) {
         for (int h = 0; h < 2; ++h)
 #pragma unroll
           for (int m = 0; m < P::MB; ++m) {
-            const bf16x8_t av = __builtin_bit_cast(bf16x8_t, x_norm_chunk(ov[h][m], inv_r[m]));
+            const U32x4 av = x_norm_chunk<F16>(ov[h][m], inv_r[m]);
 #pragma unroll
-            for (int nt = 0; nt < NTW; ++nt)
-              acc[m][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                  av, __builtin_bit_cast(bf16x8_t, wp[d][h][nt]), acc[m][nt], 0, 0, 0);
+            for (int nt = 0; nt < NTW; ++nt) acc[m][nt] = mfma16<F16>(av, wp[d][h][nt], acc[m][nt]);
           }
         issue_pair(j0 + d + DP, xp[d], wp[d]);
       }
@@ -577,11 +582,9 @@ __global__ __launch_bounds__(kKsWaves * 64) void pre_kstream_kernel(PreArgs a) {
             acc[m][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, acc[m][nt], 0, 0, 0);
           }
         } else {
-          const bf16x8_t av = __builtin_bit_cast(bf16x8_t, x_norm_chunk(xs[d][m][0], inv_r[m]));
+          const U32x4 av = x_norm_chunk<F16>(xs[d][m][0], inv_r[m]);
 #pragma unroll
-          for (int nt = 0; nt < NTW; ++nt)
-            acc[m][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                av, __builtin_bit_cast(bf16x8_t, ws[d][nt]), acc[m][nt], 0, 0, 0);
+          for (int nt = 0; nt < NTW; ++nt) acc[m][nt] = mfma16<F16>(av, ws[d][nt], acc[m][nt]);
         }
       }
       issue(j0 + d + D, xs[d], ws[d], wl[F32 ? d : 0]);
@@ -658,14 +661,19 @@ __global__ __launch_bounds__(kKsWaves * 64) void pre_kstream_kernel(PreArgs a) {
         buf_store16_nt(rsub, tt < valid ? (uint32_t)(tt * C + c) * ES : kBufOob, o);
         continue;
       }
-      uint32_t hlo[N];
-      uint32_t hhi[N];
+      U32x4 pk;
+      if constexpr (F16) {
+        pk = preagg_chunk_f16<N>(xv[b], sh.hpre[ts]);
+      } else {
+        uint32_t hlo[N];
+        uint32_t hhi[N];
 #pragma unroll
-      for (int i = 0; i < N; ++i) {
-        hlo[i] = pack_lo(sh.hpre[ts][i]);
-        hhi[i] = pack_hi(sh.hpre[ts][i]);
+        for (int i = 0; i < N; ++i) {
+          hlo[i] = pack_lo(sh.hpre[ts][i]);
+          hhi[i] = pack_hi(sh.hpre[ts][i]);
+        }
+        pk = preagg_chunk<N>(xv[b], hlo, hhi);
       }
-      const U32x4 pk = preagg_chunk<N>(xv[b], hlo, hhi);
       if constexpr (NORM) {
         if (tt < TM) nsh.stash[tt * NS::kChunks + (c >> 3)] = pk;
         continue;
@@ -777,7 +785,7 @@ __global__ __launch_bounds__(kKsWaves * 64) void pre_kstream_kernel(PreArgs a) {
     for (int ch = jl; ch < C8; ch += LPT) {
       const U32x4 pk = nsh.stash[tt * NS::kChunks + ch];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) q2 = dot2_bf16(pk.v[j], pk.v[j], q2);
+      for (int j = 0; j < 4; ++j) q2 = sumsq2<F16>(pk.v[j], q2);
     }
     q2 = ks_token_sum<LPT>(q2);
     if (jl == 0) nsh.scale[tt] = 1.0f / sqrtf(q2 / (float)C + a.norm_eps);
@@ -790,13 +798,40 @@ __global__ __launch_bounds__(kKsWaves * 64) void pre_kstream_kernel(PreArgs a) {
       const float4 w0 = *reinterpret_cast<const float4*>(&nsh.gain[c]);
       const float4 w1 = *reinterpret_cast<const float4*>(&nsh.gain[c + 4]);
       U32x4 y;
-      y.v[0] = pack_bf16x2(bf16lo(pk.v[0]) * sc * w0.x, bf16hi(pk.v[0]) * sc * w0.y);
-      y.v[1] = pack_bf16x2(bf16lo(pk.v[1]) * sc * w0.z, bf16hi(pk.v[1]) * sc * w0.w);
-      y.v[2] = pack_bf16x2(bf16lo(pk.v[2]) * sc * w1.x, bf16hi(pk.v[2]) * sc * w1.y);
-      y.v[3] = pack_bf16x2(bf16lo(pk.v[3]) * sc * w1.z, bf16hi(pk.v[3]) * sc * w1.w);
+      y.v[0] = pack2<F16>(elem_lo<F16>(pk.v[0]) * sc * w0.x, elem_hi<F16>(pk.v[0]) * sc * w0.y);
+      y.v[1] = pack2<F16>(elem_lo<F16>(pk.v[1]) * sc * w0.z, elem_hi<F16>(pk.v[1]) * sc * w0.w);
+      y.v[2] = pack2<F16>(elem_lo<F16>(pk.v[2]) * sc * w1.x, elem_hi<F16>(pk.v[2]) * sc * w1.y);
+      y.v[3] = pack2<F16>(elem_lo<F16>(pk.v[3]) * sc * w1.z, elem_hi<F16>(pk.v[3]) * sc * w1.w);
       buf_store16_nt(rsub, it < valid ? (uint32_t)(it * C + c) * 2u : kBufOob, y);
     }
   }
+}
+
+// 16-bit streams: chunk pairs where a pair's 64 columns lie in one stream
+// (C % 64 == 0), the norm in the launch where it fits, else in a second one.
+template <int N, int MODE, bool F16>
+hipError_t launch_pre_kstream_16(const PreArgs& a, unsigned tiles, hipStream_t s) {
+  const dim3 block(KsPlan<N, MODE>::WAVES * 64);
+  auto run = [&](auto norm, const PreArgs& args) {
+    constexpr bool NORM = decltype(norm)::value;
+    if constexpr (ks_pairs<N, MODE>()) {
+      if (args.C % 64 == 0) {
+        hipLaunchKernelGGL((pre_kstream_kernel<N, MODE, NORM, false, true, F16>), dim3(tiles), block, 0, s, args);
+        return hipGetLastError();
+      }
+    }
+    hipLaunchKernelGGL((pre_kstream_kernel<N, MODE, NORM, false, false, F16>), dim3(tiles), block, 0, s, args);
+    return hipGetLastError();
+  };
+  if (!a.norm_w) return run(std::false_type{}, a);
+  if constexpr (ks_norm_fits<N, MODE>()) {
+    if (a.C <= kKsNormMaxC) return run(std::true_type{}, a);
+  }
+  PreArgs plain = a;
+  plain.norm_w = nullptr;
+  const hipError_t e = run(std::false_type{}, plain);
+  if (e != hipSuccess) return e;
+  return launch_expand_norm(a.sub_in, a.x_dtype, a.norm_w, a.norm_dtype, a.sub_in, a.M, 1, a.C, a.norm_eps, s);
 }
 
 template <int N, int MODE>
@@ -817,41 +852,8 @@ hipError_t launch_pre_kstream_inst(const PreArgs& a, hipStream_t s) {
     }
     return hipErrorInvalidValue;
   }
-  // chunk pairs where a pair's 64 columns lie in one stream (C % 64 == 0)
-  const bool pairs = ks_pairs<N, MODE>() && a.C % 64 == 0;
-  if (!a.norm_w) {
-    if constexpr (ks_pairs<N, MODE>()) {
-      if (pairs) {
-        hipLaunchKernelGGL((pre_kstream_kernel<N, MODE, false, false, true>), dim3((unsigned)tiles), block, 0, s, a);
-        return hipGetLastError();
-      }
-    }
-    hipLaunchKernelGGL((pre_kstream_kernel<N, MODE, false>), dim3((unsigned)tiles), block, 0, s, a);
-    return hipGetLastError();
-  }
-  if constexpr (ks_norm_fits<N, MODE>()) {
-    if (a.C <= kKsNormMaxC) {
-      if constexpr (ks_pairs<N, MODE>()) {
-        if (pairs) {
-          hipLaunchKernelGGL((pre_kstream_kernel<N, MODE, true, false, true>), dim3((unsigned)tiles), block, 0, s, a);
-          return hipGetLastError();
-        }
-      }
-      hipLaunchKernelGGL((pre_kstream_kernel<N, MODE, true>), dim3((unsigned)tiles), block, 0, s, a);
-      return hipGetLastError();
-    }
-  }
-  PreArgs plain = a;
-  plain.norm_w = nullptr;
-  if constexpr (ks_pairs<N, MODE>()) {
-    if (pairs) hipLaunchKernelGGL((pre_kstream_kernel<N, MODE, false, false, true>), dim3((unsigned)tiles), block, 0, s, plain);
-    else hipLaunchKernelGGL((pre_kstream_kernel<N, MODE, false>), dim3((unsigned)tiles), block, 0, s, plain);
-  } else {
-    hipLaunchKernelGGL((pre_kstream_kernel<N, MODE, false>), dim3((unsigned)tiles), block, 0, s, plain);
-  }
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return launch_expand_norm(a.sub_in, kBF16, a.norm_w, a.norm_dtype, a.sub_in, a.M, 1, a.C, a.norm_eps, s);
+  return a.x_dtype == kF16 ? launch_pre_kstream_16<N, MODE, true>(a, (unsigned)tiles, s)
+                           : launch_pre_kstream_16<N, MODE, false>(a, (unsigned)tiles, s);
 }
 
 template <int N>

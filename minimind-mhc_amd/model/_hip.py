@@ -19,6 +19,7 @@ LIB_PATH = Path(os.environ.get("MHC_AMD_LIB") or
                 Path(__file__).resolve().parent.parent / "libmhc_amd.so")
 
 DTYPE_F32, DTYPE_BF16, DTYPE_F16 = 0, 1, 2
+PHI_F16_IMAGE = 0x100
 MODE_FULL, MODE_NOHRES, MODE_HEAD, MODE_RMS = 0, 1, 2, 3
 _DTYPE_TAG = {torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16}
 
@@ -34,6 +35,7 @@ _SIGNATURES = {
     "mhc_init": (_I, []),
     "mhc_phi_packed_bytes": (_I64, [_I, _I, _I]),
     "mhc_phi_pack": (_I, [_P, _I, _P, _I, _I, _I, _P]),
+    "mhc_phi_pack_f16": (_I, [_P, _P, _I, _I, _I, _P]),
     "mhc_phi_split_bytes": (_I64, [_I, _I, _I]),
     "mhc_phi_pack_split": (_I, [_P, _I, _P, _I, _I, _I, _P]),
     "mhc_pre_fwd": (_I, [_P, _I, _P, _I, _P,              # x, x_dt, phi, phi_dt, packed

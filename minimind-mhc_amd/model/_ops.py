@@ -84,7 +84,8 @@ class PhiPack:
             training: Optional[bool] = None) -> Optional[torch.Tensor]:
         """The image of phi (None when (n, C, dtype) has no MFMA kernel): the
         bf16 operand image for a bf16 phi (kernels for bf16 streams), the
-        split hi / lo image for an fp32 phi (kernels for fp32 streams).
+        split hi / lo image for an fp32 phi (kernels for fp32 streams), the
+        fp16 image for an fp16 phi (kernels for fp16 streams).
         training: whether phi trains in this call; default grad mode and
         phi.requires_grad (inside an autograd Function's forward, where grad
         mode is off, pass grad_wanted(ctx, <phi's index>))."""
@@ -95,6 +96,11 @@ class PhiPack:
         elif phi.dtype == torch.float32:
             nbytes = lib.mhc_phi_split_bytes(n, C, self.mode)
             pack = lib.mhc_phi_pack_split
+        elif phi.dtype == torch.float16 and n > 1:
+            nbytes = lib.mhc_phi_packed_bytes(n, C, self.mode)
+
+            def pack(w, _dtype, buf, *rest):
+                return lib.mhc_phi_pack_f16(w, buf, *rest)
         else:
             return None
         if nbytes <= 0:
@@ -208,6 +214,12 @@ class StreamChain:
         return out
 
 
+def _phi_tag(phi: torch.Tensor, packed: Optional[torch.Tensor]) -> int:
+    """phi's dtype tag, saying that `packed` is an fp16 image where it is one."""
+    tag = H.dtype_tag(phi)
+    return tag | H.PHI_F16_IMAGE if packed is not None and tag == H.DTYPE_F16 else tag
+
+
 def _check_numel(name: str, t: torch.Tensor, want: int) -> None:
     # The kernels index biases by stream / matrix element; a short tensor would be
     # read out of bounds, so sizes are enforced here (the C ABI sees only pointers).
@@ -273,7 +285,7 @@ def pre_full(x_flat, phi, packed, a_pre, b_pre, a_post, b_post, a_res, b_res, n,
         "inv_rms": torch.empty(M, dtype=torch.float32, device=dev) if want_saved else None,
         "mixes_raw": torch.empty(M, FD, dtype=torch.float32, device=dev) if want_saved else None,
     }
-    args = (x2.data_ptr(), H.dtype_tag(x2), phi_c.data_ptr(), H.dtype_tag(phi_c), H.ptr(packed),
+    args = (x2.data_ptr(), H.dtype_tag(x2), phi_c.data_ptr(), _phi_tag(phi_c, packed), H.ptr(packed),
             a_pre.data_ptr(), b_pre.data_ptr(), a_post.data_ptr(), b_post.data_ptr(),
             a_res.data_ptr(), b_res.data_ptr(), H.dtype_tag(a_pre),
             out["sub_in"].data_ptr(), H.ptr(out["h_pre"]), out["h_post"].data_ptr(),
@@ -312,7 +324,7 @@ def pre_nohres(x_flat, phi, packed, a_pre, b_pre, a_post, b_post, n, C, post_mul
         "inv_rms": torch.empty(M, dtype=torch.float32, device=dev) if want_saved else None,
         "mixes_raw": torch.empty(M, FD, dtype=torch.float32, device=dev) if want_saved else None,
     }
-    args = (x2.data_ptr(), H.dtype_tag(x2), phi_c.data_ptr(), H.dtype_tag(phi_c), H.ptr(packed),
+    args = (x2.data_ptr(), H.dtype_tag(x2), phi_c.data_ptr(), _phi_tag(phi_c, packed), H.ptr(packed),
             a_pre.data_ptr(), b_pre.data_ptr(), a_post.data_ptr(), b_post.data_ptr(),
             H.dtype_tag(a_pre), out["sub_in"].data_ptr(), H.ptr(out["h_pre"]),
             out["h_post"].data_ptr(), H.ptr(out["inv_rms"]), H.ptr(out["mixes_raw"]),
@@ -347,7 +359,7 @@ def head(x_flat, phi, packed, alpha, bias, n, C, pre_eps, rms_eps, *, want_saved
         _check_numel("alpha", alpha_c, 1)
         _check_numel("bias", bias_c, n)
         phi_p, a_p, b_p = phi_c.data_ptr(), alpha_c.data_ptr(), bias_c.data_ptr()
-        phi_dt, pdt = H.dtype_tag(phi_c), H.dtype_tag(alpha_c)
+        phi_dt, pdt = _phi_tag(phi_c, packed), H.dtype_tag(alpha_c)
     out = torch.empty(M, C, dtype=x2.dtype, device=dev)
     inv = torch.empty(M, dtype=torch.float32, device=dev) if want_saved else None
     mix = torch.empty(M, n, dtype=torch.float32, device=dev) if (want_saved and n > 1) else None
