@@ -388,6 +388,18 @@ int mhc_pre_bwd(const void* x, int x_dtype, const void* phi, int phi_dtype, cons
                 float* g_raw, int64_t M, int n, int C, int mode, float post_mult, float pre_eps,
                 hipStream_t stream);
 
+/* mhc_pre_bwd with g_x_in [M, n*C] (x_dtype, or NULL) added to g_x: the gradient
+ * that reaches x past the pre phase (the post phase's).  g_x is rounded to
+ * x_dtype before and after the addition, as adding the two tensors would.
+ * MHC_MODE_FULL and MHC_MODE_NOHRES. */
+int mhc_pre_bwd_add(const void* x, int x_dtype, const void* phi, int phi_dtype, const void* alpha_pre,
+                const void* bias_pre, const void* alpha_post, const void* bias_post,
+                const void* alpha_res, int param_dtype, const float* inv_rms,
+                const float* mixes_raw, const void* g_sub, const void* g_h_pre,
+                const void* g_h_post, const void* g_h_res_raw, int grad_dtype, const void* g_x_in, void* g_x,
+                float* g_raw, int64_t M, int n, int C, int mode, float post_mult, float pre_eps,
+                hipStream_t stream);
+
 /* Workspace bytes mhc_pre_bwd_weights needs for (M, n, C, mode). */
 int64_t mhc_pre_bwd_weights_workspace_bytes(int64_t M, int n, int C, int mode);
 

@@ -537,13 +537,13 @@ int mhc_post_nohres_bwd(const void* h_post, int h_dtype, const void* f_out, int 
   return hip_status(mhc::launch_post_bwd(a, stream), fn);
 }
 
-int mhc_pre_bwd(const void* x, int x_dtype, const void* phi, int phi_dtype, const void* alpha_pre,
-                const void* bias_pre, const void* alpha_post, const void* bias_post,
-                const void* alpha_res, int param_dtype, const float* inv_rms,
-                const float* mixes_raw, const void* g_sub, const void* g_h_pre,
-                const void* g_h_post, const void* g_h_res_raw, int grad_dtype, void* g_x,
-                float* g_raw, int64_t M, int n, int C, int mode, float post_mult, float pre_eps,
-                hipStream_t stream) {
+int mhc_pre_bwd_add(const void* x, int x_dtype, const void* phi, int phi_dtype, const void* alpha_pre,
+                    const void* bias_pre, const void* alpha_post, const void* bias_post,
+                    const void* alpha_res, int param_dtype, const float* inv_rms,
+                    const float* mixes_raw, const void* g_sub, const void* g_h_pre,
+                    const void* g_h_post, const void* g_h_res_raw, int grad_dtype, const void* g_x_in,
+                    void* g_x, float* g_raw, int64_t M, int n, int C, int mode, float post_mult, float pre_eps,
+                    hipStream_t stream) {
   const char* fn = "mhc_pre_bwd";
   if (M < 0 || n < 1 || n > kMaxN || C < 1) return fail(hipErrorInvalidValue, "%s: bad shape (M=%lld n=%d C=%d)", fn, (long long)M, n, C);
   if (mode != mhc::kFull && mode != mhc::kNoHres && mode != mhc::kHead && mode != mhc::kRms)
@@ -561,7 +561,9 @@ int mhc_pre_bwd(const void* x, int x_dtype, const void* phi, int phi_dtype, cons
     if (mode == mhc::kFull && !alpha_res) return fail(hipErrorInvalidValue, "%s: alpha_res is required", fn);
     if (mode == mhc::kHead && n == 1) return fail(hipErrorInvalidValue, "%s: MHCHead with n == 1 is mode MHC_MODE_RMS", fn);
   }
+  if (g_x_in && mode != mhc::kFull && mode != mhc::kNoHres) return fail(hipErrorInvalidValue, "%s: g_x_in needs the full or no-H_res mode", fn);
   mhc::PreBwdArgs a{};
+  a.g_x_in = g_x_in;
   a.x = x; a.phi = phi;
   a.alpha[0] = alpha_pre; a.alpha[1] = alpha_post; a.alpha[2] = alpha_res;
   a.bias[0] = bias_pre; a.bias[1] = bias_post; a.bias[2] = nullptr;
@@ -572,6 +574,18 @@ int mhc_pre_bwd(const void* x, int x_dtype, const void* phi, int phi_dtype, cons
   a.x_dtype = x_dtype; a.phi_dtype = phi_dtype; a.param_dtype = param_dtype; a.grad_dtype = grad_dtype;
   a.post_mult = post_mult; a.pre_eps = pre_eps;
   return hip_status(mhc::launch_pre_bwd(a, stream), fn);
+}
+
+int mhc_pre_bwd(const void* x, int x_dtype, const void* phi, int phi_dtype, const void* alpha_pre,
+                const void* bias_pre, const void* alpha_post, const void* bias_post,
+                const void* alpha_res, int param_dtype, const float* inv_rms,
+                const float* mixes_raw, const void* g_sub, const void* g_h_pre,
+                const void* g_h_post, const void* g_h_res_raw, int grad_dtype, void* g_x,
+                float* g_raw, int64_t M, int n, int C, int mode, float post_mult, float pre_eps,
+                hipStream_t stream) {
+  return mhc_pre_bwd_add(x, x_dtype, phi, phi_dtype, alpha_pre, bias_pre, alpha_post, bias_post, alpha_res,
+                         param_dtype, inv_rms, mixes_raw, g_sub, g_h_pre, g_h_post, g_h_res_raw, grad_dtype,
+                         nullptr, g_x, g_raw, M, n, C, mode, post_mult, pre_eps, stream);
 }
 
 int64_t mhc_pre_bwd_weights_workspace_bytes(int64_t M, int n, int C, int mode) {

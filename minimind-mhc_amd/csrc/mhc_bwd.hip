@@ -8,6 +8,8 @@
 //                s_* = sigmoid(alpha_* * mixes + bias_*)
 //   gxn[k]     = sum_f alpha_seg(f) g_raw[f] * phi[k, f]
 //   g_x[k]     = inv * (gxn[k] - xn[k] * mean_k(xn * gxn)) + (s_pre[i(k)] + pre_eps) * g_sub[c(k)]
+//                (rounded to x's type; with g_x_in that is added and rounded again, as a
+//                separate addition of the two gradients rounds)
 //   with mean_k(xn * gxn) = sum_f alpha_seg(f) g_raw[f] mixes_raw[f] / (n*C), since
 //   mixes_raw[f] = sum_k xn[k] phi[k, f] (the saved fp32 projection).
 // The per-token g_raw (fp32) feeds the weight gradients (model/mhc_fused.py:696-711):
@@ -111,7 +113,9 @@ __global__ __launch_bounds__(256) void pre_bwd_generic_kernel(PreBwdArgs a) {
     const int c = (int)(k - (int64_t)i * C);
     const float xn = ld_any(a.x, xb + k, xdt) * inv;
     const float gs = a.g_sub ? ld_any(a.g_sub, tok * C + c, gdt) : 0.f;
-    st_any(a.g_x, xb + k, xdt, inv * (gxn - xn * mean) + s_h[i] * gs);
+    float v = inv * (gxn - xn * mean) + s_h[i] * gs;
+    if (a.g_x_in) v = round_to(v, xdt) + ld_any(a.g_x_in, xb + k, xdt);
+    st_any(a.g_x, xb + k, xdt, v);
   }
 }
 
@@ -242,7 +246,10 @@ constexpr bool kPreBwdPhiBlock = true;
 // its own (no barrier: one wave writes and reads it, in order).  The MFMA
 // layout alone covers 16 rows x 64 bytes per load or store, half of each
 // 128-byte line.
-template <int N, int MODE, int NW, int KJ, bool F32, bool RS = false>
+// ADD: g_x_in (the gradient that reached x past the pre phase) is added at the
+// g_x store, where it costs one read; as a launch of its own the addition reads
+// two streams and writes one.
+template <int N, int MODE, int NW, int KJ, bool F32, bool RS = false, bool ADD = false>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(F32 ? 2 : 4))) void pre_bwd_mfma_kernel(PreBwdArgs a) {
   using XV = Chunk8<F32>;
   static_assert(!RS || ((!F32 || N <= 4) && KJ % 2 == 0), "row pieces: x resident, whole chunk pairs");
@@ -298,6 +305,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(F32 ? 2
   const auto rgs = make_rsrc(a.g_sub ? static_cast<const unsigned char*>(a.g_sub) + t0 * C * ES : nullptr,
                              a.g_sub ? (uint32_t)valid * C * ES : 0u);
   const auto rgx = make_rsrc(static_cast<unsigned char*>(a.g_x) + t0 * NC * ES, (uint32_t)valid * NC * ES);
+
+  const auto rgi = make_rsrc(ADD ? static_cast<const unsigned char*>(a.g_x_in) + t0 * NC * ES : nullptr,
+                             ADD ? (uint32_t)valid * NC * ES : 0u);
 
   // chunk j of this wave: stream ci, first column c0; lane column c0 + 8g
   // (RS: chunks 2 (wave + NW j/2) + j % 2, pairs of adjacent ones)
@@ -573,15 +583,30 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(F32 ? 2
     if constexpr (!XRES) in.xv[0] = x_chunk(j);
   };
   // 16 chunks a wave, or x streamed with the chunk: four sets would spill
-  constexpr int PD = PF ? (KJ <= 12 && XRES ? 4 : 2) : 1;
+  constexpr int PD = PF ? (KJ <= 12 && XRES ? (ADD && !F32 && KJ == 12 ? 3 : 4) : 2) : 1;
   ChunkIn cin[PD];
   if constexpr (PF) {
 #pragma unroll
     for (int p = 0; p < PD - 1; ++p)
       if (p < KJ) load_chunk(p, cin[p]);
   }
+  U32x4 gin[ADD && RS ? NRI : 1];  // row pieces of the pair's g_x_in
+  auto load_gin = [&](int j) {
+    const int col = 64 * (wave + NW * (j >> 1));
+#pragma unroll
+    for (int i = 0; i < NRI; ++i) {
+      const int tt = RPI * i + lane / PPR;
+      const int pc = lane % PPR;
+      gin[i] = buf_load16(rgi, col + pc * (16 / (int)ES) < NC ? (uint32_t)(tt * NC + col) * ES + 16u * pc : kBufOob);
+    }
+  };
+  // issued with the pair's first chunk; at 12 and 16 bf16 chunks a wave, where
+  // that spills, after the second chunk's products
+  constexpr bool GIN_LATE = !F32 && KJ >= 12;
 #pragma unroll
   for (int j = 0; j < KJ; ++j) {
+    if constexpr (ADD && RS && !GIN_LATE)
+      if ((j & 1) == 0) load_gin(j);
     ChunkIn& cur = cin[PF ? (j % PD) : 0];
     if constexpr (PF) {
       if (j + PD - 1 < KJ) load_chunk(j + PD - 1, cin[(j + PD - 1) % PD]);
@@ -644,6 +669,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(F32 ? 2
       }
       d2[h] = d;
     }
+    if constexpr (ADD && RS && GIN_LATE)
+      if (j & 1) load_gin(j);
     const XV gv = PF || CH ? cur.gv : XV::load(rgs, ok ? (uint32_t)(r * C + c0 + 8 * g) * ES : kBufOob);
     XV xj;
     if constexpr (XRES) xj = xs[j];
@@ -673,29 +700,42 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(F32 ? 2
         for (int i = 0; i < NRI; ++i) {
           const int tt = RPI * i + lane / PPR;
           const int pc = lane % PPR;
-          buf_store16(rgx, col + pc * (16 / (int)ES) < NC ? (uint32_t)(tt * NC + col) * ES + 16u * pc : kBufOob,
-                      s_rs[wave][tt][pc ^ (tt & 7)]);
+          U32x4 w = s_rs[wave][tt][pc ^ (tt & 7)];
+          if constexpr (ADD) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              if constexpr (F32) w.v[q] = __float_as_uint(__uint_as_float(w.v[q]) + __uint_as_float(gin[i].v[q]));
+              else w.v[q] = pack_bf16x2(bf16lo(w.v[q]) + bf16lo(gin[i].v[q]), bf16hi(w.v[q]) + bf16hi(gin[i].v[q]));
+            }
+          }
+          buf_store16(rgx, col + pc * (16 / (int)ES) < NC ? (uint32_t)(tt * NC + col) * ES + 16u * pc : kBufOob, w);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }
     } else {
-      XV::store(rgx, ok ? (uint32_t)(r * NC + ci * C + c0 + 8 * g) * ES : kBufOob, v);
+      const uint32_t off = ok ? (uint32_t)(r * NC + ci * C + c0 + 8 * g) * ES : kBufOob;
+      if constexpr (ADD) {
+        const XV gi = XV::load(rgi, off);
+#pragma unroll
+        for (int cc = 0; cc < 8; ++cc) v[cc] = (F32 ? v[cc] : round_to(v[cc], kBF16)) + XV::get(gi, cc);
+      }
+      XV::store(rgx, off, v);
     }
   }
 }
 
 // Chunks per wave instantiated: 2 .. 16 in steps that cover C <= 1024 for
 // n in {2, 4} (8 waves) and n = 8 (16 waves, bf16 only).
-template <int N, int MODE, int NW, int KJ, bool F32>
+template <int N, int MODE, int NW, int KJ, bool F32, bool ADD>
 static hipError_t launch_pre_bwd_inst(const PreBwdArgs& a, hipStream_t s) {
   if constexpr (kPreBwdRowPieces && (!F32 || N <= 4) && KJ % 2 == 0) {
     if (a.C % 64 == 0) {  // a chunk pair's 64 columns in one stream's row
-      hipLaunchKernelGGL((pre_bwd_mfma_kernel<N, MODE, NW, KJ, F32, true>), dim3((unsigned)((a.M + 15) / 16)),
+      hipLaunchKernelGGL((pre_bwd_mfma_kernel<N, MODE, NW, KJ, F32, true, ADD>), dim3((unsigned)((a.M + 15) / 16)),
                          dim3(NW * 64), 0, s, a);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((pre_bwd_mfma_kernel<N, MODE, NW, KJ, F32>), dim3((unsigned)((a.M + 15) / 16)),
+  hipLaunchKernelGGL((pre_bwd_mfma_kernel<N, MODE, NW, KJ, F32, false, ADD>), dim3((unsigned)((a.M + 15) / 16)),
                      dim3(NW * 64), 0, s, a);
   return hipGetLastError();
 }
@@ -704,7 +744,11 @@ template <int N, int MODE, int NW, bool F32, int... KJS>
 static hipError_t launch_pre_bwd_mfma_kj(const PreBwdArgs& a, int kj, hipStream_t s) {
   hipError_t r = hipErrorInvalidValue;
   bool done = false;
-  ((!done && KJS >= kj ? (r = launch_pre_bwd_inst<N, MODE, NW, KJS, F32>(a, s), done = true) : false), ...);
+  // MHCHead's input goes nowhere else: no gradient to add (mhc_pre_bwd refuses one)
+  if (MODE != kHead && a.g_x_in)
+    ((!done && KJS >= kj ? (r = launch_pre_bwd_inst<N, MODE, NW, KJS, F32, MODE != kHead>(a, s), done = true) : false), ...);
+  else
+    ((!done && KJS >= kj ? (r = launch_pre_bwd_inst<N, MODE, NW, KJS, F32, false>(a, s), done = true) : false), ...);
   return r;
 }
 
@@ -730,7 +774,7 @@ static bool pre_bwd_mfma_ok(const PreBwdArgs& a) {
   if (fd % 8 != 0 && fd != 4 && fd != 2) return false;  // whole 8-feature operands, or one short one
   if (a.C % 8 != 0 || a.C > 32 * kMfmaMaxColBlocks) return false;
   if ((int64_t)a.n * a.C * mode_fd(a.mode, a.n) * dtype_bytes(a.x_dtype) > 0x7fffffffLL) return false;
-  return al(a.x) && al(a.phi) && al(a.g_x) && (a.g_sub == nullptr || al(a.g_sub));
+  return al(a.x) && al(a.phi) && al(a.g_x) && al(a.g_sub) && al(a.g_x_in);  // null is aligned
 }
 
 template <int N, bool F32>

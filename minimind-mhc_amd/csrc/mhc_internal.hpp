@@ -104,6 +104,7 @@ struct PreBwdArgs {
   const void* g_hpre;     // [M, n]
   const void* g_hpost;    // [M, n]
   const void* g_hres;     // [M, n*n] d h_res_raw
+  const void* g_x_in;     // [M, n*C]  x_dtype: added to g_x, or null (full and no-H_res modes)
   void* g_x;              // [M, n*C]  x_dtype
   float* g_raw;           // [M, FD]   fp32: d(alpha*m + bias) per segment (null for kRms)
   int64_t M;

@@ -77,6 +77,12 @@ _SIGNATURES = {
                          _P, _P, _P, _P, _I,              # g_sub, g_h_pre, g_h_post, g_h_res_raw, grad_dt
                          _P, _P,                          # g_x, g_raw
                          _I64, _I, _I, _I, _F, _F, _P]),
+    "mhc_pre_bwd_add": (_I, [_P, _I, _P, _I,                  # x, x_dt, phi, phi_dt
+                         _P, _P, _P, _P, _P, _I,          # a_pre, b_pre, a_post, b_post, a_res, param_dt
+                         _P, _P,                          # inv_rms, mixes_raw
+                         _P, _P, _P, _P, _I,              # g_sub, g_h_pre, g_h_post, g_h_res_raw, grad_dt
+                         _P, _P, _P,                      # g_x_in, g_x, g_raw
+                         _I64, _I, _I, _I, _F, _F, _P]),
     "mhc_pre_bwd_weights_workspace_bytes": (_I64, [_I64, _I, _I, _I]),
     "mhc_pre_bwd_weights": (_I, [_P, _I, _P, _P, _P,      # x, x_dt, inv, mixes, g_raw
                                  _P, _P, _P, _I,          # alphas, param_dt

@@ -507,9 +507,10 @@ def post_bwd(x_flat, h_res, h_post, f_out, n, C, g_out):
 
 
 def pre_bwd(x2, phi, alphas, biases, inv_rms, mixes, n, C, mode, post_mult, pre_eps,
-            g_sub=None, g_hpre=None, g_hpost=None, g_hres=None):
+            g_sub=None, g_hpre=None, g_hpost=None, g_hres=None, g_x_in=None):
     """Per-token pre-phase backward.  alphas / biases: (pre, post, res) with
-    None for absent segments.  Returns (g_x [M, n*C] x dtype, g_raw [M, FD] fp32
+    None for absent segments.  g_x_in: a gradient of x from elsewhere, added to
+    g_x in the same launch.  Returns (g_x [M, n*C] x dtype, g_raw [M, FD] fp32
     or None for mode RMS)."""
     grads = [g for g in (g_sub, g_hpre, g_hpost, g_hres) if g is not None]
     dev = H.require_device(x2, inv_rms, *grads)
@@ -517,6 +518,9 @@ def pre_bwd(x2, phi, alphas, biases, inv_rms, mixes, n, C, mode, post_mult, pre_
     gdt = grads[0].dtype if grads else x2.dtype
     g_sub, g_hpre, g_hpost, g_hres = (None if g is None else g.to(gdt).contiguous()
                                       for g in (g_sub, g_hpre, g_hpost, g_hres))
+    if g_x_in is not None:
+        H.require_device(x2, g_x_in)
+        g_x_in = g_x_in.to(x2.dtype).reshape(x2.shape).contiguous()
     g_x = torch.empty_like(x2)
     if mode == H.MODE_RMS:
         phi_p = phi_dt = None
@@ -533,11 +537,11 @@ def pre_bwd(x2, phi, alphas, biases, inv_rms, mixes, n, C, mode, post_mult, pre_
               for p in (alphas[0], biases[0], alphas[1], biases[1], alphas[2])]
         pdt = H.dtype_tag(ps[0])
         g_raw = torch.empty(M, FD, dtype=torch.float32, device=dev)
-    rc = H.load().mhc_pre_bwd(
+    rc = H.load().mhc_pre_bwd_add(
         x2.data_ptr(), H.dtype_tag(x2), phi_p, phi_dt if phi_dt is not None else H.DTYPE_F32,
         *[H.ptr(p) for p in ps], pdt, inv_rms.data_ptr(), H.ptr(mixes),
         H.ptr(g_sub), H.ptr(g_hpre), H.ptr(g_hpost), H.ptr(g_hres),
-        H.dtype_tag(g_sub if g_sub is not None else x2), g_x.data_ptr(), H.ptr(g_raw),
+        H.dtype_tag(g_sub if g_sub is not None else x2), H.ptr(g_x_in), g_x.data_ptr(), H.ptr(g_raw),
         M, n, C, mode, float(post_mult), float(pre_eps), H.stream(dev))
     H.check(rc, "mhc_pre_bwd")
     return g_x, g_raw

@@ -64,11 +64,11 @@ def sinkhorn_normalize(M: torch.Tensor, iters: int = 10, eps: float = 1e-6) -> t
 # --------------------------------------------------------- pre / post phases
 
 def _pre_full_grads(x2, w, alphas, biases, inv, mixes, n, c, post_mult, pre_eps, shape,
-                    g_sub, g_hpre, g_hpost, g_hres_raw):
+                    g_sub, g_hpre, g_hpost, g_hres_raw, g_pass=None):
     """(g_x, g_phi, g_alpha_pre, g_bias_pre, g_alpha_post, g_bias_post, g_alpha_res,
     g_bias_res) of the full pre phase, each in its forward input's dtype and shape."""
     g_x, g_raw = _ops.pre_bwd(x2, w, alphas, biases, inv, mixes, n, c, H.MODE_FULL, post_mult,
-                              pre_eps, g_sub, g_hpre, g_hpost, g_hres_raw)
+                              pre_eps, g_sub, g_hpre, g_hpost, g_hres_raw, g_x_in=g_pass)
     g_w, g_a, g_b = _ops.pre_bwd_weights(x2, inv, mixes, g_raw, w, alphas, n, c, H.MODE_FULL)
     out = [g_x.view(shape), g_w]
     for a, b, ga, gb in zip(alphas, biases, g_a, g_b):
@@ -110,11 +110,16 @@ class _PrePhaseFullFn(_ops.GradAwareFunction):
 class _PreSinkhornFn(_ops.GradAwareFunction):
     """Fused pre phase + Sinkhorn -> (sublayer_in, h_post, h_res): the single
     launch MHCConnection_Fused.forward uses in place of the reference's
-    _PrePhaseFullFn + sinkhorn_normalize pair (model/mhc_fused.py:820-830)."""
+    _PrePhaseFullFn + sinkhorn_normalize pair (model/mhc_fused.py:820-830).
+
+    pass_x: also return x_flat itself, for the post phase to read.  Its gradient
+    then arrives here, and the pre-phase launch adds it to its own as it stores
+    g_x; otherwise autograd sums the two in a launch of its own."""
 
     @staticmethod
     def forward(ctx, x_flat, w_phi, packed, alpha_pre, bias_pre, alpha_post, bias_post,
-                alpha_res, bias_res, post_mult, pre_eps, rms_eps, n, c, iters, sk_eps, ssq=None):
+                alpha_res, bias_res, post_mult, pre_eps, rms_eps, n, c, iters, sk_eps, ssq=None,
+                pass_x=False):
         B, L, NC = x_flat.shape
         train = _ops.grad_wanted(ctx)
         if train:
@@ -127,11 +132,11 @@ class _PreSinkhornFn(_ops.GradAwareFunction):
                                   alpha_pre, bias_pre, alpha_post, bias_post, alpha_res,
                                   bias_res, o["inv_rms"], o["mixes_raw"], o["h_res_raw"])
         ctx.cfg = (n, c, float(post_mult), float(pre_eps), (B, L, NC), iters, float(sk_eps))
-        return (o["sub_in"].view(B, L, c), o["h_post"].view(B, L, n),
-                o["h_res"].view(B, L, n, n))
+        out = (o["sub_in"].view(B, L, c), o["h_post"].view(B, L, n), o["h_res"].view(B, L, n, n))
+        return (*out, x_flat) if pass_x else out
 
     @staticmethod
-    def backward(ctx, g_sub, g_hpost, g_hres):
+    def backward(ctx, g_sub, g_hpost, g_hres, g_pass=None):
         x2, w, a_pre, b_pre, a_post, b_post, a_res, b_res, inv, mixes, raw = ctx.saved_tensors
         n, c, post_mult, pre_eps, shape, iters, sk_eps = ctx.cfg
         g_raw = None
@@ -141,8 +146,8 @@ class _PreSinkhornFn(_ops.GradAwareFunction):
             g_raw = _ops.sinkhorn_bwd(raw, g_hres.reshape(raw.shape), iters, sk_eps,
                                       out_dtype=x2.dtype)
         g = _pre_full_grads(x2, w, (a_pre, a_post, a_res), (b_pre, b_post, b_res), inv, mixes,
-                            n, c, post_mult, pre_eps, shape, g_sub, None, g_hpost, g_raw)
-        return (g[0], g[1], None, *g[2:], None, None, None, None, None, None, None, None)
+                            n, c, post_mult, pre_eps, shape, g_sub, None, g_hpost, g_raw, g_pass)
+        return (g[0], g[1], None, *g[2:], *[None] * 9)
 
 
 class _PostPhaseFullFn(_ops.GradAwareFunction):
@@ -239,12 +244,13 @@ class MHCConnection_Fused(nn.Module):
                 return chain.put(out, ssq_out) if chain is not None else out
             fn = sublayer_fn
             sublayer_fn = lambda z: fn(in_norm(z))  # noqa: E731
-        sublayer_in, h_post, h_res = _PreSinkhornFn.apply(
+        grad = torch.is_grad_enabled()
+        sublayer_in, h_post, h_res, *passed = _PreSinkhornFn.apply(
             x_flat, self.phi_weight, packed,
             self.alpha_pre, self.bias_pre, self.alpha_post, self.bias_post,
             self.alpha_res, self.bias_res,
             self.post_mult_value, self.pre_eps, self.eps, self.n, self.dim,
-            self.sinkhorn_iters, self.sinkhorn_eps, ssq)
+            self.sinkhorn_iters, self.sinkhorn_eps, ssq, grad)
         f_out = sublayer_fn(sublayer_in)
-        out = _PostPhaseFullFn.apply(x_flat, h_res, h_post, f_out, self.n, self.dim, ssq_out)
+        out = _PostPhaseFullFn.apply(passed[0] if grad else x_flat, h_res, h_post, f_out, self.n, self.dim, ssq_out)
         return chain.put(out, ssq_out) if chain is not None else out

@@ -23,11 +23,12 @@ def _is_pow2(n: int) -> bool:
 
 
 class _PrePhaseFn(_ops.GradAwareFunction):
-    """Pre phase -> (sublayer_in, h_pre, h_post) (model/mhc_fused_no_hres.py:397-529)."""
+    """Pre phase -> (sublayer_in, h_pre, h_post) (model/mhc_fused_no_hres.py:397-529),
+    and x_flat itself with pass_x (see mhc_fused._PreSinkhornFn)."""
 
     @staticmethod
     def forward(ctx, x_flat, w_phi, alpha_pre, bias_pre, alpha_post, bias_post,
-                post_mult, pre_eps, rms_eps, n, c, packed=None, ssq=None):
+                post_mult, pre_eps, rms_eps, n, c, packed=None, ssq=None, pass_x=False):
         B, L, NC = x_flat.shape
         train = _ops.grad_wanted(ctx)
         if packed is None:  # called as the reference's Function, without the module's pack
@@ -40,21 +41,22 @@ class _PrePhaseFn(_ops.GradAwareFunction):
                                   alpha_pre, bias_pre, alpha_post, bias_post,
                                   o["inv_rms"], o["mixes_raw"])
         ctx.cfg = (n, c, float(post_mult), float(pre_eps), (B, L, NC))
-        return (o["sub_in"].view(B, L, c), o["h_pre"].view(B, L, n), o["h_post"].view(B, L, n))
+        out = (o["sub_in"].view(B, L, c), o["h_pre"].view(B, L, n), o["h_post"].view(B, L, n))
+        return (*out, x_flat) if pass_x else out
 
     @staticmethod
-    def backward(ctx, g_sub, g_hpre, g_hpost):
+    def backward(ctx, g_sub, g_hpre, g_hpost, g_pass=None):
         x2, w, a_pre, b_pre, a_post, b_post, inv, mixes = ctx.saved_tensors
         n, c, post_mult, pre_eps, shape = ctx.cfg
         alphas, biases = (a_pre, a_post, None), (b_pre, b_post, None)
         g_x, g_raw = _ops.pre_bwd(x2, w, alphas, biases, inv, mixes, n, c, H.MODE_NOHRES,
-                                  post_mult, pre_eps, g_sub, g_hpre, g_hpost)
+                                  post_mult, pre_eps, g_sub, g_hpre, g_hpost, g_x_in=g_pass)
         g_w, g_a, g_b = _ops.pre_bwd_weights(x2, inv, mixes, g_raw, w, alphas, n, c,
                                              H.MODE_NOHRES)
         return (g_x.view(shape), g_w,
                 g_a[0].to(a_pre.dtype).reshape(a_pre.shape), g_b[0].to(b_pre.dtype).view(b_pre.shape),
                 g_a[1].to(a_post.dtype).reshape(a_post.shape), g_b[1].to(b_post.dtype).view(b_post.shape),
-                None, None, None, None, None, None, None)
+                *[None] * 8)
 
 
 class _PostPhaseFn(_ops.GradAwareFunction):
@@ -132,10 +134,12 @@ class MHCConnection_FusedNoHres(nn.Module):
                 return chain.put(out, ssq_out) if chain is not None else out
             fn = sublayer_fn
             sublayer_fn = lambda z: fn(in_norm(z))  # noqa: E731
-        sublayer_in, _h_pre, h_post = _PrePhaseFn.apply(
+        grad = torch.is_grad_enabled()
+        sublayer_in, _h_pre, h_post, *passed = _PrePhaseFn.apply(
             x_flat, self.phi_weight, self.alpha_pre, self.bias_pre,
             self.alpha_post, self.bias_post,
-            self.post_mult_value, self.pre_eps, self.eps, self.n, self.dim, packed, ssq)
+            self.post_mult_value, self.pre_eps, self.eps, self.n, self.dim, packed, ssq,
+            grad)
         f_out = sublayer_fn(sublayer_in)
-        out = _PostPhaseFn.apply(x_flat, h_post, f_out, self.n, self.dim, ssq_out)
+        out = _PostPhaseFn.apply(passed[0] if grad else x_flat, h_post, f_out, self.n, self.dim, ssq_out)
         return chain.put(out, ssq_out) if chain is not None else out
