@@ -522,6 +522,20 @@ int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
                 int64_t workspace_bytes, int64_t M, int hidden, int inter, int experts, int topk,
                 int norm_topk, int dtype, hipStream_t stream);
 
+/* -------------------------------- linear layers of the sublayers (inference)
+ * 16-bit tensors (bf16 or fp16) of one dtype, fp32 sums rounded once; K a
+ * multiple of 32, every weight's row count of 4; pointers 16-byte aligned.
+ */
+
+/* out[i] [M, n[i]] = x [M, K] w[i]^T for `count` (one to three) weights
+ * w[i] [n[i], K]; w, out and n are host arrays. */
+int mhc_linear_fwd(const void* x, const void* const* w, void* const* out, const int* n, int count,
+                   int64_t M, int K, int dtype, hipStream_t stream);
+
+/* out [M, N] = silu(x gate_w^T) * (x up_w^T), gate_w and up_w [N, K]. */
+int mhc_glu_fwd(const void* x, const void* gate_w, const void* up_w, void* out, int64_t M, int K,
+                int N, int dtype, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

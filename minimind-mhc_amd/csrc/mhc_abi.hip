@@ -765,4 +765,44 @@ int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
   return hip_status(mhc::launch_moe(a, stream), fn);
 }
 
+// -------------------------------------------------- linear layers (inference)
+
+static int run_linear(mhc::LinearArgs& a, int dtype, hipStream_t stream, const char* fn) {
+  if (a.M < 0 || a.K < 32 || a.K % 32 != 0) return fail(hipErrorInvalidValue, "%s: bad shape (M=%lld K=%d)", fn, (long long)a.M, a.K);
+  if (dtype != mhc::kBF16 && dtype != mhc::kF16) return fail(hipErrorInvalidValue, "%s: dtype must be bf16 or fp16 (got %d)", fn, dtype);
+  int64_t cols = 0;
+  for (int i = 0; i < a.count; ++i) {
+    if (a.n[i] < 4 || a.n[i] % 4 != 0) return fail(hipErrorInvalidValue, "%s: weight %d has %d rows", fn, i, a.n[i]);
+    cols += a.n[i];
+  }
+  if ((a.M / 64 + 1) * (cols / 32 + 3) > kMaxBlocks) return fail(hipErrorInvalidValue, "%s: too large", fn);
+  if (a.M == 0) return 0;
+  for (int i = 0; i < a.count; ++i)
+    if (!a.w[i] || !aligned16(a.w[i]) || (!(a.glu && i == 1) && (!a.out[i] || !aligned16(a.out[i]))))
+      return fail(hipErrorInvalidValue, "%s: null or unaligned weight or output %d", fn, i);
+  if (!a.x || !aligned16(a.x)) return fail(hipErrorInvalidValue, "%s: null or unaligned x", fn);
+  a.f16 = dtype == mhc::kF16;
+  return hip_status(mhc::launch_linear(a, stream), fn);
+}
+
+int mhc_linear_fwd(const void* x, const void* const* w, void* const* out, const int* n, int count,
+                   int64_t M, int K, int dtype, hipStream_t stream) {
+  const char* fn = "mhc_linear_fwd";
+  if (count < 1 || count > 3 || !w || !out || !n) return fail(hipErrorInvalidValue, "%s: one to three weights (got %d)", fn, count);
+  mhc::LinearArgs a{};
+  for (int i = 0; i < count; ++i) {
+    a.w[i] = w[i]; a.out[i] = out[i]; a.n[i] = n[i];
+  }
+  a.x = x; a.count = count; a.M = M; a.K = K;
+  return run_linear(a, dtype, stream, fn);
+}
+
+int mhc_glu_fwd(const void* x, const void* gate_w, const void* up_w, void* out, int64_t M, int K,
+                int N, int dtype, hipStream_t stream) {
+  mhc::LinearArgs a{};
+  a.x = x; a.w[0] = gate_w; a.w[1] = up_w; a.out[0] = out;
+  a.n[0] = a.n[1] = N; a.count = 2; a.M = M; a.K = K; a.glu = true;
+  return run_linear(a, dtype, stream, "mhc_glu_fwd");
+}
+
 }  // extern "C"

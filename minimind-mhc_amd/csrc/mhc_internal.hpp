@@ -317,4 +317,19 @@ struct MoeArgs {
 int64_t moe_workspace(MoeArgs& a, char* base);
 hipError_t launch_moe(const MoeArgs& a, hipStream_t s);
 
+// out[i] [M, n[i]] = x [M, K] w[i]^T for `count` weights [n[i], K]; glu: one output,
+// silu(x w[0]^T) * (x w[1]^T), w[0] and w[1] [n[0], K].  16-bit tensors; K a
+// multiple of 32, n[i] of 4.
+struct LinearArgs {
+  const void* x;
+  const void* w[3];
+  void* out[3];
+  int n[3];
+  int count;
+  int64_t M;
+  int K;
+  bool glu, f16;
+};
+hipError_t launch_linear(const LinearArgs& a, hipStream_t s);
+
 }  // namespace mhc

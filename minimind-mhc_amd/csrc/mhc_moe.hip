@@ -2,7 +2,7 @@
 // top-k selection, grouping of the tokens by expert, the experts' SwiGLU products on
 // MFMA and the weighted sum, with no host synchronisation.  16-bit tensors (bf16 or
 // fp16), fp32 sums.
-#include "mhc_internal.hpp"
+#include "mhc_gemm.hpp"
 
 namespace mhc {
 namespace {
@@ -103,28 +103,18 @@ __global__ __launch_bounds__(kRouteTok) void moe_group_kernel(MoeArgs a) {
 }
 
 // ------------------------------------------------------------ grouped products
-// C[row][n] of one expert's rows: 128 rows x 256 weight rows a 4-wave workgroup,
-// K in steps of 32 through a ring of three LDS stages filled by direct-to-LDS
-// loads (two steps ahead).  Each wave holds 64 rows x 128 columns: 128
-// accumulator registers, 12 LDS reads for 32 MFMAs.
-//   * Both operands lie K-contiguous in memory, so a lane's 16 bytes are the MFMA
-//     operand.  A stage row is 64 bytes; its four 16-byte slots are permuted by the
-//     row's bits 2 and 3 (on the global side), so 16 rows hit all 64 banks.
-//   * The product is formed as W x^T, so a lane ends with four neighbouring columns
-//     of one row.
-//   * GLU: 128 gate and the matching 128 up columns; stores silu(gate) * up.
-//     Otherwise: 256 columns of the down projection, scaled by the row's weight.
+// C[row][n] of one expert's rows, a BM x BN tile (gemm_tile) a workgroup.
+//   * GLU: BN / 2 gate and the matching BN / 2 up columns; stores silu(gate) * up.
+//     Otherwise: BN columns of the down projection, scaled by the row's weight.
 //   * Workgroups of one XCD take neighbouring tiles (the same expert's weights stay
 //     in its L2).
-// 8192 tokens, 8 experts, top 2, 768 x 1024: 84 us for gate and up (51.5 GFLOP, 613
-// TFLOP/s), 48 us for down (25.8 GFLOP, 535 TFLOP/s); bound by the LDS reads beside
-// the MFMAs (12 reads of 1 KiB against 512 MFMA cycles a wave and step).  The layer's
-// loop over experts took 1.6 ms, of which library products were 290 us.
-template <bool F16, bool GLU>
-__global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeArgs a) {
-  constexpr int BM = 128, BN = 256, STAGES = 3;
-  constexpr int kStageBytes = (BM + BN) * 64;
-  __shared__ __align__(16) char lds[STAGES * kStageBytes];
+// 8192 tokens, 8 experts, top 2, 768 x 1024: 76 us for gate and up (51.5 GFLOP, 680
+// TFLOP/s), 47 us for down (25.8 GFLOP, 549 TFLOP/s); 128 x 256 tiles 84 and 48 us.
+// The layer's loop over experts took 1.6 ms, of which library products were 290 us.
+template <bool F16, typename G, bool GLU>
+__global__ __launch_bounds__(G::THREADS, 2) void moe_gemm_kernel(MoeArgs a) {
+  constexpr int BM = G::BM, BN = G::BN;
+  __shared__ __align__(16) char lds[G::LDS];
   const int N = GLU ? a.inter : a.hidden;
   const int K = GLU ? a.hidden : a.inter;
   constexpr int kCols = GLU ? BN / 2 : BN;
@@ -144,103 +134,48 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeArgs a) {
   }
   const int row_end = a.offsets[e + 1], row0 = a.offsets[e] + mt * BM;
 
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int wm = wave & 1, wn = wave >> 1;
-
-  // stage pieces of 16 rows x 64 bytes: 8 of x rows, then 16 of weight rows
-  constexpr int PIECES = (BM + BN) / 16 / 4;
-  const char* src[PIECES];
-#pragma unroll
-  for (int i = 0; i < PIECES; ++i) {
-    const int piece = wave * PIECES + i;
-    const int prow = lane >> 2, slot = (lane & 3) ^ ((prow >> 2) & 3);
-    const char* base;
-    if (piece < BM / 16) {
-      const int row = min(row0 + piece * 16 + prow, row_end - 1);
-      base = GLU ? static_cast<const char*>(a.x) + (int64_t)a.row_tok[row] * K * 2
-                 : static_cast<const char*>(a.h) + (int64_t)row * K * 2;
-    } else {
-      const int n = (piece - BM / 16) * 16 + prow;
-      const void* w = GLU ? (n < kCols ? a.gate_w[e] : a.up_w[e]) : a.down_w[e];
-      base = static_cast<const char*>(w) + (int64_t)min(n0 + n % kCols, N - 1) * K * 2;
-    }
-    src[i] = base + slot * 16;
-  }
-  auto issue = [&](int stage) {
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)src[i],
-          (__attribute__((address_space(3))) void*)(lds + stage * kStageBytes + (wave * PIECES + i) * 1024),
-          16, 0, 0);
-      src[i] += 64;
-    }
+  const int wm = wave % G::WGM, wn = wave / G::WGM;
+  auto a_row = [&](int i) {
+    const int row = min(row0 + i, row_end - 1);
+    return GLU ? static_cast<const char*>(a.x) + (int64_t)a.row_tok[row] * K * 2
+               : static_cast<const char*>(a.h) + (int64_t)row * K * 2;
   };
-  f32x4_t acc[8][4];
+  auto b_row = [&](int n) {
+    const void* w = GLU ? (n < kCols ? a.gate_w[e] : a.up_w[e]) : a.down_w[e];
+    return static_cast<const char*>(w) + (int64_t)min(n0 + n % kCols, N - 1) * K * 2;
+  };
+  // GLU: this wave's gate columns, then its up columns
+  constexpr int HALF = G::NT / 2;
+  auto col_tile = [&](int n) {
+    return GLU ? wn * HALF + (n >= HALF ? n - HALF + BN / 32 : n) : wn * G::NT + n;
+  };
+  f32x4_t acc[G::NT][G::MT];
+  gemm_tile<F16, G>(lds, K, a_row, b_row, col_tile, acc);
 #pragma unroll
-  for (int n = 0; n < 8; ++n)
-#pragma unroll
-    for (int m = 0; m < 4; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  const int steps = K / 32;
-  issue(0);
-  if (steps > 1) issue(1);
-  const int off = r * 64 + ((g ^ (r >> 2)) & 3) * 16;
-  int stage = 0;
-  for (int kt = 0; kt < steps; ++kt) {
-    // this step's pieces have landed when at most the next step's are in flight
-    if (kt + 1 < steps)
-      asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (kt + 2 < steps) issue(stage == 0 ? 2 : stage - 1);
-    const char* sa = lds + stage * kStageBytes + wm * 64 * 64 + off;
-    // GLU: this wave's 64 gate columns, then its 64 up columns
-    const char* sb = lds + stage * kStageBytes + BM * 64 + wn * (GLU ? 64 : 128) * 64 + off;
-    U32x4 xa[4], wb[8];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) xa[m] = *reinterpret_cast<const U32x4*>(sa + m * 1024);
-#pragma unroll
-    for (int n = 0; n < 8; ++n)
-      wb[n] = *reinterpret_cast<const U32x4*>(sb + (GLU && n >= 4 ? n - 4 + 8 : n) * 1024);
-#pragma unroll
-    for (int n = 0; n < 8; ++n)
-#pragma unroll
-      for (int m = 0; m < 4; ++m) acc[n][m] = mfma16<F16>(wb[n], xa[m], acc[n][m]);
-    stage = stage == 2 ? 0 : stage + 1;
-  }
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int row = row0 + wm * 64 + m * 16 + r;
+  for (int m = 0; m < G::MT; ++m) {
+    const int row = row0 + wm * G::WM + m * 16 + r;
     if (row >= row_end) continue;
     if constexpr (GLU) {
       uint16_t* out = static_cast<uint16_t*>(a.h) + (int64_t)row * N;
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        const int col = n0 + wn * 64 + n * 16 + 4 * g;
+      for (int n = 0; n < HALF; ++n) {
+        const int col = n0 + wn * HALF * 16 + n * 16 + 4 * g;
         if (col >= N) continue;
-        float v[4];
+        f32x4_t v;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float z = acc[n][m][i];
-          v[i] = z / (1.f + expf(-z)) * acc[n + 4][m][i];
-        }
-        *reinterpret_cast<uint2*>(out + col) = make_uint2(pack2<F16>(v[0], v[1]), pack2<F16>(v[2], v[3]));
+        for (int i = 0; i < 4; ++i) v[i] = silu_mul(acc[n][m][i], acc[n + HALF][m][i]);
+        store4<F16>(out + col, v);
       }
     } else {
       uint16_t* out = static_cast<uint16_t*>(a.y) + (int64_t)row * N;
       const float w = a.row_w[row];
 #pragma unroll
-      for (int n = 0; n < 8; ++n) {
-        const int col = n0 + wn * 128 + n * 16 + 4 * g;
-        if (col >= N) continue;
-        *reinterpret_cast<uint2*>(out + col) =
-            make_uint2(pack2<F16>(acc[n][m][0] * w, acc[n][m][1] * w),
-                       pack2<F16>(acc[n][m][2] * w, acc[n][m][3] * w));
+      for (int n = 0; n < G::NT; ++n) {
+        const int col = n0 + wn * G::WN + n * 16 + 4 * g;
+        if (col < N) store4<F16>(out + col, acc[n][m] * w);
       }
     }
   }
@@ -270,17 +205,34 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
   *reinterpret_cast<U32x4*>(static_cast<uint16_t*>(a.out) + tok * a.hidden + col) = o;
 }
 
+template <bool F16, bool GLU, typename G>
+hipError_t launch_tiles(const MoeArgs& a, hipStream_t s) {
+  // most row tiles: every expert's last one may be partly filled
+  const int64_t rows = a.M * a.topk, tiles = rows / G::BM + (rows < a.experts ? rows : a.experts);
+  constexpr int cols = GLU ? G::BN / 2 : G::BN;
+  const int64_t work = tiles * (((GLU ? a.inter : a.hidden) + cols - 1) / cols);
+  moe_gemm_kernel<F16, G, GLU><<<dim3((unsigned)((work + 7) / 8 * 8)), G::THREADS, 0, s>>>(a);
+  return hipGetLastError();
+}
+
+// The dense layers' rule (mhc_linear.hip): 64 x 64 tiles while 128 x 128 ones would
+// be fewer than 160.
+template <bool F16, bool GLU>
+hipError_t launch_gemm(const MoeArgs& a, hipStream_t s) {
+  const int N = GLU ? a.inter : a.hidden, K = GLU ? a.hidden : a.inter;
+  const int64_t rows = a.M * a.topk, tiles = (rows / 128 + 1) * ((N + (GLU ? 63 : 127)) / (GLU ? 64 : 128));
+  if (K % 64 != 0) return launch_tiles<F16, GLU, GemmTile<64, 64, 2, 2, 4, 1>>(a, s);
+  if (tiles < 160) return launch_tiles<F16, GLU, GemmTile<64, 64, 2, 2, 4, 2>>(a, s);
+  return launch_tiles<F16, GLU, GemmTile<128, 128, 2, 2, 2, 2>>(a, s);
+}
+
 template <bool F16>
 hipError_t launch(const MoeArgs& a, hipStream_t s) {
   const unsigned route = (unsigned)((a.M + kRouteTok - 1) / kRouteTok);
   moe_route_kernel<F16><<<dim3(route), kRouteTok, 0, s>>>(a);
   moe_group_kernel<<<dim3(route), kRouteTok, 0, s>>>(a);
-  // most row tiles: every expert's last one may be partly filled
-  const int64_t rows = a.M * a.topk;
-  const int64_t tiles = rows / 128 + (rows < a.experts ? rows : a.experts);
-  auto grid = [&](int64_t ntn) { return dim3((unsigned)((tiles * ntn + 7) / 8 * 8)); };
-  moe_gemm_kernel<F16, true><<<grid((a.inter + 127) / 128), 256, 0, s>>>(a);
-  moe_gemm_kernel<F16, false><<<grid((a.hidden + 255) / 256), 256, 0, s>>>(a);
+  if (hipError_t e = launch_gemm<F16, true>(a, s); e != hipSuccess) return e;
+  if (hipError_t e = launch_gemm<F16, false>(a, s); e != hipSuccess) return e;
   const int64_t vec = a.M * (a.hidden / 8);
   moe_combine_kernel<F16><<<dim3((unsigned)((vec + 255) / 256)), 256, 0, s>>>(a);
   return hipGetLastError();

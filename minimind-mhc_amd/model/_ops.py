@@ -641,6 +641,75 @@ def plain_tensors(dtype: torch.dtype, dev: torch.device, *ts) -> bool:
                and t.device == dev and t.data_ptr() % 16 == 0 for t in ts)
 
 
+# Multiply-adds up to which one linear layer runs on mhc_linear_fwd.  The library's
+# call costs the host 19 us (MI355X box, torch 2.10), the kernel's 7; up to here the
+# kernel takes at most 15 us, so the cheaper call wins although the library's kernel
+# is a little faster (512 rows, 768 x 6400: 14.6 against 11.1 us; 2048 rows,
+# 2048 x 768: 14.7 against 14.1).  Past it the library's kernel does (8192 rows,
+# 768 x 768: 19.1 against 15.5 us).
+LINEAR_MAX_MACS = 3_300_000_000
+
+
+def _linear_weights(x: torch.Tensor, mods):
+    """The weights of bias-free nn.Linear layers the kernels can apply to x, or None."""
+    if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or not plain_call()
+            or x.dim() < 2 or x.numel() == 0 or not x.is_contiguous()):
+        return None
+    K = x.shape[-1]
+    if K % 32 != 0:
+        return None
+    ws = []
+    for m in mods:
+        if not plain_module(m, torch.nn.Linear) or m.bias is not None:
+            return None
+        w = m.weight
+        if w.dim() != 2 or w.shape[1] != K or w.shape[0] % 4 != 0 or not w.is_contiguous():
+            return None
+        ws.append(w)
+    return ws if plain_tensors(x.dtype, x.device, x, *ws) else None
+
+
+def linears(x: torch.Tensor, *mods):
+    """[m(x) for m in mods] for one to three bias-free nn.Linear layers in one
+    launch, or None for a call the kernels do not take (or, for a single layer,
+    one that is faster in the library)."""
+    ws = _linear_weights(x, mods)
+    if ws is None:
+        return None
+    K = x.shape[-1]
+    M = x.numel() // K
+    if len(ws) == 1 and M * K * ws[0].shape[0] > LINEAR_MAX_MACS:
+        return None
+    n = len(ws)
+    outs = [x.new_empty(*x.shape[:-1], w.shape[0]) for w in ws]
+    H.check(H.load().mhc_linear_fwd(
+        x.data_ptr(), (ctypes.c_void_p * n)(*[w.data_ptr() for w in ws]),
+        (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs]),
+        (ctypes.c_int * n)(*[w.shape[0] for w in ws]), n, M, K, H.dtype_tag(x),
+        H.stream(x.device)), "mhc_linear_fwd")
+    return outs
+
+
+def linear(x: torch.Tensor, m: torch.nn.Module) -> torch.Tensor:
+    """m(x), on mhc_linear_fwd where `linears` takes it."""
+    out = linears(x, m)
+    return m(x) if out is None else out[0]
+
+
+def glu(x: torch.Tensor, gate: torch.nn.Module, up: torch.nn.Module) -> Optional[torch.Tensor]:
+    """silu(gate(x)) * up(x) for bias-free nn.Linear layers in one launch, or None
+    for a call the kernels do not take."""
+    ws = _linear_weights(x, (gate, up))
+    if ws is None or ws[0].shape != ws[1].shape:
+        return None
+    K, N = x.shape[-1], ws[0].shape[0]
+    out = x.new_empty(*x.shape[:-1], N)
+    H.check(H.load().mhc_glu_fwd(x.data_ptr(), ws[0].data_ptr(), ws[1].data_ptr(), out.data_ptr(),
+                                 x.numel() // K, K, N, H.dtype_tag(x), H.stream(x.device)),
+            "mhc_glu_fwd")
+    return out
+
+
 ATTN_HEAD_DIMS = (64, 96, 128)
 
 

@@ -149,17 +149,18 @@ class Attention(nn.Module):
     def forward(self, x, position_embeddings, past_key_value=None, use_cache=False,
                 attention_mask=None):
         bsz, seq_len, _ = x.shape
-        xq, xk, xv = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        xq, xk, xv = (_ops.linears(x, self.q_proj, self.k_proj, self.v_proj)
+                      or (self.q_proj(x), self.k_proj(x), self.v_proj(x)))
         route = None if attention_mask is not None else _ops.attn_route(
             self, xq, xk, xv, position_embeddings, past_key_value)
         if route == "decode":
             out, past_kv = _ops.attn_decode(self, xq, xk, xv, position_embeddings,
                                             past_key_value, use_cache)
-            return self.o_proj(out), past_kv
+            return _ops.linear(out, self.o_proj), past_kv
         if route == "prefill":
             out, xk = _ops.attn_prefill(self, xq, xk, xv, position_embeddings)
             kv_shape = (bsz, seq_len, self.n_local_kv_heads, self.head_dim)
-            return self.o_proj(out), ((xk.view(kv_shape), xv.view(kv_shape)) if use_cache else None)
+            return _ops.linear(out, self.o_proj), ((xk.view(kv_shape), xv.view(kv_shape)) if use_cache else None)
         xq = xq.view(bsz, seq_len, self.n_local_heads, self.head_dim)
         xk = xk.view(bsz, seq_len, self.n_local_kv_heads, self.head_dim)
         xv = xv.view(bsz, seq_len, self.n_local_kv_heads, self.head_dim)
@@ -196,7 +197,8 @@ class Attention(nn.Module):
 
 
 class FeedForward(nn.Module):
-    """SwiGLU FFN (model/model_minimind.py:258-268)."""
+    """SwiGLU FFN (model/model_minimind.py:258-268); inference on 16-bit tensors
+    forms silu(gate) * up in one launch (_ops.glu says when)."""
 
     def __init__(self, config: MiniMindConfig, intermediate_size: int = None):
         super().__init__()
@@ -206,7 +208,10 @@ class FeedForward(nn.Module):
         self.up_proj = nn.Linear(config.hidden_size, inter, bias=False)
 
     def forward(self, x):
-        return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
+        h = _ops.glu(x, self.gate_proj, self.up_proj)
+        if h is None:
+            h = F.silu(self.gate_proj(x)) * self.up_proj(x)
+        return _ops.linear(h, self.down_proj)
 
 
 class MOEFeedForward(nn.Module):
@@ -362,7 +367,7 @@ class MiniMindForCausalLM(nn.Module):
                 logits_to_keep=0, labels=None, **kwargs):
         h, pkv, aux = self.model(input_ids, attention_mask, past_key_values, use_cache, **kwargs)
         sl = slice(-logits_to_keep, None) if isinstance(logits_to_keep, int) else logits_to_keep
-        logits = self.lm_head(h[:, sl, :])
+        logits = _ops.linear(h[:, sl, :], self.lm_head)
         loss = None
         if labels is not None:
             x, y = logits[..., :-1, :].contiguous(), labels[..., 1:].contiguous()
