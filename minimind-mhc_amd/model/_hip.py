@@ -153,7 +153,7 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 def require_device(*tensors: Optional[torch.Tensor]) -> torch.device:
     """All tensors must live on one ROCm device; returns it."""
-    dev = None
+    dev, index = None, -1
     for t in tensors:
         if t is None:
             continue
@@ -161,8 +161,8 @@ def require_device(*tensors: Optional[torch.Tensor]) -> torch.device:
             raise RuntimeError(
                 "mhc_amd: tensors must be on a ROCm GPU; the mHC kernels have no CPU path")
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
+            dev, index = t.device, t.get_device()
+        elif t.get_device() != index:
             raise RuntimeError(f"mhc_amd: tensors on different devices ({dev} vs {t.device})")
     if dev is None:
         raise RuntimeError("mhc_amd: no device tensor given")
@@ -170,7 +170,9 @@ def require_device(*tensors: Optional[torch.Tensor]) -> torch.device:
 
 
 def stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The current stream's handle.  torch.cuda.current_stream(dev).cuda_stream builds a
+    Stream object for it: 2 us a launch."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 def check(rc: int, fn: str) -> None:
@@ -182,11 +184,6 @@ def check(rc: int, fn: str) -> None:
 def params_like(ref: torch.Tensor, *ps: torch.Tensor):
     """alpha/bias tensors as contiguous device tensors of one dtype (the first's)."""
     dt = ps[0].dtype
-    out = []
-    for p in ps:
-        p = p.detach()
-        if p.dtype != dt:
-            p = p.to(dt)
-        out.append(p.contiguous())
-    dtype_tag(out[0])
-    return out
+    dtype_tag(ps[0])
+    return [p if p.dtype == dt and p.is_contiguous() else p.detach().to(dt).contiguous()
+            for p in ps]

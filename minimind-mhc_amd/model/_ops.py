@@ -44,6 +44,11 @@ def grad_wanted(ctx, index: Optional[int] = None) -> bool:
     return any(ctx.needs_input_grad) if index is None else bool(ctx.needs_input_grad[index])
 
 
+def _contiguous(t: torch.Tensor) -> torch.Tensor:
+    """t itself where its data already lie in order (only its pointer is used)."""
+    return t if t.is_contiguous() else t.detach().contiguous()
+
+
 class PhiPack:
     """MFMA operand image of a projection weight, rebuilt when the weight changes.
 
@@ -89,6 +94,16 @@ class PhiPack:
         training: whether phi trains in this call; default grad mode and
         phi.requires_grad (inside an autograd Function's forward, where grad
         mode is off, pass grad_wanted(ctx, <phi's index>))."""
+        if training is None:
+            training = torch.is_grad_enabled() and phi.requires_grad
+        try:
+            version = None if training else phi._version
+        except RuntimeError:
+            version = None
+        key = (phi.data_ptr(), version, phi.device, phi.dtype, n, C)
+        if (version is not None and self._buf is not None and self._src() is phi
+                and key == self._key):
+            return self._buf
         lib = H.load()
         if phi.dtype == torch.bfloat16:
             nbytes = lib.mhc_phi_packed_bytes(n, C, self.mode)
@@ -105,17 +120,7 @@ class PhiPack:
             return None
         if nbytes <= 0:
             return None
-        if training is None:
-            training = torch.is_grad_enabled() and phi.requires_grad
-        try:
-            version = None if training else phi._version
-        except RuntimeError:
-            version = None
-        key = (phi.data_ptr(), version, phi.device, phi.dtype, n, C)
-        src = self._src() if self._src is not None else None
-        if version is not None and src is phi and key == self._key and self._buf is not None:
-            return self._buf
-        w = phi.detach().contiguous()
+        w = _contiguous(phi)
         buf = torch.empty(nbytes, dtype=torch.uint8, device=phi.device)
         H.check(pack(w.data_ptr(), H.dtype_tag(w), buf.data_ptr(), n, C, self.mode,
                      H.stream(phi.device)), "mhc_phi_pack")
@@ -230,7 +235,15 @@ def _check_numel(name: str, t: torch.Tensor, want: int) -> None:
 def _rows(x_flat: torch.Tensor, NC: int) -> torch.Tensor:
     if x_flat.shape[-1] != NC:
         raise ValueError(f"mhc_amd: last dim {x_flat.shape[-1]} != n*C = {NC}")
-    return x_flat.contiguous().view(-1, NC)
+    return _contiguous(x_flat).view(-1, NC)
+
+
+def _flat(t: torch.Tensor, name: str, numel: int) -> torch.Tensor:
+    """t in order, with that many elements (only its pointer is used)."""
+    if t.numel() != numel:
+        raise RuntimeError(f"mhc_amd: {name} of shape {tuple(t.shape)} has {t.numel()} elements, "
+                           f"not {numel}")
+    return _contiguous(t)
 
 
 def _norm_args(norm, C: int, dev):
@@ -240,7 +253,7 @@ def _norm_args(norm, C: int, dev):
         return None, 0, 0.0, None
     w, eps = norm
     H.require_device(w)
-    wc = w.detach().contiguous()
+    wc = _contiguous(w)
     _check_numel("norm weight", wc, C)
     if wc.device != dev:
         raise ValueError("mhc_amd: norm weight is on another device")
@@ -269,21 +282,25 @@ def pre_full(x_flat, phi, packed, a_pre, b_pre, a_post, b_post, a_res, b_res, n,
         raise ValueError(f"mhc_amd: phi_weight shape {tuple(phi.shape)} != ({NC}, {FD})")
     x2 = _rows(x_flat, NC)
     M = x2.shape[0]
-    phi_c = phi.detach().contiguous()
+    phi_c = _contiguous(phi)
     a_pre, b_pre, a_post, b_post, a_res, b_res = H.params_like(
         x2, a_pre, b_pre, a_post, b_post, a_res, b_res)
-    for nm, tt, want in (("alpha_pre", a_pre, 1), ("alpha_post", a_post, 1), ("alpha_res", a_res, 1),
-                         ("bias_pre", b_pre, n), ("bias_post", b_post, n), ("bias_res", b_res, n * n)):
-        _check_numel(nm, tt, want)
-    kw = dict(dtype=x2.dtype, device=dev)
+    _check_numel("alpha_pre", a_pre, 1)
+    _check_numel("alpha_post", a_post, 1)
+    _check_numel("alpha_res", a_res, 1)
+    _check_numel("bias_pre", b_pre, n)
+    _check_numel("bias_post", b_post, n)
+    _check_numel("bias_res", b_res, n * n)
+    new = x2.new_empty
+    f32 = torch.float32
     out = {
-        "sub_in": torch.empty(M, C, **kw),
-        "h_post": torch.empty(M, n, **kw),
-        "h_pre": torch.empty(M, n, **kw) if want_h_pre else None,
-        "h_res_raw": torch.empty(M, n, n, **kw) if want_raw else None,
-        "h_res": torch.empty(M, n, n, **kw) if sinkhorn else None,
-        "inv_rms": torch.empty(M, dtype=torch.float32, device=dev) if want_saved else None,
-        "mixes_raw": torch.empty(M, FD, dtype=torch.float32, device=dev) if want_saved else None,
+        "sub_in": new((M, C)),
+        "h_post": new((M, n)),
+        "h_pre": new((M, n)) if want_h_pre else None,
+        "h_res_raw": new((M, n, n)) if want_raw else None,
+        "h_res": new((M, n, n)) if sinkhorn else None,
+        "inv_rms": new((M,), dtype=f32) if want_saved else None,
+        "mixes_raw": new((M, FD), dtype=f32) if want_saved else None,
     }
     args = (x2.data_ptr(), H.dtype_tag(x2), phi_c.data_ptr(), _phi_tag(phi_c, packed), H.ptr(packed),
             a_pre.data_ptr(), b_pre.data_ptr(), a_post.data_ptr(), b_post.data_ptr(),
@@ -311,18 +328,20 @@ def pre_nohres(x_flat, phi, packed, a_pre, b_pre, a_post, b_post, n, C, post_mul
         raise ValueError(f"mhc_amd: phi_weight shape {tuple(phi.shape)} != ({NC}, {FD})")
     x2 = _rows(x_flat, NC)
     M = x2.shape[0]
-    phi_c = phi.detach().contiguous()
+    phi_c = _contiguous(phi)
     a_pre, b_pre, a_post, b_post = H.params_like(x2, a_pre, b_pre, a_post, b_post)
-    for nm, tt, want in (("alpha_pre", a_pre, 1), ("alpha_post", a_post, 1),
-                         ("bias_pre", b_pre, n), ("bias_post", b_post, n)):
-        _check_numel(nm, tt, want)
-    kw = dict(dtype=x2.dtype, device=dev)
+    _check_numel("alpha_pre", a_pre, 1)
+    _check_numel("alpha_post", a_post, 1)
+    _check_numel("bias_pre", b_pre, n)
+    _check_numel("bias_post", b_post, n)
+    new = x2.new_empty
+    f32 = torch.float32
     out = {
-        "sub_in": torch.empty(M, C, **kw),
-        "h_post": torch.empty(M, n, **kw),
-        "h_pre": torch.empty(M, n, **kw) if want_h_pre else None,
-        "inv_rms": torch.empty(M, dtype=torch.float32, device=dev) if want_saved else None,
-        "mixes_raw": torch.empty(M, FD, dtype=torch.float32, device=dev) if want_saved else None,
+        "sub_in": new((M, C)),
+        "h_post": new((M, n)),
+        "h_pre": new((M, n)) if want_h_pre else None,
+        "inv_rms": new((M,), dtype=f32) if want_saved else None,
+        "mixes_raw": new((M, FD), dtype=f32) if want_saved else None,
     }
     args = (x2.data_ptr(), H.dtype_tag(x2), phi_c.data_ptr(), _phi_tag(phi_c, packed), H.ptr(packed),
             a_pre.data_ptr(), b_pre.data_ptr(), a_post.data_ptr(), b_post.data_ptr(),
@@ -354,7 +373,7 @@ def head(x_flat, phi, packed, alpha, bias, n, C, pre_eps, rms_eps, *, want_saved
         dev = H.require_device(x_flat, phi, alpha, bias)
         if tuple(phi.shape) != (NC, n):
             raise ValueError(f"mhc_amd: phi_weight shape {tuple(phi.shape)} != ({NC}, {n})")
-        phi_c = phi.detach().contiguous()
+        phi_c = _contiguous(phi)
         alpha_c, bias_c = H.params_like(x2, alpha, bias)
         _check_numel("alpha", alpha_c, 1)
         _check_numel("bias", bias_c, n)
@@ -383,15 +402,15 @@ def post(x_flat, h_res, h_post, f_out, n, C, ssq_out=None):
     NC = n * C
     x2 = _rows(x_flat, NC)
     M = x2.shape[0]
-    hp = h_post.contiguous().view(M, n)
-    f2 = f_out.contiguous().view(M, C)
+    hp = _flat(h_post, "h_post", M * n)
+    f2 = _flat(f_out, "f_out", M * C)
     if hp.dtype != (h_res.dtype if h_res is not None else hp.dtype):
         raise TypeError("mhc_amd: h_res and h_post must share a dtype")
     out = torch.empty_like(x2)
     lib = H.load()
     sp = _ssq_ptr(ssq_out, M, C)
     if h_res is not None:
-        hr = h_res.contiguous().view(M, n, n)
+        hr = _flat(h_res, "h_res", M * n * n)
         rc = lib.mhc_post_fwd(x2.data_ptr(), H.dtype_tag(x2), hr.data_ptr(), hp.data_ptr(),
                               H.dtype_tag(hp), f2.data_ptr(), H.dtype_tag(f2), out.data_ptr(),
                               M, n, C, sp, H.stream(dev))
@@ -477,8 +496,8 @@ def post_bwd(x_flat, h_res, h_post, f_out, n, C, g_out):
     dev = H.require_device(g_out, h_post, f_out, h_res, x_flat if h_res is not None else None)
     NC = n * C
     M = g_out.numel() // NC
-    hp = h_post.contiguous().view(M, n)
-    f2 = f_out.contiguous().view(M, C)
+    hp = _contiguous(h_post).view(M, n)
+    f2 = _contiguous(f_out).view(M, C)
     g_hp = torch.empty_like(hp)
     g_f = torch.empty_like(f2)
     lib = H.load()
@@ -493,7 +512,7 @@ def post_bwd(x_flat, h_res, h_post, f_out, n, C, g_out):
     g2 = _rows(g_out, NC)
     if g2.dtype != x2.dtype:
         g2 = g2.to(x2.dtype)
-    hr = h_res.contiguous().view(M, n, n)
+    hr = _contiguous(h_res).view(M, n, n)
     if hr.dtype != hp.dtype:
         raise TypeError("mhc_amd: h_res and h_post must share a dtype")
     g_x = torch.empty_like(x2)
@@ -516,8 +535,9 @@ def pre_bwd(x2, phi, alphas, biases, inv_rms, mixes, n, C, mode, post_mult, pre_
     dev = H.require_device(x2, inv_rms, *grads)
     M = x2.shape[0]
     gdt = grads[0].dtype if grads else x2.dtype
-    g_sub, g_hpre, g_hpost, g_hres = (None if g is None else g.to(gdt).contiguous()
-                                      for g in (g_sub, g_hpre, g_hpost, g_hres))
+    g_sub, g_hpre, g_hpost, g_hres = (
+        g if g is None or (g.dtype == gdt and g.is_contiguous()) else g.to(gdt).contiguous()
+        for g in (g_sub, g_hpre, g_hpost, g_hres))
     if g_x_in is not None:
         H.require_device(x2, g_x_in)
         g_x_in = g_x_in.to(x2.dtype).reshape(x2.shape).contiguous()
@@ -529,7 +549,7 @@ def pre_bwd(x2, phi, alphas, biases, inv_rms, mixes, n, C, mode, post_mult, pre_
         g_raw = None
     else:
         FD = {H.MODE_FULL: 2 * n + n * n, H.MODE_NOHRES: 2 * n, H.MODE_HEAD: n}[mode]
-        phi_c = phi.detach().contiguous()
+        phi_c = _contiguous(phi)
         phi_p, phi_dt = phi_c.data_ptr(), H.dtype_tag(phi_c)
         present = [p for p in (alphas[0], biases[0], alphas[1], biases[1], alphas[2]) if p is not None]
         conv = iter(H.params_like(x2, *present))

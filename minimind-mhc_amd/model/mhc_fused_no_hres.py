@@ -121,19 +121,20 @@ class MHCConnection_FusedNoHres(nn.Module):
         packed = self._phi_pack.get(self.phi_weight, self.n, self.dim) if x_flat.is_cuda else None
         ssq = chain.take(x_flat, self.n, self.dim) if chain is not None else None
         ssq_out = chain.buffer(x_flat, self.n, self.dim) if chain is not None else None
-        if in_norm is not None:
-            if fusable_norm(in_norm, self.dim, x_flat):
-                o = _ops.pre_nohres(x_flat, self.phi_weight, packed, self.alpha_pre, self.bias_pre,
-                                    self.alpha_post, self.bias_post, self.n, self.dim,
-                                    self.post_mult_value, self.pre_eps, self.eps,
-                                    norm=(in_norm.weight, norm_eps(in_norm, x_flat)), ssq=ssq)
-                B, L, NC = x_flat.shape
-                f_out = sublayer_fn(o["sub_in"].view(B, L, self.dim))
-                out = _ops.post(x_flat, None, o["h_post"], f_out, self.n, self.dim,
-                                ssq_out=ssq_out).view(B, L, NC)
-                return chain.put(out, ssq_out) if chain is not None else out
+        fused = in_norm is not None and fusable_norm(in_norm, self.dim, x_flat)
+        if in_norm is not None and not fused:
             fn = sublayer_fn
             sublayer_fn = lambda z: fn(in_norm(z))  # noqa: E731
+        if fused or _ops.plain_call():  # nothing to record: the launches without the Functions
+            o = _ops.pre_nohres(x_flat, self.phi_weight, packed, self.alpha_pre, self.bias_pre,
+                                self.alpha_post, self.bias_post, self.n, self.dim,
+                                self.post_mult_value, self.pre_eps, self.eps, ssq=ssq,
+                                norm=(in_norm.weight, norm_eps(in_norm, x_flat)) if fused else None)
+            B, L, NC = x_flat.shape
+            f_out = sublayer_fn(o["sub_in"].view(B, L, self.dim))
+            out = _ops.post(x_flat, None, o["h_post"], f_out, self.n, self.dim,
+                            ssq_out=ssq_out).view(B, L, NC)
+            return chain.put(out, ssq_out) if chain is not None else out
         grad = torch.is_grad_enabled()
         sublayer_in, _h_pre, h_post, *passed = _PrePhaseFn.apply(
             x_flat, self.phi_weight, self.alpha_pre, self.bias_pre,
