@@ -690,9 +690,10 @@ int64_t mhc_attn_decode_workspace_bytes(int64_t B, int S, int heads, int kv_head
   if (B < 0 || S < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || heads / kv_heads > 4) return -1;
   if (head_dim != 64 && head_dim != 96 && head_dim != 128) return -1;
   if (B == 0) return 0;
-  int per = 0;
-  const int splits = mhc::attn_decode_splits(B, S, kv_heads, &per);
-  return splits == 1 ? 0 : B * heads * splits * (head_dim + 2) * 4;
+  mhc::AttnDecodeArgs a{};
+  a.B = B; a.S = S; a.kv_heads = kv_heads;
+  mhc::attn_decode_plan(a);
+  return a.parts == 1 ? 0 : B * heads * a.parts * (head_dim + 2) * 4;
 }
 
 int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void* q_gain,
@@ -723,7 +724,7 @@ int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void*
   a.ks_b = k_stride_b; a.ks_s = k_stride_s; a.ks_h = k_stride_h;
   a.vs_b = v_stride_b; a.vs_s = v_stride_s; a.vs_h = v_stride_h;
   a.B = B; a.S = S; a.heads = heads; a.kv_heads = kv_heads; a.head_dim = head_dim;
-  a.splits = mhc::attn_decode_splits(B, S, kv_heads, &a.tiles_per_split);
+  mhc::attn_decode_plan(a);
   a.f16 = dtype == mhc::kF16; a.q_eps = q_eps; a.k_eps = k_eps;
   return hip_status(mhc::launch_attn_decode(a, stream), fn);
 }

@@ -107,10 +107,9 @@ __global__ __launch_bounds__(256) void k_norm_rope_kernel(KRopeArgs a) {
 // ------------------------------------------------------------------ decode step
 // One query token per sequence over S cached positions and the new one.  The
 // step is bound by the cache's bytes (and, when a grown cache is returned, by
-// writing them back), so a wave reads each K and V row of its (sequence, kv
-// head, range of positions) once, serves all REP query heads of that kv head
-// with it, and stores the row to the grown cache on the way.
-//   * q, and in the wave whose range ends with the new position k, are normed
+// writing them back), so each K and V row is read once, serves all REP query heads
+// of its kv head, and is stored to the grown cache on the way.
+//   * q, and in the range that ends with the new position k, are normed
 //     and rotated here: the raw projections are the inputs.
 //   * Scores on v_mfma 16x16x32: A rows 4g + i all hold query head i, so lane
 //     (r, g) gets its REP scores of position r without a shuffle; B is the K row
@@ -118,13 +117,14 @@ __global__ __launch_bounds__(256) void k_norm_rope_kernel(KRopeArgs a) {
 //   * Each lane keeps its own running maximum, sum and output columns (8 per
 //     32-column chunk) of the positions r mod 16 it saw: no cross-lane step in
 //     the loop.  The 16 lanes merge at the end, the ranges in a second launch.
-//   * Rows are loaded (non-temporal: read once) and stored as their bytes run;
-//     in the operand layout each access is 16 rows x 64 bytes, and the launch
-//     took 94 us instead of 84 (64 sequences, 4 kv heads of 96, S = 2048, grown
-//     cache: 403 MB, now 81 us or 5.0 TB/s; a large torch copy runs at 4.9).
-//     Cached loads 97.5 us, non-temporal stores 101 us, four waves a SIMD (six
-//     registers spilled) 117 us.  The torch ops (cat, two expanded copies, SDPA,
-//     norms and rotary) took 670 us.
+//   * A workgroup takes four waves' worth of rows (a tile): 4, 2 or 1 kv heads of 16,
+//     32 or 64 positions, loaded (non-temporal: read once) and stored as their bytes
+//     run, whole lines across the workgroup, and regrouped through LDS.  64
+//     sequences, 4 kv heads of 96, S = 2048, grown cache, 403 MB: 72.6 us, 5.55 TB/s
+//     (a large torch copy runs at 4.9).  Each wave loading and storing its own head's
+//     rows 80 us (cached loads 97, non-temporal stores 101), in the operand layout
+//     (16 rows x 64 bytes) 94; here non-temporal stores 85.  The torch ops (cat, two
+//     expanded copies, SDPA, norms and rotary) took 670 us.
 //   * The maximum is raised (and the sums rescaled) only when some score exceeds
 //     it by more than 2^8 in the exponent; fp32 sums lose nothing by that.
 constexpr float kLazyMax = 8.f;
@@ -143,48 +143,53 @@ template <bool F16, int HD, int REP>
 __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
   constexpr int NC = HD / 32;
   constexpr int LST = HD + 8;  // 16 rows on distinct banks
-  __shared__ __align__(16) uint16_t lds[4 * 2 * 16 * LST];
-  const int wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
+  __shared__ __align__(16) uint16_t kl[2][4 * 16 * LST];
+  __shared__ __align__(16) uint16_t vl[2][4 * 16 * LST];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
   const int r = lane & 15, g = lane >> 4;
-  // consecutive waves take the kv heads of the same positions: their rows are
-  // neighbours in memory
-  const int64_t unit = wave_uniform((int64_t)blockIdx.x * 4 + wave);
-  const int64_t units = (int64_t)a.B * a.splits * a.kv_heads;
-  if (unit >= units) return;
-  const int kvh = (int)(unit % a.kv_heads);
-  const int64_t bs = unit / a.kv_heads;
+  // the workgroup's kv heads (1, 2 or 4), its waves' rows: wave = sub * G + head
+  const int G = a.group, rows = 64 / G;  // positions a tile
+  const int hg = blockIdx.x % (a.kv_heads / G);
+  const int64_t bs = blockIdx.x / (a.kv_heads / G);
   const int split = (int)(bs % a.splits);
   const int64_t b = bs / a.splits;
+  const int kvh = hg * G + wave % G;
+  const int sub = wave / G * 16;
   const int t0 = split * a.tiles_per_split;
-  const int tiles = (a.S + 15) >> 4;
-  const int t1 = min(t0 + a.tiles_per_split, tiles);
-  const bool has_new = split == a.splits - 1;
+  const int t1 = min(t0 + a.tiles_per_split, (a.S + rows - 1) / rows);
+  const bool has_new = split == a.splits - 1 && wave < G;
 
-  const uint16_t* kb = static_cast<const uint16_t*>(a.k_past) + b * a.ks_b + kvh * a.ks_h;
-  const uint16_t* vb = static_cast<const uint16_t*>(a.v_past) + b * a.vs_b + kvh * a.vs_h;
+  // A tile is loaded and stored as its bytes run in the cache (whole lines across the
+  // workgroup: the heads of a position are neighbours), piece p * 256 + tid, and
+  // reaches the waves' operand layout through LDS.
+  const uint16_t* kb = static_cast<const uint16_t*>(a.k_past) + b * a.ks_b + hg * G * a.ks_h;
+  const uint16_t* vb = static_cast<const uint16_t*>(a.v_past) + b * a.vs_b + hg * G * a.vs_h;
   const int64_t orow = (int64_t)a.kv_heads * HD;  // grown cache: contiguous [B, S + 1, kv, HD]
   uint16_t* ko = static_cast<uint16_t*>(a.k_out);
   uint16_t* vo = static_cast<uint16_t*>(a.v_out);
-  const int64_t obase = (b * (a.S + 1)) * orow + kvh * HD;
-
-  // A tile (16 rows of this kv head) is loaded and stored as its rows' bytes run,
-  // piece p * 64 + lane, and regrouped into the operand layout through an LDS
-  // block of the wave's own (in-order, so no barrier).
-  uint16_t* kl = lds + wave * 2 * 16 * LST;
-  uint16_t* vl = kl + 16 * LST;
-  int prow[NC], pcol[NC];
+  const int64_t obase = b * (a.S + 1) * orow;
+  const uint16_t* kp[NC];
+  const uint16_t* vp[NC];
+  int prow[NC], ocol[NC], lpos[NC];
 #pragma unroll
   for (int p = 0; p < NC; ++p) {
-    prow[p] = (p * 64 + lane) / (HD / 8);
-    pcol[p] = (p * 64 + lane) % (HD / 8) * 8;
+    const int piece = p * 256 + tid, per = G * (HD / 8);
+    prow[p] = piece / per;
+    const int in_row = piece - prow[p] * per;
+    const int head = in_row / (HD / 8), col = in_row % (HD / 8) * 8;
+    kp[p] = kb + head * a.ks_h + col;
+    vp[p] = vb + head * a.vs_h + col;
+    ocol[p] = (hg * G + head) * HD + col;
+    lpos[p] = ((prow[p] / 16 * G + head) * 16 + prow[p] % 16) * LST + col;
   }
   U32x4 kn[NC], vn[NC];  // next tile
   auto load = [&](int t) {
 #pragma unroll
-    for (int p = 0; p < NC; ++p) kn[p] = ld16_nt(kb + (int64_t)min(t * 16 + prow[p], a.S - 1) * a.ks_s + pcol[p]);
+    for (int p = 0; p < NC; ++p) kn[p] = ld16_nt(kp[p] + (int64_t)min(t * rows + prow[p], a.S - 1) * a.ks_s);
 #pragma unroll
-    for (int p = 0; p < NC; ++p) vn[p] = ld16_nt(vb + (int64_t)min(t * 16 + prow[p], a.S - 1) * a.vs_s + pcol[p]);
+    for (int p = 0; p < NC; ++p) vn[p] = ld16_nt(vp[p] + (int64_t)min(t * rows + prow[p], a.S - 1) * a.vs_s);
   };
   if (t0 < t1) load(t0);
 
@@ -248,25 +253,27 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
         }
       }
   };
-  for (int t = t0; t < t1; ++t) {
+  for (int t = t0; t < t1; ++t) {  // uniform: two buffers, so one barrier a tile
+    const int buf = (t - t0) & 1;
 #pragma unroll
     for (int p = 0; p < NC; ++p) {
-      *reinterpret_cast<U32x4*>(kl + prow[p] * LST + pcol[p]) = kn[p];
-      *reinterpret_cast<U32x4*>(vl + prow[p] * LST + pcol[p]) = vn[p];
-      const int row = t * 16 + prow[p];
+      *reinterpret_cast<U32x4*>(&kl[buf][lpos[p]]) = kn[p];
+      *reinterpret_cast<U32x4*>(&vl[buf][lpos[p]]) = vn[p];
+      const int row = t * rows + prow[p];
       if (ko && row < a.S) {
-        *reinterpret_cast<U32x4*>(ko + obase + row * orow + pcol[p]) = kn[p];
-        *reinterpret_cast<U32x4*>(vo + obase + row * orow + pcol[p]) = vn[p];
+        *reinterpret_cast<U32x4*>(ko + obase + row * orow + ocol[p]) = kn[p];
+        *reinterpret_cast<U32x4*>(vo + obase + row * orow + ocol[p]) = vn[p];
       }
     }
     if (t + 1 < t1) load(t + 1);
+    __syncthreads();
     U32x4 kc[NC], vc[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      kc[c] = *reinterpret_cast<const U32x4*>(kl + r * LST + 32 * c + 8 * g);
-      vc[c] = *reinterpret_cast<const U32x4*>(vl + r * LST + 32 * c + 8 * g);
+      kc[c] = *reinterpret_cast<const U32x4*>(&kl[buf][(wave * 16 + r) * LST + 32 * c + 8 * g]);
+      vc[c] = *reinterpret_cast<const U32x4*>(&vl[buf][(wave * 16 + r) * LST + 32 * c + 8 * g]);
     }
-    step(kc, vc, t * 16 + r < a.S);
+    step(kc, vc, t * rows + sub + r < a.S);
   }
   if (has_new) {  // the new position: one row, in the lanes with r == 0
     U32x4 kc[NC], vc[NC];
@@ -276,7 +283,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
 #pragma unroll
     for (int c = 0; c < NC; ++c) vc[c] = ld16(vp + 32 * c);
     if (ko && r == 0) {
-      const int64_t o = obase + a.S * orow + 8 * g;
+      const int64_t o = obase + a.S * orow + kvh * HD + 8 * g;
 #pragma unroll
       for (int c = 0; c < NC; ++c) *reinterpret_cast<U32x4*>(ko + o + 32 * c) = kc[c];
 #pragma unroll
@@ -296,7 +303,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
       for (int e = 0; e < 8; ++e) acc[i][c][e] = row16_sum(acc[i][c][e] * f);
     if (r != 0) continue;
     const int64_t row = b * a.heads + kvh * REP + i;
-    if (a.splits == 1) {
+    if (a.parts == 1) {
       uint16_t* o = static_cast<uint16_t*>(a.out) + row * HD + 8 * g;
       const float inv = 1.f / ls;
 #pragma unroll
@@ -307,7 +314,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
         *reinterpret_cast<U32x4*>(o + 32 * c) = w;
       }
     } else {
-      const int64_t part = row * a.splits + split;
+      const int64_t part = row * a.parts + split * (4 / G) + wave / G;
       float* o = a.work + part * HD + 8 * g;
 #pragma unroll
       for (int c = 0; c < NC; ++c)
@@ -316,7 +323,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
           *reinterpret_cast<f32x4_t*>(o + 32 * c + e) =
               f32x4_t{acc[i][c][e], acc[i][c][e + 1], acc[i][c][e + 2], acc[i][c][e + 3]};
       if (g == 0) {
-        float* ml = a.work + (int64_t)a.B * a.heads * a.splits * HD + 2 * part;
+        float* ml = a.work + a.B * a.heads * a.parts * HD + 2 * part;
         ml[0] = mx;
         ml[1] = ls;
       }
@@ -334,17 +341,17 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(AttnDecodeArgs a) {
   const int sub = threadIdx.x / LPR;
   const int64_t row = blockIdx.x;
   const bool live = lane < HD / 4;
-  const float* part = a.work + row * a.splits * HD + (live ? 4 * lane : 0);
-  const float* ml = a.work + (int64_t)a.B * a.heads * a.splits * HD + 2 * row * a.splits;
+  const float* part = a.work + row * a.parts * HD + (live ? 4 * lane : 0);
+  const float* ml = a.work + a.B * a.heads * a.parts * HD + 2 * row * a.parts;
   float mx = kNegBig;
-  for (int s = threadIdx.x; s < a.splits; s += 64) mx = fmaxf(mx, ml[2 * s]);
+  for (int s = threadIdx.x; s < a.parts; s += 64) mx = fmaxf(mx, ml[2 * s]);
   mx = row16_max(mx);
   mx = fmaxf(mx, xor_lane16(mx));
   mx = fmaxf(mx, xor_lane32(mx));
   float l = 0.f;
   f32x4_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-  for (int s = sub; s < a.splits; s += PAR) {
+  for (int s = sub; s < a.parts; s += PAR) {
     const float f = exp2_f(ml[2 * s] - mx);
     l += f * ml[2 * s + 1];
     const f32x4_t v = *reinterpret_cast<const f32x4_t*>(part + (int64_t)s * HD);
@@ -560,8 +567,7 @@ hipError_t rope_hd(const KRopeArgs& a, hipStream_t s) {
 
 template <bool F16, int HD>
 hipError_t decode_hd(const AttnDecodeArgs& a, hipStream_t s) {
-  const int64_t units = (int64_t)a.B * a.splits * a.kv_heads;
-  const dim3 grid((unsigned)((units + 3) / 4));
+  const dim3 grid((unsigned)(a.B * a.splits * (a.kv_heads / a.group)));
   switch (a.heads / a.kv_heads) {
     case 1: attn_decode_kernel<F16, HD, 1><<<grid, 256, 0, s>>>(a); break;
     case 2: attn_decode_kernel<F16, HD, 2><<<grid, 256, 0, s>>>(a); break;
@@ -570,7 +576,7 @@ hipError_t decode_hd(const AttnDecodeArgs& a, hipStream_t s) {
     default: return hipErrorInvalidValue;
   }
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  if (a.splits > 1) attn_merge_kernel<F16, HD><<<dim3((unsigned)(a.B * a.heads)), 64, 0, s>>>(a);
+  if (a.parts > 1) attn_merge_kernel<F16, HD><<<dim3((unsigned)(a.B * a.heads)), 64, 0, s>>>(a);
   return hipGetLastError();
 }
 
@@ -589,20 +595,21 @@ hipError_t prefill_hd(AttnPrefillArgs a, hipStream_t s) {
 
 }  // namespace
 
-// Ranges of the cache a decode step is cut into.  A wave takes one range of one
-// kv head; three waves a SIMD fit, and two to three rounds of them even out the
-// ends (64 sequences, 4 kv heads of 96, S = 2048, cache grown: 8 waves a CU
-// 97.8 us, 16 84.0, 32 81.1 us).  A range of under two 16-position tiles would
-// spend more on its own set-up and on the merge than on its rows.
-int attn_decode_splits(int64_t B, int S, int kv_heads, int* tiles_per_split) {
-  const int tiles = (S + 15) / 16;
-  const int64_t target = (int64_t)device_cus() * 32;
-  int64_t want = (target + B * kv_heads - 1) / (B * kv_heads);
+// Cuts a decode step into ranges of the cache, one workgroup for each and for each
+// group of 4, 2 or 1 kv heads.  Two fit a CU at once;
+// with eight (four rounds) the ends even out: the step above took 75 us with four a
+// CU, 72.6 with eight, 81 with sixteen.  A range of under two tiles would spend more
+// on its own set-up and on the merge than on its rows.
+void attn_decode_plan(AttnDecodeArgs& a) {
+  a.group = a.kv_heads % 4 == 0 ? 4 : a.kv_heads % 2 == 0 ? 2 : 1;
+  const int tiles = (a.S + 64 / a.group - 1) / (64 / a.group);
+  const int64_t units = a.B * (a.kv_heads / a.group);
+  int64_t want = ((int64_t)device_cus() * 8 + units - 1) / units;
   if (want > tiles / 2) want = tiles / 2;
   if (want < 1) want = 1;
-  const int per = (int)((tiles + want - 1) / want);
-  *tiles_per_split = per;
-  return (tiles + per - 1) / per;
+  a.tiles_per_split = (int)((tiles + want - 1) / want);
+  a.splits = (tiles + a.tiles_per_split - 1) / a.tiles_per_split;
+  a.parts = a.splits * (4 / a.group);
 }
 
 #define MHC_ATTN_HD(fn, a, s)                                      \

@@ -246,7 +246,8 @@ hipError_t launch_k_norm_rope(const KRopeArgs& a, hipStream_t s);
 // One decode step: B query tokens over S >= 1 cached positions and the new one.
 // k_past / v_past: [B, S, kv_heads, head_dim] with the given element strides (a
 // head's elements contiguous).  k_out / v_out (optional): the grown caches,
-// contiguous [B, S + 1, kv_heads, head_dim].  work: attn_decode_work_floats.
+// contiguous [B, S + 1, kv_heads, head_dim].  work: parts x (head_dim + 2) floats a
+// head, with more than one part.
 struct AttnDecodeArgs {
   const void* q;
   const void* k;
@@ -264,11 +265,13 @@ struct AttnDecodeArgs {
   int64_t ks_b, ks_s, ks_h, vs_b, vs_s, vs_h;
   int64_t B;
   int S, heads, kv_heads, head_dim;
-  int splits, tiles_per_split;
+  // attn_decode_plan: kv heads a workgroup takes, ranges, tiles of a range, partial
+  // results of a head
+  int group, splits, tiles_per_split, parts;
   bool f16;
   float q_eps, k_eps;
 };
-int attn_decode_splits(int64_t B, int S, int kv_heads, int* tiles_per_split);
+void attn_decode_plan(AttnDecodeArgs& a);
 hipError_t launch_attn_decode(const AttnDecodeArgs& a, hipStream_t s);
 
 // Causal attention of B sequences of T positions: q raw (normed and rotated

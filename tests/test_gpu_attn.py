@@ -77,7 +77,8 @@ def test_prefill(dev, hd, heads, kv, dtype, B, T):
 @pytest.mark.parametrize("hd,heads,kv,dtype,B,S,cache", [
     (96, 8, 4, BF, 1, 1, True), (96, 8, 4, BF, 3, 15, True), (96, 8, 4, BF, 2, 16, False),
     (64, 4, 4, BF, 2, 17, True), (128, 8, 2, BF, 1, 1000, True), (64, 3, 1, F16, 5, 47, True),
-    (96, 8, 4, F16, 64, 130, True), (128, 4, 1, F16, 1, 333, False), (96, 6, 2, BF, 300, 33, True)])
+    (96, 8, 4, F16, 64, 130, True), (128, 4, 1, F16, 1, 333, False), (96, 6, 2, BF, 300, 33, True),
+    (64, 6, 6, BF, 2, 95, True), (96, 3, 3, BF, 1, 129, True)])
 def test_decode(dev, hd, heads, kv, dtype, B, S, cache):
     m = _layer(hd, heads, kv, dtype)
     x, pos = torch.randn(B, 1, 128).to(dtype), _pos(hd, S, 1, dtype)
