@@ -508,7 +508,7 @@ int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void*
 
 /* Bytes of workspace mhc_moe_fwd needs, or -1 for a shape it does not take:
  * hidden and inter multiples of 32, 1 <= topk <= 8, topk <= experts <= 32,
- * M <= 262144. */
+ * M <= 262144, x of at most 4 GiB. */
 int64_t mhc_moe_workspace_bytes(int64_t M, int hidden, int inter, int experts, int topk);
 
 /* out [M, hidden] = sum over a token's topk experts of weight * expert(x).
@@ -524,7 +524,7 @@ int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
 
 /* -------------------------------- linear layers of the sublayers (inference)
  * 16-bit tensors (bf16 or fp16) of one dtype, fp32 sums rounded once; K a
- * multiple of 32, every weight's row count of 4; pointers 16-byte aligned.
+ * multiple of 32 up to 2^22, every weight's row count of 4; pointers 16-byte aligned.
  */
 
 /* out[i] [M, n[i]] = x [M, K] w[i]^T for `count` (one to three) weights

@@ -733,6 +733,7 @@ int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void*
 
 int64_t mhc_moe_workspace_bytes(int64_t M, int hidden, int inter, int experts, int topk) {
   if (M < 0 || M > 262144 || hidden < 32 || hidden % 32 != 0 || inter < 32 || inter % 32 != 0) return -1;
+  if (M * hidden > (int64_t)1 << 31) return -1;  // x rows are 32-bit byte offsets apart
   if (experts < 1 || experts > mhc::kMoeMaxExperts || topk < 1 || topk > mhc::kMoeMaxTopk || topk > experts) return -1;
   mhc::MoeArgs a{};
   a.M = M; a.hidden = hidden; a.inter = inter; a.experts = experts; a.topk = topk;

@@ -89,7 +89,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(LinearArgs a) {
 // ------------------------------------------------------------------ many rows
 // gemm_tile over BM x BN tiles; workgroups of one XCD take neighbouring tiles.
 template <bool F16, typename G, bool GLU>
-__global__ __launch_bounds__(G::THREADS, G::LDS > 80 * 1024 ? 1 : 2) void linear_kernel(LinearArgs a, int col_tiles) {
+__global__ __launch_bounds__(G::THREADS, G::WAVES) void linear_kernel(LinearArgs a, int col_tiles) {
   __shared__ __align__(16) char lds[G::LDS];
   constexpr int BM = G::BM, BN = G::BN;
   constexpr int kCols = GLU ? BN / 2 : BN;
@@ -99,45 +99,29 @@ __global__ __launch_bounds__(G::THREADS, G::LDS > 80 * 1024 ? 1 : 2) void linear
   const int logical = xcd * chunk - max(0, xcd - full) + blockIdx.x / 8;
   const Segment s = segment<kCols>(a, logical % col_tiles);
   const int64_t row0 = (int64_t)(logical / col_tiles) * BM;
-  const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r = lane & 15, g = lane >> 4;
   const int wm = wave % G::WGM, wn = wave / G::WGM;
   const int64_t kb = (int64_t)a.K * 2;
-  auto a_row = [&](int i) { return static_cast<const char*>(a.x) + min(row0 + i, a.M - 1) * kb; };
-  auto b_row = [&](int n) {
-    const char* w = GLU && n >= kCols ? static_cast<const char*>(a.w[1]) : s.w;
-    return w + min(s.n0 + n % kCols, s.N - 1) * kb;
-  };
+  auto a_row = [&](int i) { return (uint32_t)(min(row0 + i, a.M - 1) - row0) * (uint32_t)kb; };
+  auto b_base = [&](int n) { return (GLU && n >= kCols ? static_cast<const char*>(a.w[1]) : s.w) + s.n0 * kb; };
+  auto b_row = [&](int n) { return (uint32_t)min(n % kCols, s.N - 1 - s.n0) * (uint32_t)kb; };
   constexpr int HALF = G::NT / 2;
   auto col_tile = [&](int n) {
     return GLU ? wn * HALF + (n >= HALF ? n - HALF + BN / 32 : n) : wn * G::NT + n;
   };
   f32x4_t acc[G::NT][G::MT];
-  gemm_tile<F16, G>(lds, a.K, a_row, b_row, col_tile, acc);
+  gemm_tile<F16, G>(lds, a.K, static_cast<const char*>(a.x) + row0 * kb, a_row, b_base, b_row, col_tile, acc);
+  const int64_t row = row0 + wm * G::WM;
+  const int col = s.n0 + wn * (GLU ? G::WN / 2 : G::WN);
+  if constexpr (GLU)
 #pragma unroll
-  for (int m = 0; m < G::MT; ++m) {
-    const int64_t row = row0 + wm * G::WM + m * 16 + r;
-    if (row >= a.M) continue;
-    uint16_t* out = s.out + row * s.N;
-    if constexpr (GLU) {
+    for (int n = 0; n < HALF; ++n)
 #pragma unroll
-      for (int n = 0; n < HALF; ++n) {
-        const int col = s.n0 + wn * HALF * 16 + n * 16 + 4 * g;
-        if (col >= s.N) continue;
-        f32x4_t v;
+      for (int m = 0; m < G::MT; ++m)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = silu_mul(acc[n][m][i], acc[n + HALF][m][i]);
-        store4<F16>(out + col, v);
-      }
-    } else {
-#pragma unroll
-      for (int n = 0; n < G::NT; ++n) {
-        const int col = s.n0 + wn * G::WN + n * 16 + 4 * g;
-        if (col < s.N) store4<F16>(out + col, acc[n][m]);
-      }
-    }
-  }
+        for (int i = 0; i < 4; ++i) acc[n][m][i] = silu_mul(acc[n][m][i], acc[n + HALF][m][i]);
+  store_tile<F16, G, GLU ? G::WN / 2 : G::WN>(lds, s.out + row * s.N + col, s.N, a.M - row, s.N - col,
+                                              [&](int n, int m) { return acc[n][m]; });
 }
 
 template <bool F16, bool GLU, typename G>
@@ -146,38 +130,37 @@ hipError_t launch_tiles(const LinearArgs& a, int64_t work, int col_tiles, hipStr
   return hipGetLastError();
 }
 
-// Measured (K = 768 unless noted, us):
-//   * 16 x 16 tiles up to 448 of them: 384 (64 rows x 1536) 5.4 against 5.8 for
-//     64 x 64 tiles, 384 (128 x 768, K = 2048) 9.4 against 11.1; 512 (64 x 2048, GLU)
-//     7.9 against 6.8, 768 (256 x 768) 7.6 against 6.4.
-//   * 64 x 64 tiles while 128 x 128 ones would be fewer than 160: 96 (1024 x 1536)
-//     8.4 against 11.9, 192 (2048 x 1536) 12.8 against 12.6, 256 (1024 x 2048, GLU)
-//     19.7 against 15.1.
-//   8192 rows: 1536 columns 28.4 us (681 TFLOP/s; the three library products 39.0),
-//   GLU 2048 columns 64.2 us (803 TFLOP/s; two library products, silu and the
-//   multiplication 83.3).
+// 16 x 16 tiles up to 448 of them (K = 768 unless noted, us): 384 (64 rows x 1536) 5.4
+// against 5.8 for 64 x 64 tiles, 384 (128 x 768, K = 2048) 9.4 against 11.1; 512 (64 x
+// 2048, GLU) 7.9 against 6.8, 768 (256 x 768) 7.6 against 6.4.  Above, pick_tile's:
+// 8192 rows: 1536 columns 22.2 us (868 TFLOP/s; 28.4 with 128 x 128 tiles of 32-column
+// slices and stores from the accumulators, the three library products 39.0), GLU 2048
+// columns 52.1 us (990 TFLOP/s; 64.2 before, two library products, silu and the
+// multiplication 83.3).
 template <bool F16, bool GLU>
 hipError_t launch(const LinearArgs& a, hipStream_t s) {
-  auto cols = [&](int width) {
+  auto tiles = [&](int width) {
     int t = 0;
     for (int i = 0; i < (GLU ? 1 : a.count); ++i) t += (a.n[i] + width - 1) / width;
     return t;
   };
   auto rows = [&](int height) { return (a.M + height - 1) / height; };
-  if (cols(16) * rows(16) <= 448) {
-    const dim3 grid((unsigned)cols(16), (unsigned)rows(16));
+  if (tiles(16) * rows(16) <= 448) {
+    const dim3 grid((unsigned)tiles(16), (unsigned)rows(16));
     if (a.K >= 1536) skinny_kernel<F16, 16, GLU><<<grid, 16 * 64, 0, s>>>(a);
     else skinny_kernel<F16, 8, GLU><<<grid, 8 * 64, 0, s>>>(a);
     return hipGetLastError();
   }
-  constexpr int half = GLU ? 2 : 1;  // a GLU tile's columns are half gate, half up
-  if (a.K % 64 != 0) {
-    using G = GemmTile<64, 64, 2, 2, 4, 1>;
-    return launch_tiles<F16, GLU, G>(a, rows(64) * cols(64 / half), cols(64 / half), s);
+  auto cols = [&](int width) { return tiles(GLU ? width / 2 : width); };  // GLU: half gate, half up
+  switch (pick_tile(rows, cols, GLU)) {
+    case Tile::k256x256: return launch_tiles<F16, GLU, GemmTile<256, 256, 4, 2, 2>>(a, rows(256) * cols(256), cols(256), s);
+    case Tile::k128x192:
+      if constexpr (!GLU) return launch_tiles<F16, GLU, GemmTile<128, 192, 4, 2, 2>>(a, rows(128) * cols(192), cols(192), s);
+      [[fallthrough]];
+    case Tile::k128x128: return launch_tiles<F16, GLU, GemmTile<128, 128, 4, 2, 2>>(a, rows(128) * cols(128), cols(128), s);
+    case Tile::k128x64: return launch_tiles<F16, GLU, GemmTile<128, 64, 4, 1, 2>>(a, rows(128) * cols(64), cols(64), s);
+    default: return launch_tiles<F16, GLU, GemmTile<64, 64, 2, 2, 4>>(a, rows(64) * cols(64), cols(64), s);
   }
-  if (rows(128) * cols(128 / half) < 160)
-    return launch_tiles<F16, GLU, GemmTile<64, 64, 2, 2, 4, 2>>(a, rows(64) * cols(64 / half), cols(64 / half), s);
-  return launch_tiles<F16, GLU, GemmTile<128, 128, 2, 2, 2, 2>>(a, rows(128) * cols(128 / half), cols(128 / half), s);
 }
 
 }  // namespace

@@ -108,11 +108,13 @@ __global__ __launch_bounds__(kRouteTok) void moe_group_kernel(MoeArgs a) {
 //     Otherwise: BN columns of the down projection, scaled by the row's weight.
 //   * Workgroups of one XCD take neighbouring tiles (the same expert's weights stay
 //     in its L2).
-// 8192 tokens, 8 experts, top 2, 768 x 1024: 76 us for gate and up (51.5 GFLOP, 680
-// TFLOP/s), 47 us for down (25.8 GFLOP, 549 TFLOP/s); 128 x 256 tiles 84 and 48 us.
+// 8192 tokens, 8 experts, top 2, 768 x 1024: 71 us for gate and up (128 x 128 tiles, 51.5
+// GFLOP, 725 TFLOP/s; 77 with 32-column slices and stores from the accumulators), 41 us
+// for down (128 x 192 tiles, 25.8 GFLOP, 629 TFLOP/s; 47 before).  The dense layer's rows
+// take 56 and 27 us: the rest is the gathered rows and the experts' partly filled tiles.
 // The layer's loop over experts took 1.6 ms, of which library products were 290 us.
 template <bool F16, typename G, bool GLU>
-__global__ __launch_bounds__(G::THREADS, 2) void moe_gemm_kernel(MoeArgs a) {
+__global__ __launch_bounds__(G::THREADS, G::WAVES) void moe_gemm_kernel(MoeArgs a) {
   constexpr int BM = G::BM, BN = G::BN;
   __shared__ __align__(16) char lds[G::LDS];
   const int N = GLU ? a.inter : a.hidden;
@@ -134,51 +136,46 @@ __global__ __launch_bounds__(G::THREADS, 2) void moe_gemm_kernel(MoeArgs a) {
   }
   const int row_end = a.offsets[e + 1], row0 = a.offsets[e] + mt * BM;
 
-  const int lane = threadIdx.x & 63;
+  const int r = threadIdx.x & 15;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r = lane & 15, g = lane >> 4;
   const int wm = wave % G::WGM, wn = wave / G::WGM;
+  const uint32_t kb = (uint32_t)K * 2;
+  const char* x = GLU ? static_cast<const char*>(a.x) : static_cast<const char*>(a.h) + (int64_t)row0 * kb;
   auto a_row = [&](int i) {
     const int row = min(row0 + i, row_end - 1);
-    return GLU ? static_cast<const char*>(a.x) + (int64_t)a.row_tok[row] * K * 2
-               : static_cast<const char*>(a.h) + (int64_t)row * K * 2;
+    return GLU ? (uint32_t)a.row_tok[row] * kb : (uint32_t)(row - row0) * kb;
   };
-  auto b_row = [&](int n) {
+  auto b_base = [&](int n) {
     const void* w = GLU ? (n < kCols ? a.gate_w[e] : a.up_w[e]) : a.down_w[e];
-    return static_cast<const char*>(w) + (int64_t)min(n0 + n % kCols, N - 1) * K * 2;
+    return static_cast<const char*>(w) + (int64_t)n0 * kb;
   };
+  auto b_row = [&](int n) { return (uint32_t)min(n % kCols, N - 1 - n0) * kb; };
   // GLU: this wave's gate columns, then its up columns
   constexpr int HALF = G::NT / 2;
   auto col_tile = [&](int n) {
     return GLU ? wn * HALF + (n >= HALF ? n - HALF + BN / 32 : n) : wn * G::NT + n;
   };
   f32x4_t acc[G::NT][G::MT];
-  gemm_tile<F16, G>(lds, K, a_row, b_row, col_tile, acc);
+  gemm_tile<F16, G>(lds, K, x, a_row, b_base, b_row, col_tile, acc);
+  const int row = row0 + wm * G::WM, col = n0 + wn * (GLU ? G::WN / 2 : G::WN);
+  float w[G::MT];
+  if constexpr (!GLU)
 #pragma unroll
-  for (int m = 0; m < G::MT; ++m) {
-    const int row = row0 + wm * G::WM + m * 16 + r;
-    if (row >= row_end) continue;
-    if constexpr (GLU) {
-      uint16_t* out = static_cast<uint16_t*>(a.h) + (int64_t)row * N;
+    for (int m = 0; m < G::MT; ++m) w[m] = a.row_w[min(row + m * 16 + r, row_end - 1)];
+  uint16_t* out = static_cast<uint16_t*>(GLU ? a.h : a.y) + (int64_t)row * N + col;
 #pragma unroll
-      for (int n = 0; n < HALF; ++n) {
-        const int col = n0 + wn * HALF * 16 + n * 16 + 4 * g;
-        if (col >= N) continue;
-        f32x4_t v;
+  for (int n = 0; n < (GLU ? HALF : G::NT); ++n)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = silu_mul(acc[n][m][i], acc[n + HALF][m][i]);
-        store4<F16>(out + col, v);
-      }
-    } else {
-      uint16_t* out = static_cast<uint16_t*>(a.y) + (int64_t)row * N;
-      const float w = a.row_w[row];
+    for (int m = 0; m < G::MT; ++m) {
+      if constexpr (GLU) {
 #pragma unroll
-      for (int n = 0; n < G::NT; ++n) {
-        const int col = n0 + wn * G::WN + n * 16 + 4 * g;
-        if (col < N) store4<F16>(out + col, acc[n][m] * w);
+        for (int i = 0; i < 4; ++i) acc[n][m][i] = silu_mul(acc[n][m][i], acc[n + HALF][m][i]);
+      } else {
+        acc[n][m] *= w[m];
       }
     }
-  }
+  store_tile<F16, G, GLU ? G::WN / 2 : G::WN>(lds, out, N, row_end - row, N - col,
+                                              [&](int n, int m) { return acc[n][m]; });
 }
 
 // out[token] = the sum of its experts' rows, 8 columns a thread.
@@ -215,15 +212,23 @@ hipError_t launch_tiles(const MoeArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// The dense layers' rule (mhc_linear.hip): 64 x 64 tiles while 128 x 128 ones would
-// be fewer than 160.
+// The dense layers' rule; half an expert's last row tile is padding on average.
 template <bool F16, bool GLU>
 hipError_t launch_gemm(const MoeArgs& a, hipStream_t s) {
-  const int N = GLU ? a.inter : a.hidden, K = GLU ? a.hidden : a.inter;
-  const int64_t rows = a.M * a.topk, tiles = (rows / 128 + 1) * ((N + (GLU ? 63 : 127)) / (GLU ? 64 : 128));
-  if (K % 64 != 0) return launch_tiles<F16, GLU, GemmTile<64, 64, 2, 2, 4, 1>>(a, s);
-  if (tiles < 160) return launch_tiles<F16, GLU, GemmTile<64, 64, 2, 2, 4, 2>>(a, s);
-  return launch_tiles<F16, GLU, GemmTile<128, 128, 2, 2, 2, 2>>(a, s);
+  auto rows = [&](int height) { return a.M * a.topk / height + (a.experts + 1) / 2; };
+  auto cols = [&](int width) {
+    const int w = GLU ? width / 2 : width;
+    return ((GLU ? a.inter : a.hidden) + w - 1) / w;
+  };
+  switch (pick_tile(rows, cols, GLU)) {
+    case Tile::k256x256: return launch_tiles<F16, GLU, GemmTile<256, 256, 4, 2, 2>>(a, s);
+    case Tile::k128x192:
+      if constexpr (!GLU) return launch_tiles<F16, GLU, GemmTile<128, 192, 4, 2, 2>>(a, s);
+      [[fallthrough]];
+    case Tile::k128x128: return launch_tiles<F16, GLU, GemmTile<128, 128, 4, 2, 2>>(a, s);
+    case Tile::k128x64: return launch_tiles<F16, GLU, GemmTile<128, 64, 4, 1, 2>>(a, s);
+    default: return launch_tiles<F16, GLU, GemmTile<64, 64, 2, 2, 4>>(a, s);
+  }
 }
 
 template <bool F16>

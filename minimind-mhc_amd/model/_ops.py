@@ -662,12 +662,11 @@ def plain_tensors(dtype: torch.dtype, dev: torch.device, *ts) -> bool:
 
 
 # Multiply-adds up to which one linear layer runs on mhc_linear_fwd.  The library's
-# call costs the host 19 us (MI355X box, torch 2.10), the kernel's 7; up to here the
-# kernel takes at most 15 us, so the cheaper call wins although the library's kernel
-# is a little faster (512 rows, 768 x 6400: 14.6 against 11.1 us; 2048 rows,
-# 2048 x 768: 14.7 against 14.1).  Past it the library's kernel does (8192 rows,
-# 768 x 768: 19.1 against 15.5 us).
-LINEAR_MAX_MACS = 3_300_000_000
+# call costs the host 19 us (MI355X, torch 2.10), the kernel's 7, and up to here the
+# kernel is as fast: 8192 rows, 768 x 768: 14.6 against 15.5 us; 2048 x 768: 30.1
+# against 30.5; 512 rows, 768 x 6400: 11.9 against 11.1.  Past it the library's kernel
+# is the faster one (8192 rows, 768 x 6400: 86 against 97 us).
+LINEAR_MAX_MACS = 13_000_000_000
 
 
 def _linear_weights(x: torch.Tensor, mods):
@@ -676,7 +675,7 @@ def _linear_weights(x: torch.Tensor, mods):
             or x.dim() < 2 or x.numel() == 0 or not x.is_contiguous()):
         return None
     K = x.shape[-1]
-    if K % 32 != 0:
+    if K % 32 != 0 or K > 1 << 22:
         return None
     ws = []
     for m in mods:

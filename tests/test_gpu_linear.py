@@ -36,8 +36,14 @@ def _close(want, got, dt):
     # 64 x 64 tiles: just past the count, ragged both ways, K of 64 and of 32
     (768, (768, 384, 384), 75, BF), (64, (1536,), 1025, BF), (160, (516, 68), 300, BF),
     (32, (4096,), 63, F16), (768, (6400,), 65, BF), (2048, (768,), 700, BF),
-    # 128 x 128 tiles: the first count, ragged, one and two stages of K
-    (64, (2048,), 1280, BF), (128, (1540, 260), 1700, F16), (768, (768, 384, 384), 2300, BF)])
+    # 128 x 64 tiles: the first count, ragged, K of 64 and of 32
+    (64, (2048,), 768, BF), (160, (516, 68), 2200, F16), (2048, (768,), 2050, BF),
+    # 128 x 128 tiles: one and two slices of K, ragged
+    (64, (2048,), 2176, BF), (128, (1540, 260), 2100, F16), (96, (1024, 512), 3001, BF),
+    # 128 x 192 tiles: the first count, ragged rows, columns and K
+    (64, (768,), 8192, BF), (160, (764, 380), 5400, F16), (768, (768, 384, 384), 4225, BF),
+    # 256 x 256 tiles: nearly full rounds, ragged rows, columns and K
+    (96, (6396,), 4001, BF), (64, (4096, 2048, 260), 3900, F16)])
 def test_products(dev, K, Ns, M, dt):
     mods = _linears(K, Ns, dt, dev)
     x = torch.randn(M, K, device=dev).to(dt)
@@ -50,7 +56,8 @@ def test_products(dev, K, Ns, M, dt):
 
 @pytest.mark.parametrize("K,N,M,dt", [
     (768, 2048, 1, BF), (768, 2048, 48, BF), (768, 2048, 64, BF), (2048, 20, 30, F16), (32, 36, 7, BF),
-    (96, 1100, 130, BF), (64, 4100, 600, BF), (768, 2048, 515, F16), (128, 2432, 1111, BF)])
+    (96, 1100, 130, BF), (64, 4100, 600, BF), (768, 2048, 515, F16), (128, 2432, 1111, BF),
+    (96, 2052, 1100, BF), (32, 4100, 1500, F16), (64, 4100, 3500, BF), (160, 2048, 7300, F16)])
 def test_glu(dev, K, N, M, dt):
     gate, up = _linears(K, (N, N), dt, dev)
     x = torch.randn(1, M, K, device=dev).to(dt)
@@ -99,4 +106,4 @@ def test_calls_left_to_torch(dev):
         with torch.amp.autocast("cuda", dtype=BF):
             assert _ops.linears(x, a) is None
         big = torch.empty(6000, 768, device=dev, dtype=BF)
-        assert _ops.linears(big, *_linears(768, (768,), BF, dev)) is None  # faster in the library
+        assert _ops.linears(big, *_linears(768, (4096,), BF, dev)) is None  # faster in the library

@@ -58,7 +58,8 @@ def _check(m, x, probs):
 @pytest.mark.parametrize("D,inter,experts,topk,dtype,M", [
     (768, 1024, 8, 2, BF, 300), (768, 1024, 8, 2, BF, 1), (512, 512, 4, 1, BF, 129),
     (32, 32, 2, 2, BF, 127), (64, 96, 8, 3, BF, 128), (1024, 160, 4, 2, F16, 257),
-    (288, 416, 32, 8, BF, 64), (768, 768, 1, 1, F16, 200), (96, 1056, 5, 2, BF, 1025)])
+    (288, 416, 32, 8, BF, 64), (768, 768, 1, 1, F16, 200), (96, 1056, 5, 2, BF, 1025),
+    (768, 64, 8, 2, BF, 4100), (32, 2048, 8, 2, BF, 3200), (6400, 32, 4, 2, F16, 2048)])
 def test_experts(dev, D, inter, experts, topk, dtype, M):
     m = _layer(D, inter, experts, topk, dtype, norm=M != 129).to(dev)
     x = torch.randn(M, D, device=dev).to(dtype)
