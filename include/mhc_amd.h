@@ -515,10 +515,11 @@ int64_t mhc_moe_workspace_bytes(int64_t M, int hidden, int inter, int experts, i
  * probs [M, experts]: the router's softmax; the topk largest are taken (the
  * lower index where two are equal) and, with norm_topk, divided by their sum.
  * gate_w, up_w, down_w: host arrays of `experts` device pointers to
- * [inter, hidden], [inter, hidden] and [hidden, inter].  Device pointers are
+ * [inter, hidden], [inter, hidden] and [hidden, inter].  zero: one element set to
+ * 0 on the way (the layer's auxiliary loss in inference), or null.  Device pointers are
  * 16-byte aligned. */
 int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
-                const void* const* up_w, const void* const* down_w, void* out, void* workspace,
+                const void* const* up_w, const void* const* down_w, void* out, void* zero, void* workspace,
                 int64_t workspace_bytes, int64_t M, int hidden, int inter, int experts, int topk,
                 int norm_topk, int dtype, hipStream_t stream);
 

@@ -741,7 +741,7 @@ int64_t mhc_moe_workspace_bytes(int64_t M, int hidden, int inter, int experts, i
 }
 
 int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
-                const void* const* up_w, const void* const* down_w, void* out, void* workspace,
+                const void* const* up_w, const void* const* down_w, void* out, void* zero, void* workspace,
                 int64_t workspace_bytes, int64_t M, int hidden, int inter, int experts, int topk,
                 int norm_topk, int dtype, hipStream_t stream) {
   const char* fn = "mhc_moe_fwd";
@@ -760,7 +760,7 @@ int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
       if (!w || !aligned16(w)) return fail(hipErrorInvalidValue, "%s: null or unaligned weight of expert %d", fn, e);
     a.gate_w[e] = gate_w[e]; a.up_w[e] = up_w[e]; a.down_w[e] = down_w[e];
   }
-  a.x = x; a.probs = probs; a.out = out;
+  a.x = x; a.probs = probs; a.out = out; a.zero = zero;
   a.M = M; a.hidden = hidden; a.inter = inter; a.experts = experts; a.topk = topk;
   a.norm_topk = norm_topk != 0; a.f16 = dtype == mhc::kF16;
   mhc::moe_workspace(a, static_cast<char*>(workspace));

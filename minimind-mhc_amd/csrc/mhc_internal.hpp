@@ -299,6 +299,7 @@ struct MoeArgs {
   const void* x;
   const void* probs;
   void* out;
+  void* zero;  // one element set to 0, or null
   const void* gate_w[kMoeMaxExperts];
   const void* up_w[kMoeMaxExperts];
   const void* down_w[kMoeMaxExperts];

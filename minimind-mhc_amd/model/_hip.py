@@ -100,7 +100,7 @@ _SIGNATURES = {
     "mhc_linear_fwd": (_I, [_P, _P, _P, _P, _I, _I64, _I, _I, _P]),
     "mhc_glu_fwd": (_I, [_P, _P, _P, _P, _I64, _I, _I, _I, _P]),
     "mhc_moe_workspace_bytes": (_I64, [_I64, _I, _I, _I, _I]),
-    "mhc_moe_fwd": (_I, [_P, _P, _P, _P, _P, _P,          # x, probs, gate_w, up_w, down_w, out
+    "mhc_moe_fwd": (_I, [_P, _P, _P, _P, _P, _P, _P,      # x, probs, gate_w, up_w, down_w, out, zero
                          _P, _I64, _I64, _I, _I, _I, _I, _I, _I, _P]),
     "mhc_attn_prefill_fwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P,  # q, k, v, gains, cos, sin, k_out, out
                                   _I64, _I, _I, _I, _I, _I, _F, _F, _P]),

@@ -812,14 +812,18 @@ def attn_decode(m, q, k, v, position_embeddings, past, use_cache: bool):
     return out, grown
 
 
-def moe_experts(experts, x: torch.Tensor, probs: torch.Tensor, topk: int, norm_topk: bool):
+def moe_experts(experts, x: torch.Tensor, probs: torch.Tensor, topk: int, norm_topk: bool,
+                zero: Optional[torch.Tensor] = None):
     """The routed experts' weighted sum for x [M, hidden] on the HIP kernels, or
     None for a call they do not take.  experts: modules with gate_proj, up_proj
     and down_proj (plain nn.Linear without bias) and SiLU between them; probs
-    [M, experts], the router's softmax."""
+    [M, experts], the router's softmax; zero: a tensor of x's type whose one element
+    the last launch sets to 0."""
     if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or not plain_call()
             or x.dim() != 2 or x.shape[0] == 0 or not x.is_contiguous()
             or probs.shape != (x.shape[0], len(experts)) or not probs.is_contiguous()):
+        return None
+    if zero is not None and (zero.numel() != 1 or zero.dtype != x.dtype or zero.device != x.device):
         return None
     M, D = x.shape
     kind, ws = type(experts[0]), ([], [], [])
@@ -842,7 +846,7 @@ def moe_experts(experts, x: torch.Tensor, probs: torch.Tensor, topk: int, norm_t
     out = torch.empty_like(x)
     work = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     ptrs = [(ctypes.c_void_p * len(w))(*[t.data_ptr() for t in w]) for w in ws]
-    H.check(lib.mhc_moe_fwd(x.data_ptr(), probs.data_ptr(), *ptrs, out.data_ptr(),
+    H.check(lib.mhc_moe_fwd(x.data_ptr(), probs.data_ptr(), *ptrs, out.data_ptr(), H.ptr(zero),
                             work.data_ptr(), nbytes, M, D, inter, len(experts), topk,
                             int(norm_topk), H.dtype_tag(x), H.stream(x.device)), "mhc_moe_fwd")
     return out

@@ -231,11 +231,12 @@ class MOEFeedForward(nn.Module):
         b, l, d = x.shape
         xf = x.view(-1, d)
         scores = F.softmax(self.gate(xf), dim=-1)
-        if not self.training:
+        if not self.training and type(self.experts[0]) is FeedForward:
+            aux = scores.new_empty(())
             y = _ops.moe_experts(self.experts, xf, scores, self.config.num_experts_per_tok,
-                                 self.config.norm_topk_prob)
+                                 self.config.norm_topk_prob, zero=aux)
             if y is not None:
-                self.aux_loss = scores.new_zeros(1).squeeze()
+                self.aux_loss = aux
                 return y.view(b, l, d)
         w, idx = torch.topk(scores, k=self.config.num_experts_per_tok, dim=-1, sorted=False)
         if self.config.norm_topk_prob:

@@ -11,7 +11,7 @@ import torch
 import torch.nn.functional as F
 
 from model import _ops
-from model.model_minimind import MiniMindConfig, MOEFeedForward
+from model.model_minimind import FeedForward, MiniMindConfig, MOEFeedForward
 
 pytestmark = pytest.mark.gpu
 BF, F16 = torch.bfloat16, torch.float16
@@ -129,6 +129,21 @@ def test_replay_in_a_graph(dev):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(y, m(x)), i
+
+
+def test_other_experts_keep_their_own_forward(dev):
+    class Doubled(FeedForward):
+        def forward(self, x):
+            return 2 * super().forward(x)
+
+    m = _layer(64, 64, 4, 2, BF).to(dev)
+    twice = copy.deepcopy(m)
+    for e in twice.experts:
+        e.__class__ = Doubled
+    x = torch.randn(1, 40, 64, device=dev).to(BF)
+    with torch.inference_mode():
+        want, got = 2 * m(x).float(), twice(x).float()
+    assert float((got - want).abs().max()) <= 0.02 * float(want.abs().max())
 
 
 def test_calls_left_to_the_loop(dev):
