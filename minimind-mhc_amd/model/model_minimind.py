@@ -2,11 +2,12 @@
 
 Restates the reference model (model/model_minimind.py:76-461) as the
 end-to-end harness for prefill / decode measurements: same config fields,
-module tree and parameter names (so reference state dicts load), with the
-sublayers F (attention, SwiGLU FFN, MoE) on PyTorch-ROCm ops and every mHC
+module tree and parameter names (so reference state dicts load), with every mHC
 piece (StreamExpand, MHCConnection_Fused / _FusedNoHres, MHCHead) on the HIP
-kernels of this package.  Attention uses torch SDPA (the reference's second
-backend, model/model_minimind.py:208-232); flash-attn is not used.
+kernels of this package.  The sublayers F (attention, SwiGLU FFN, MoE) run on HIP
+kernels in 16-bit inference (model/_ops.py says for which calls) and on PyTorch-ROCm
+ops otherwise, attention then on torch SDPA (the reference's second backend,
+model/model_minimind.py:208-232); flash-attn is not used.
 
 Differences from the reference, all outside the mHC path:
   * MiniMindConfig is a plain class (no transformers.PretrainedConfig) and
