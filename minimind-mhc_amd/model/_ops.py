@@ -633,6 +633,13 @@ def sinkhorn_bwd(m: torch.Tensor, g: torch.Tensor, iters: int, eps: float,
 # transform, no tracing or compiling, no dispatch mode, no autocast, and
 # submodules that nobody has hooked or patched.
 
+def on_current_device(t: torch.Tensor) -> bool:
+    """Whether t, a GPU tensor, lies on the device the library would launch on.  Its entry points set no
+    device, and a device's default stream is handle 0 on every device, so for a tensor
+    of another one the launch would go to the wrong GPU; torch ops set the device."""
+    return t.get_device() == torch.cuda.current_device()
+
+
 def plain_call() -> bool:
     """Whether nothing is recording, transforming or tracing torch ops here."""
     return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda")
@@ -672,7 +679,7 @@ LINEAR_MAX_MACS = 13_000_000_000
 def _linear_weights(x: torch.Tensor, mods):
     """The weights of bias-free nn.Linear layers the kernels can apply to x, or None."""
     if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or not plain_call()
-            or x.dim() < 2 or x.numel() == 0 or not x.is_contiguous()):
+            or not on_current_device(x) or x.dim() < 2 or x.numel() == 0 or not x.is_contiguous()):
         return None
     K = x.shape[-1]
     if K % 32 != 0 or K > 1 << 22:
@@ -738,7 +745,7 @@ def attn_route(m, q, k, v, position_embeddings, past) -> Optional[str]:
     q [B, T, heads * head_dim]; k, v [B, T, kv_heads * head_dim]."""
     H_, KV, hd = m.n_local_heads, m.n_local_kv_heads, m.head_dim
     if (not q.is_cuda or q.dtype not in (torch.bfloat16, torch.float16) or hd not in ATTN_HEAD_DIMS
-            or q.dim() != 3 or H_ % KV != 0 or not plain_call()):
+            or q.dim() != 3 or H_ % KV != 0 or not plain_call() or not on_current_device(q)):
         return None
     B, T, _ = q.shape
     if B * T == 0 or (m.training and m.dropout > 0) or (T > 1 and not m.is_causal):
@@ -820,7 +827,7 @@ def moe_experts(experts, x: torch.Tensor, probs: torch.Tensor, topk: int, norm_t
     [M, experts], the router's softmax; zero: a tensor of x's type whose one element
     the last launch sets to 0."""
     if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or not plain_call()
-            or x.dim() != 2 or x.shape[0] == 0 or not x.is_contiguous()
+            or not on_current_device(x) or x.dim() != 2 or x.shape[0] == 0 or not x.is_contiguous()
             or probs.shape != (x.shape[0], len(experts)) or not probs.is_contiguous()):
         return None
     if zero is not None and (zero.numel() != 1 or zero.dtype != x.dtype or zero.device != x.device):

@@ -1,0 +1,83 @@
+"""Which calls of the sublayers (attention, feed-forward, routed experts, lm_head) run on
+the HIP kernels: every other call has to reach the torch ops, as the layers' plain source
+says it would."""
+from __future__ import annotations
+
+import pytest
+import torch
+from torch import nn
+
+from model import _ops
+from model.model_minimind import (Attention, FeedForward, MiniMindConfig, MOEFeedForward,
+                                  precompute_freqs_cis)
+
+BF = torch.bfloat16
+
+
+def _cfg(**kw):
+    return MiniMindConfig(hidden_size=128, num_hidden_layers=1, num_attention_heads=2,
+                          num_key_value_heads=1, head_dim=64, intermediate_size=64, vocab_size=64,
+                          max_position_embeddings=64, **kw)
+
+
+def _fake(shape, device="cuda:1"):
+    """A tensor of that device with no storage: enough for the rules to look at."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        return torch.empty(shape, device=device, dtype=BF)
+
+
+def _taken(monkeypatch, device, current):
+    """What the rules say to calls that nothing but the device speaks against; with the
+    device right, they get as far as the first look at the data."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current)
+    monkeypatch.setattr(_ops, "plain_tensors", lambda *a: True)
+    attn, moe = Attention(_cfg()).to(BF).eval(), MOEFeedForward(_cfg()).to(BF).eval()
+    seen = []
+
+    def library():
+        seen.append(1)
+        raise RuntimeError("the library")
+
+    monkeypatch.setattr(_ops.H, "load", library)
+    lin = nn.Linear(128, 64, bias=False).to(BF)
+    q, kv, pos = _fake((1, 4, 128), device), _fake((1, 4, 64), device), _fake((4, 64), device)
+    out = [_ops._linear_weights(q, (lin,)) is not None,
+           _ops.attn_route(attn, q, kv, kv, (pos, pos), None) is not None]
+    for call in (lambda: _ops.linears(q, lin), lambda: _ops.glu(q, lin, lin),
+                 lambda: _ops.moe_experts(moe.experts, q[0], _fake((4, 4), device), 1, True)):
+        seen.clear()
+        try:
+            call()
+        except RuntimeError:
+            pass
+        out.append(bool(seen))
+    return out
+
+
+@pytest.mark.parametrize("current,taken", [(1, True), (0, False)])
+def test_only_tensors_of_the_current_device(monkeypatch, current, taken):
+    """The library launches on the current device: tensors of another one are torch's."""
+    with torch.no_grad():
+        assert _taken(monkeypatch, "cuda:1", current) == [taken] * 5
+
+
+@pytest.mark.gpu
+def test_another_device_current_runs_torch_ops(dev, monkeypatch):
+    torch.manual_seed(0)
+    ff, moe, attn = FeedForward(_cfg()), MOEFeedForward(_cfg()), Attention(_cfg())
+    x = torch.randn(1, 4, 128, device=dev).to(BF)
+    pos = tuple(t.to(dev).to(BF) for t in precompute_freqs_cis(64, 4))
+    with torch.no_grad():
+        for m in (ff, moe, attn):
+            m.to(dev).to(BF).eval()
+        want = [ff(x), moe(x), attn(x, pos, None, True)[0]]
+        monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+        q, k, v = attn.q_proj(x), attn.k_proj(x), attn.v_proj(x)
+        assert _ops.linears(x, attn.q_proj) is None and _ops.glu(x, ff.gate_proj, ff.up_proj) is None
+        assert _ops.attn_route(attn, q, k, v, pos, None) is None
+        assert _ops.moe_experts(moe.experts, x[0], torch.softmax(moe.gate(x[0]), -1), 1, True) is None
+        got = [ff(x), moe(x), attn(x, pos, None, True)[0]]
+    for w, g in zip(want, got):
+        # both round sums and intermediates to bf16 (8 bits): a few half-steps of the largest
+        assert float((w.float() - g.float()).abs().max()) <= 6 * 2.0 ** -9 * float(w.float().abs().max())
