@@ -678,6 +678,8 @@ LINEAR_MAX_MACS = 13_000_000_000
 
 def _linear_weights(x: torch.Tensor, mods):
     """The weights of bias-free nn.Linear layers the kernels can apply to x, or None."""
+    if not isinstance(x, torch.Tensor):  # an fx Proxy: the torch ops are traced
+        return None
     if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or not plain_call()
             or not on_current_device(x) or x.dim() < 2 or x.numel() == 0 or not x.is_contiguous()):
         return None

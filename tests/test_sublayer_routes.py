@@ -81,3 +81,13 @@ def test_another_device_current_runs_torch_ops(dev, monkeypatch):
     for w, g in zip(want, got):
         # both round sums and intermediates to bf16 (8 bits): a few half-steps of the largest
         assert float((w.float() - g.float()).abs().max()) <= 6 * 2.0 ** -9 * float(w.float().abs().max())
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_feed_forward_traces_with_fx(grad):
+    ff, x = FeedForward(_cfg()), torch.randn(2, 3, 128)
+    with torch.set_grad_enabled(grad):
+        gm = torch.fx.symbolic_trace(ff)
+        assert torch.equal(gm(x), ff(x))
+    called = {n.target for n in gm.graph.nodes if n.op == "call_module"}
+    assert called == {"gate_proj", "up_proj", "down_proj"}
