@@ -209,10 +209,13 @@ class FeedForward(nn.Module):
         self.up_proj = nn.Linear(config.hidden_size, inter, bias=False)
 
     def forward(self, x):
-        h = _ops.glu(x, self.gate_proj, self.up_proj)
-        if h is None:
-            h = F.silu(self.gate_proj(x)) * self.up_proj(x)
-        return _ops.linear(h, self.down_proj)
+        if torch.jit.is_scripting():  # the script compiler leaves the other branch out
+            return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
+        else:
+            h = _ops.glu(x, self.gate_proj, self.up_proj)
+            if h is None:
+                h = F.silu(self.gate_proj(x)) * self.up_proj(x)
+            return _ops.linear(h, self.down_proj)
 
 
 class MOEFeedForward(nn.Module):

@@ -91,3 +91,10 @@ def test_feed_forward_traces_with_fx(grad):
         assert torch.equal(gm(x), ff(x))
     called = {n.target for n in gm.graph.nodes if n.op == "call_module"}
     assert called == {"gate_proj", "up_proj", "down_proj"}
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_feed_forward_scripts(grad):
+    ff, x = FeedForward(_cfg()), torch.randn(2, 3, 128)
+    with torch.set_grad_enabled(grad):
+        assert torch.equal(torch.jit.script(ff)(x), ff(x))
