@@ -641,12 +641,14 @@ def on_current_device(t: torch.Tensor) -> bool:
 
 
 def plain_call() -> bool:
-    """Whether nothing is recording, transforming or tracing torch ops here."""
-    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda")
+    """Whether nothing is recording, transforming or tracing torch ops here.
+    Compiling is asked first: Dynamo knows that answer, and cannot trace the rest."""
+    return not (torch.compiler.is_compiling()
+                or torch.is_grad_enabled() or torch.is_autocast_enabled("cuda")
                 or torch.autograd.forward_ad._current_level >= 0
                 or torch._C._len_torch_dispatch_stack() > 0
                 or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.compiler.is_compiling() or torch.jit.is_tracing())
+                or torch.jit.is_tracing())
 
 
 _GLOBAL_HOOKS = torch.nn.modules.module

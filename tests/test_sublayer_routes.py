@@ -98,3 +98,49 @@ def test_feed_forward_scripts(grad):
     ff, x = FeedForward(_cfg()), torch.randn(2, 3, 128)
     with torch.set_grad_enabled(grad):
         assert torch.equal(torch.jit.script(ff)(x), ff(x))
+
+
+def _plain_calls():
+    """plain_call as each kind of tracer and transform sees it, without grad mode."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    seen = {}
+
+    def ask(name, out=None):
+        def call(x):
+            seen[name] = _ops.plain_call()
+            return x + 1
+        return call
+
+    x = torch.randn(3)
+    with torch.no_grad():
+        ask("eager")(x)
+        make_fx(ask("make_fx"))(x)
+        torch.vmap(ask("vmap"))(x)
+        torch.func.jvp(ask("jvp"), (x,), (x,))
+        torch.jit.trace(ask("jit.trace"), (x,), check_trace=False)
+        with torch.autograd.forward_ad.dual_level():
+            ask("dual level")(x)
+        seen["compile"] = torch.compile(_ops.plain_call, fullgraph=True, backend="eager")()
+    ask("grad mode")(x)
+    return seen
+
+
+def test_plain_call_under_tracers_and_transforms():
+    seen = _plain_calls()
+    assert seen.pop("eager") is True
+    assert len(seen) == 7 and not any(seen.values()), seen
+
+
+@pytest.mark.gpu
+def test_compiled_sublayers_keep_one_graph(dev):
+    """16-bit inference under torch.compile: the torch ops in one graph, as in the source."""
+    torch.manual_seed(0)
+    ff, attn = FeedForward(_cfg()).to(dev).to(BF).eval(), Attention(_cfg()).to(dev).to(BF).eval()
+    x = torch.randn(1, 4, 128, device=dev).to(BF)
+    pos = tuple(t.to(dev).to(BF) for t in precompute_freqs_cis(64, 4))
+    with torch.no_grad():
+        for fn in (ff, lambda t: attn(t, pos, None, True)[0]):
+            torch._dynamo.reset()
+            got, want = torch.compile(fn, fullgraph=True, backend="eager")(x), fn(x)
+            # the compiled call's torch ops round intermediates that the kernels do not
+            assert float((want.float() - got.float()).abs().max()) <= 6 * 2.0 ** -9 * float(want.float().abs().max())
