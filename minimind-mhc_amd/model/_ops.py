@@ -13,6 +13,7 @@ import weakref
 from typing import Optional
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import _hip as H
 
@@ -630,7 +631,7 @@ def sinkhorn_bwd(m: torch.Tensor, g: torch.Tensor, iters: int, eps: float,
 # Kernels in place of the torch ops of the sublayers.  They record no autograd
 # graph and see only data pointers, so a call takes them only when nothing but
 # the numbers could tell: no grad mode, no forward-mode level, no functorch
-# transform, no tracing or compiling, no dispatch mode, no autocast, and
+# transform, no tracing or compiling, no dispatch or function mode, no autocast, and
 # submodules that nobody has hooked or patched.
 
 def on_current_device(t: torch.Tensor) -> bool:
@@ -640,13 +641,22 @@ def on_current_device(t: torch.Tensor) -> bool:
     return t.get_device() == torch.cuda.current_device()
 
 
+def _function_modes() -> bool:
+    """Whether a torch-function mode could see or replace the torch ops.  The one that
+    torch.set_default_device and `with torch.device(...)` leave on the stack only changes
+    factory calls without a device, of which the sublayers make none."""
+    return (torch._C._len_torch_function_stack() > 0
+            and any(type(m) is not DeviceContext
+                    for m in torch.overrides._get_current_function_mode_stack()))
+
+
 def plain_call() -> bool:
     """Whether nothing is recording, transforming or tracing torch ops here.
     Compiling is asked first: Dynamo knows that answer, and cannot trace the rest."""
     return not (torch.compiler.is_compiling()
                 or torch.is_grad_enabled() or torch.is_autocast_enabled("cuda")
                 or torch.autograd.forward_ad._current_level >= 0
-                or torch._C._len_torch_dispatch_stack() > 0
+                or torch._C._len_torch_dispatch_stack() > 0 or _function_modes()
                 or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.jit.is_tracing())
 

@@ -144,3 +144,43 @@ def test_compiled_sublayers_keep_one_graph(dev):
             got, want = torch.compile(fn, fullgraph=True, backend="eager")(x), fn(x)
             # the compiled call's torch ops round intermediates that the kernels do not
             assert float((want.float() - got.float()).abs().max()) <= 6 * 2.0 ** -9 * float(want.float().abs().max())
+
+
+def test_plain_call_under_torch_function_modes():
+    """A mode that could observe or replace the ops is not a plain call; the default
+    device's own mode is one."""
+    from torch.overrides import TorchFunctionMode
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad():
+        with Mode():
+            assert not _ops.plain_call()
+            with torch.device("cpu"):
+                assert not _ops.plain_call()
+        with torch.device("cpu"):
+            assert _ops.plain_call()
+        assert _ops.plain_call()
+
+
+@pytest.mark.gpu
+def test_function_mode_sees_the_sublayers_ops(dev):
+    from torch.overrides import TorchFunctionMode
+    seen = set()
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.add(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    x = torch.randn(1, 4, 128, device=dev).to(BF)
+    pos = tuple(t.to(dev).to(BF) for t in precompute_freqs_cis(64, 4))
+    ff, moe, attn = (m.to(dev).to(BF).eval() for m in (FeedForward(_cfg()), MOEFeedForward(_cfg()), Attention(_cfg())))
+    for call, ops in ((lambda: ff(x), {"linear", "silu"}), (lambda: moe(x), {"linear", "silu", "topk"}),
+                      (lambda: attn(x, pos), {"linear", "rms_norm", "scaled_dot_product_attention"})):
+        seen.clear()
+        with torch.no_grad(), Mode():
+            call()
+        assert ops <= seen, (ops, seen)
