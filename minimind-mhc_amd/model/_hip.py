@@ -169,10 +169,15 @@ def require_device(*tensors: Optional[torch.Tensor]) -> torch.device:
     return dev
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # no public name
+
+
 def stream(dev: torch.device) -> int:
     """The current stream's handle.  torch.cuda.current_stream(dev).cuda_stream builds a
     Stream object for it: 2 us a launch."""
-    return torch._C._cuda_getCurrentRawStream(dev.index)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return _raw_stream(dev.index)
 
 
 def check(rc: int, fn: str) -> None:

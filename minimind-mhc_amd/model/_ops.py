@@ -13,9 +13,21 @@ import weakref
 from typing import Optional
 
 import torch
-from torch.utils._device import DeviceContext
 
 from . import _hip as H
+
+# What plain_call looks at has no public name.  On a torch where one is missing no call
+# counts as plain, and the torch ops run.
+try:
+    from torch._C import _len_torch_dispatch_stack, _len_torch_function_stack
+    from torch._C._functorch import peek_interpreter_stack
+    from torch.autograd import forward_ad
+    from torch.nn.modules.module import _global_forward_hooks, _global_forward_pre_hooks
+    from torch.overrides import _get_current_function_mode_stack
+    from torch.utils._device import DeviceContext
+    CAN_TELL = isinstance(forward_ad._current_level, int)
+except (ImportError, AttributeError):
+    CAN_TELL = False
 
 _GRAD = threading.local()
 
@@ -645,23 +657,19 @@ def _function_modes() -> bool:
     """Whether a torch-function mode could see or replace the torch ops.  The one that
     torch.set_default_device and `with torch.device(...)` leave on the stack only changes
     factory calls without a device, of which the sublayers make none."""
-    return (torch._C._len_torch_function_stack() > 0
-            and any(type(m) is not DeviceContext
-                    for m in torch.overrides._get_current_function_mode_stack()))
+    return (_len_torch_function_stack() > 0
+            and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
 
 
 def plain_call() -> bool:
     """Whether nothing is recording, transforming or tracing torch ops here.
     Compiling is asked first: Dynamo knows that answer, and cannot trace the rest."""
-    return not (torch.compiler.is_compiling()
+    return not (torch.compiler.is_compiling() or not CAN_TELL
                 or torch.is_grad_enabled() or torch.is_autocast_enabled("cuda")
-                or torch.autograd.forward_ad._current_level >= 0
-                or torch._C._len_torch_dispatch_stack() > 0 or _function_modes()
-                or torch._C._functorch.peek_interpreter_stack() is not None
+                or forward_ad._current_level >= 0
+                or _len_torch_dispatch_stack() > 0 or _function_modes()
+                or peek_interpreter_stack() is not None
                 or torch.jit.is_tracing())
-
-
-_GLOBAL_HOOKS = torch.nn.modules.module
 
 
 def plain_module(m: torch.nn.Module, kind: type) -> bool:
@@ -669,8 +677,7 @@ def plain_module(m: torch.nn.Module, kind: type) -> bool:
     on it or on all modules, no forward of its own."""
     return (type(m) is kind and "forward" not in m.__dict__
             and not (m._forward_hooks or m._forward_pre_hooks)
-            and not (_GLOBAL_HOOKS._global_forward_hooks
-                     or _GLOBAL_HOOKS._global_forward_pre_hooks))
+            and not (_global_forward_hooks or _global_forward_pre_hooks))
 
 
 def plain_tensors(dtype: torch.dtype, dev: torch.device, *ts) -> bool:

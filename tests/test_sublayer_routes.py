@@ -3,6 +3,9 @@ the HIP kernels: every other call has to reach the torch ops, as the layers' pla
 says it would."""
 from __future__ import annotations
 
+import importlib.util
+import types
+
 import pytest
 import torch
 from torch import nn
@@ -184,3 +187,32 @@ def test_function_mode_sees_the_sublayers_ops(dev):
         with torch.no_grad(), Mode():
             call()
         assert ops <= seen, (ops, seen)
+
+
+def _again(module):
+    """A second copy of a module of the package, imported now."""
+    spec = importlib.util.spec_from_file_location(module.__name__ + "_again", module.__file__)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+@pytest.mark.parametrize("owner,name", [
+    ("torch._C", "_len_torch_dispatch_stack"), ("torch._C", "_len_torch_function_stack"),
+    ("torch._C._functorch", "peek_interpreter_stack"),
+    ("torch.autograd.forward_ad", "_current_level"),
+    ("torch.nn.modules.module", "_global_forward_hooks"),
+    ("torch.overrides", "_get_current_function_mode_stack"),
+    ("torch.utils._device", "DeviceContext")])
+def test_no_call_is_plain_on_a_torch_without_a_name(monkeypatch, owner, name):
+    with torch.no_grad():
+        assert _again(_ops).plain_call()
+        monkeypatch.delattr(f"{owner}.{name}")
+        ops = _again(_ops)
+        assert not ops.plain_call()
+
+
+def test_stream_on_a_torch_without_the_raw_handle(monkeypatch):
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: types.SimpleNamespace(cuda_stream=77))
+    assert _again(_ops.H).stream(torch.device("cuda:0")) == 77
