@@ -273,7 +273,12 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
       kc[c] = *reinterpret_cast<const U32x4*>(&kl[buf][(wave * 16 + r) * LST + 32 * c + 8 * g]);
       vc[c] = *reinterpret_cast<const U32x4*>(&vl[buf][(wave * 16 + r) * LST + 32 * c + 8 * g]);
     }
-    step(kc, vc, t * rows + sub + r < a.S);
+    const bool ok = t * rows + sub + r < a.S;
+    if ((t + 1) * rows > a.S && !ok) {  // a row that is not there: 0 x infinity would be NaN
+#pragma unroll
+      for (int c = 0; c < NC; ++c) vc[c] = U32x4{};
+    }
+    step(kc, vc, ok);
   }
   if (has_new) {  // the new position: one row, in the lanes with r == 0
     U32x4 kc[NC], vc[NC];
@@ -281,7 +286,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
                                a.cos, a.sin, a.k_eps, g, kc);
     const uint16_t* vp = static_cast<const uint16_t*>(a.v) + (b * a.kv_heads + kvh) * HD + 8 * g;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) vc[c] = ld16(vp + 32 * c);
+    for (int c = 0; c < NC; ++c) vc[c] = r == 0 ? ld16(vp + 32 * c) : U32x4{};
     if (ko && r == 0) {
       const int64_t o = obase + a.S * orow + kvh * HD + 8 * g;
 #pragma unroll

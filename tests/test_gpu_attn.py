@@ -121,6 +121,32 @@ def test_decode_rising_scores(dev):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("hd,heads,kv,dtype,S", [
+    (96, 8, 4, F16, 1), (96, 8, 4, BF, 15), (64, 4, 2, F16, 37), (128, 3, 3, BF, 70),
+    (64, 4, 1, F16, 1000), (96, 8, 4, BF, 2001)])
+def test_decode_infinite_value(dev, hd, heads, kv, dtype, S):
+    """One infinite element of a V row (the newest position's, or the cache's last, whose
+    row the kernel also reads for the rows that are not there) makes its column infinite
+    and changes no other."""
+    m = _layer(hd, heads, kv, dtype).to(dev)
+    pos = tuple(t.to(dev) for t in _pos(hd, S, 1, dtype))
+    q, k, v = (torch.randn(2, 1, n * hd, device=dev).to(dtype) for n in (heads, kv, kv))
+    past = tuple(torch.randn(2, S, kv, hd, device=dev).to(dtype) for _ in range(2))
+    with torch.inference_mode():
+        want, _ = _ops.attn_decode(m, q, k, v, pos, past, False)
+        for cached in (False, True):
+            v2, pv = v.clone(), past[1].clone()
+            row = pv[1, S - 1, kv - 1] if cached else v2[1, 0].view(kv, hd)[kv - 1]
+            row[5] = float("inf")
+            got, _ = _ops.attn_decode(m, q, k, v2, pos, (past[0], pv), False)
+            hit = torch.zeros(2, heads, hd, dtype=torch.bool, device=dev)
+            hit[1, heads - heads // kv:, 5] = True
+            hit = hit.view(got.shape)
+            assert bool((got[hit] == float("inf")).all())
+            assert torch.equal(got[~hit], want[~hit]) and bool(torch.isfinite(want).all())
+
+
+@pytest.mark.gpu
 def test_calls_left_to_torch(dev):
     """Calls the kernels do not take, or that would tell: the route is None."""
     m = _layer(96, 8, 4, BF).to(dev)
