@@ -439,12 +439,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
       vr[p] = ld16(vg + row * rs + col);
     }
   };
-  auto stash = [&](int buf) {
+  auto stash = [&](int buf, int s0) {
 #pragma unroll
     for (int p = 0; p < PPT; ++p) {
       const int piece = p * 256 + tid;
       const int row = piece / (HD / 8);
       const int col = (piece % (HD / 8)) * 8;
+      if (s0 + KT > T && s0 + row >= T) vr[p] = U32x4{};  // no such row: 0 x infinity would be NaN
       *reinterpret_cast<U32x4*>(&ks[buf][row * KST + col]) = kr[p];
       *reinterpret_cast<U32x4*>(&vs[buf][row * VST + col]) = vr[p];
     }
@@ -470,7 +471,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
   const int nt = (last + KT - 1) / KT;
   for (int t = 0; t < nt; ++t) {
     const int buf = t & 1;
-    stash(buf);
+    stash(buf, t * KT);
     __syncthreads();
     if (t + 1 < nt) load((t + 1) * KT);
     const int s0 = t * KT;

@@ -147,6 +147,27 @@ def test_decode_infinite_value(dev, hd, heads, kv, dtype, S):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("hd,heads,kv,dtype,T", [
+    (96, 8, 4, F16, 1), (96, 8, 4, BF, 100), (64, 3, 1, F16, 129), (128, 4, 4, BF, 190), (64, 4, 2, F16, 64)])
+def test_prefill_infinite_value(dev, hd, heads, kv, dtype, T):
+    """One infinite element of the last position's V row makes the last row's column
+    infinite (rows that are not there are read as copies of it); the other columns, and
+    the rows of the tiles before, are as without it."""
+    m = _layer(hd, heads, kv, dtype).to(dev)
+    pos = tuple(t.to(dev) for t in _pos(hd, 0, T, dtype))
+    q, k, v = (torch.randn(2, T, n * hd, device=dev).to(dtype) for n in (heads, kv, kv))
+    with torch.inference_mode():
+        want = _ops.attn_prefill(m, q, k, v, pos)[0].view(2, T, heads, hd)
+        v2 = v.clone()
+        v2[1, T - 1].view(kv, hd)[kv - 1, 5] = float("inf")
+        got = _ops.attn_prefill(m, q, k, v2, pos)[0].view(2, T, heads, hd)
+    hit = torch.zeros_like(want, dtype=torch.bool)
+    hit[1, (T - 1) // 64 * 64:, heads - heads // kv:, 5] = True  # the tile that holds the position
+    assert bool((got[1, T - 1, heads - heads // kv:, 5] == float("inf")).all())
+    assert torch.equal(got[~hit], want[~hit]) and bool(torch.isfinite(want).all())
+
+
+@pytest.mark.gpu
 def test_calls_left_to_torch(dev):
     """Calls the kernels do not take, or that would tell: the route is None."""
     m = _layer(96, 8, 4, BF).to(dev)
