@@ -758,6 +758,7 @@ def glu(x: torch.Tensor, gate: torch.nn.Module, up: torch.nn.Module) -> Optional
 
 
 ATTN_HEAD_DIMS = (64, 96, 128)
+ATTN_MAX_ROWS = 1 << 20  # sequences x kv heads of a decode step; mhc_attn_decode_fwd refuses more
 
 
 def attn_route(m, q, k, v, position_embeddings, past) -> Optional[str]:
@@ -786,7 +787,8 @@ def attn_route(m, q, k, v, position_embeddings, past) -> Optional[str]:
     pk, pv = past[0], past[1]
     if (T != 1 or H_ // KV > 4 or not plain_tensors(q.dtype, q.device, pk, pv)
             or pk.dim() != 4 or pk.shape != pv.shape
-            or pk.shape[0] != B or pk.shape[1] < 1 or tuple(pk.shape[2:]) != (KV, hd)):
+            or pk.shape[0] != B or pk.shape[1] < 1 or tuple(pk.shape[2:]) != (KV, hd)
+            or B * KV > ATTN_MAX_ROWS):
         return None
     for t in (pk, pv):
         if t.stride(3) != 1 or any(s % 8 for s in t.stride()[:3]):

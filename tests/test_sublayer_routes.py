@@ -216,3 +216,16 @@ def test_stream_on_a_torch_without_the_raw_handle(monkeypatch):
     monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda d: types.SimpleNamespace(cuda_stream=77))
     assert _again(_ops.H).stream(torch.device("cuda:0")) == 77
+
+
+def test_decode_past_the_librarys_limit_is_torchs(monkeypatch):
+    """mhc_attn_decode_fwd takes up to 2^20 sequences x kv heads and raises past that."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(_ops, "plain_tensors", lambda *a: True)
+    attn = Attention(_cfg()).to(BF).eval()
+    pos = _fake((1, 64))
+    with torch.no_grad():
+        for B, want in ((1 << 20, "decode"), ((1 << 20) + 1, None)):
+            kv, past = _fake((B, 1, 64)), _fake((B, 7, 1, 64))
+            got = _ops.attn_route(attn, _fake((B, 1, 128)), kv, kv, (pos, pos), (past, past))
+            assert got == want, B
