@@ -229,3 +229,13 @@ def test_decode_past_the_librarys_limit_is_torchs(monkeypatch):
             kv, past = _fake((B, 1, 64)), _fake((B, 7, 1, 64))
             got = _ops.attn_route(attn, _fake((B, 1, 128)), kv, kv, (pos, pos), (past, past))
             assert got == want, B
+
+
+@pytest.mark.parametrize("n,taken", [(0, False), (2, False), (4, True)])
+def test_linear_widths(monkeypatch, n, taken):
+    """mhc_linear_fwd takes multiples of four output features, and none of zero."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(_ops, "plain_tensors", lambda *a: True)
+    lin = nn.utils.skip_init(nn.Linear, 128, n, bias=False).to(BF)
+    with torch.no_grad():
+        assert (_ops._linear_weights(_fake((4, 128)), (lin,)) is not None) == taken
