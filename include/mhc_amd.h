@@ -507,7 +507,7 @@ int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void*
  */
 
 /* Bytes of workspace mhc_moe_fwd needs, or -1 for a shape it does not take:
- * hidden and inter multiples of 32, 1 <= topk <= 8, topk <= experts <= 32,
+ * hidden and inter multiples of 32 up to 2^22, 1 <= topk <= 8, topk <= experts <= 32,
  * M <= 262144, x of at most 4 GiB. */
 int64_t mhc_moe_workspace_bytes(int64_t M, int hidden, int inter, int experts, int topk);
 

@@ -38,6 +38,9 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 constexpr int kMaxN = 16;
 constexpr int64_t kMaxBlocks = 0x7fffffff;
+// Columns of a product's inputs: a tile forms the byte offsets of its up to 256 rows of
+// 2 K bytes in 32 bits.
+constexpr int kMaxProductK = 1 << 22;
 
 // Shared checks for the three pre-phase style entry points.
 int check_pre(const mhc::PreArgs& a, const char* fn) {
@@ -734,6 +737,7 @@ int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void*
 int64_t mhc_moe_workspace_bytes(int64_t M, int hidden, int inter, int experts, int topk) {
   if (M < 0 || M > 262144 || hidden < 32 || hidden % 32 != 0 || inter < 32 || inter % 32 != 0) return -1;
   if (M * hidden > (int64_t)1 << 31) return -1;  // x rows are 32-bit byte offsets apart
+  if (hidden > kMaxProductK || inter > kMaxProductK) return -1;
   if (experts < 1 || experts > mhc::kMoeMaxExperts || topk < 1 || topk > mhc::kMoeMaxTopk || topk > experts) return -1;
   mhc::MoeArgs a{};
   a.M = M; a.hidden = hidden; a.inter = inter; a.experts = experts; a.topk = topk;
@@ -770,7 +774,8 @@ int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
 // -------------------------------------------------- linear layers (inference)
 
 static int run_linear(mhc::LinearArgs& a, int dtype, hipStream_t stream, const char* fn) {
-  if (a.M < 0 || a.K < 32 || a.K % 32 != 0) return fail(hipErrorInvalidValue, "%s: bad shape (M=%lld K=%d)", fn, (long long)a.M, a.K);
+  if (a.M < 0 || a.K < 32 || a.K % 32 != 0 || a.K > kMaxProductK)
+    return fail(hipErrorInvalidValue, "%s: bad shape (M=%lld K=%d)", fn, (long long)a.M, a.K);
   if (dtype != mhc::kBF16 && dtype != mhc::kF16) return fail(hipErrorInvalidValue, "%s: dtype must be bf16 or fp16 (got %d)", fn, dtype);
   int64_t cols = 0;
   for (int i = 0; i < a.count; ++i) {

@@ -142,6 +142,19 @@ def test_sums_of_squares_argument_checks(lib):
     assert rc == 1 and b"out_ssq" in lib.mhc_last_error()
 
 
+def test_product_widths_are_limited(lib):
+    """A tile forms its rows' byte offsets in 32 bits, which holds for K up to 2^22; an
+    empty call (M = 0) is refused too, so this needs no device."""
+    p = ctypes.c_void_p(256)
+    ptrs, n = (ctypes.c_void_p * 1)(256), (ctypes.c_int * 1)(64)
+    for K, rc in ((1 << 22, 0), ((1 << 22) + 32, 1)):
+        assert lib.mhc_linear_fwd(p, ptrs, ptrs, n, 1, 0, K, 1, None) == rc, K
+        assert lib.mhc_glu_fwd(p, p, p, p, 0, K, 64, 1, None) == rc, K
+        for hidden, inter in ((K, 64), (64, K)):
+            assert (lib.mhc_moe_workspace_bytes(1, hidden, inter, 4, 1) < 0) == bool(rc), (hidden, inter)
+            assert lib.mhc_moe_fwd(p, p, ptrs, ptrs, ptrs, p, None, p, 0, 0, hidden, inter, 4, 1, 1, 1, None) == rc
+
+
 def test_row_staging_round_trip(lib):
     old = lib.mhc_pre_row_staging(-1)
     assert old in (0, 1)
