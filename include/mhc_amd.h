@@ -483,7 +483,7 @@ int mhc_attn_prefill_fwd(const void* q, const void* k, const void* v, const void
                          int dtype, float q_eps, float k_eps, hipStream_t stream);
 
 /* Bytes of workspace mhc_attn_decode_fwd needs (0: none), or -1 for a shape it
- * does not take (heads / kv_heads > 4, another head_dim, S < 1). */
+ * does not take (heads / kv_heads > 4, another head_dim, S < 1 or > 2^30). */
 int64_t mhc_attn_decode_workspace_bytes(int64_t B, int S, int heads, int kv_heads, int head_dim);
 
 /* One decode step.  q, k, v: the raw projections of one new token per sequence

@@ -692,6 +692,7 @@ int mhc_attn_prefill_fwd(const void* q, const void* k, const void* v, const void
 int64_t mhc_attn_decode_workspace_bytes(int64_t B, int S, int heads, int kv_heads, int head_dim) {
   if (B < 0 || S < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || heads / kv_heads > 4) return -1;
   if (head_dim != 64 && head_dim != 96 && head_dim != 128) return -1;
+  if (S > 1 << 30) return -1;  // the plan rounds S up to tiles in 32 bits
   if (B == 0) return 0;
   mhc::AttnDecodeArgs a{};
   a.B = B; a.S = S; a.kv_heads = kv_heads;
@@ -709,8 +710,8 @@ int mhc_attn_decode_fwd(const void* q, const void* k, const void* v, const void*
   const char* fn = "mhc_attn_decode_fwd";
   if (int rc = check_attn(B, heads, kv_heads, head_dim, dtype, fn)) return rc;
   const int64_t need = mhc_attn_decode_workspace_bytes(B, S, heads, kv_heads, head_dim);
-  if (need < 0) return fail(hipErrorInvalidValue, "%s: needs S >= 1 and heads / kv_heads <= 4 (S=%d heads=%d kv_heads=%d)", fn, S, heads, kv_heads);
-  if (S > (1 << 30) || B * kv_heads > (1 << 20)) return fail(hipErrorInvalidValue, "%s: too large", fn);
+  if (need < 0) return fail(hipErrorInvalidValue, "%s: needs 1 <= S <= 2^30 and heads / kv_heads <= 4 (S=%d heads=%d kv_heads=%d)", fn, S, heads, kv_heads);
+  if (B * kv_heads > (1 << 20)) return fail(hipErrorInvalidValue, "%s: too large", fn);
   if (B == 0) return 0;
   for (const void* p : {q, k, v, q_gain, k_gain, cos, sin, k_past, v_past, (const void*)out})
     if (!p || !aligned16(p)) return fail(hipErrorInvalidValue, "%s: null or unaligned pointer", fn);

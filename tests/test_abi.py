@@ -155,6 +155,12 @@ def test_product_widths_are_limited(lib):
             assert lib.mhc_moe_fwd(p, p, ptrs, ptrs, ptrs, p, None, p, 0, 0, hidden, inter, 4, 1, 1, 1, None) == rc
 
 
+def test_decode_workspace_limits(lib):
+    """S is rounded up to tiles in 32 bits: past 2^30 the shape is refused, not planned."""
+    for S, ok in ((0, False), (1, True), (1 << 30, True), ((1 << 30) + 1, False), ((1 << 31) - 1, False)):
+        assert (lib.mhc_attn_decode_workspace_bytes(1, S, 8, 4, 96) >= 0) == ok, S
+
+
 def test_row_staging_round_trip(lib):
     old = lib.mhc_pre_row_staging(-1)
     assert old in (0, 1)
