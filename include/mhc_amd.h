@@ -525,7 +525,8 @@ int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
 
 /* -------------------------------- linear layers of the sublayers (inference)
  * 16-bit tensors (bf16 or fp16) of one dtype, fp32 sums rounded once; K a
- * multiple of 32 up to 2^22, every weight's row count of 4; pointers 16-byte aligned.
+ * multiple of 32 up to 2^22, every weight's row count of 4 up to 2^30; pointers 16-byte
+ * aligned.
  */
 
 /* out[i] [M, n[i]] = x [M, K] w[i]^T for `count` (one to three) weights

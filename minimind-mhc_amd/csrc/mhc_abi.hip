@@ -780,7 +780,7 @@ static int run_linear(mhc::LinearArgs& a, int dtype, hipStream_t stream, const c
   if (dtype != mhc::kBF16 && dtype != mhc::kF16) return fail(hipErrorInvalidValue, "%s: dtype must be bf16 or fp16 (got %d)", fn, dtype);
   int64_t cols = 0;
   for (int i = 0; i < a.count; ++i) {
-    if (a.n[i] < 4 || a.n[i] % 4 != 0) return fail(hipErrorInvalidValue, "%s: weight %d has %d rows", fn, i, a.n[i]);
+    if (a.n[i] < 4 || a.n[i] % 4 != 0 || a.n[i] > 1 << 30) return fail(hipErrorInvalidValue, "%s: weight %d has %d rows", fn, i, a.n[i]);
     cols += a.n[i];
   }
   if ((a.M / 64 + 1) * (cols / 32 + 3) > kMaxBlocks) return fail(hipErrorInvalidValue, "%s: too large", fn);

@@ -710,7 +710,7 @@ def _linear_weights(x: torch.Tensor, mods):
         if not plain_module(m, torch.nn.Linear) or m.bias is not None:
             return None
         w = m.weight
-        if w.dim() != 2 or w.shape[1] != K or w.shape[0] < 4 or w.shape[0] % 4 != 0 or not w.is_contiguous():
+        if w.dim() != 2 or w.shape[1] != K or not 4 <= w.shape[0] <= 1 << 30 or w.shape[0] % 4 != 0 or not w.is_contiguous():
             return None
         ws.append(w)
     return ws if plain_tensors(x.dtype, x.device, x, *ws) else None

@@ -155,6 +155,14 @@ def test_product_widths_are_limited(lib):
             assert lib.mhc_moe_fwd(p, p, ptrs, ptrs, ptrs, p, None, p, 0, 0, hidden, inter, 4, 1, 1, 1, None) == rc
 
 
+def test_output_widths_are_limited(lib):
+    """A weight's rows are rounded up to tiles in 32 bits; an empty call needs no device."""
+    p, ptrs = ctypes.c_void_p(256), (ctypes.c_void_p * 1)(256)
+    for n, rc in ((1 << 30, 0), ((1 << 30) + 4, 1), ((1 << 31) - 4, 1), (2, 1), (0, 1)):
+        assert lib.mhc_linear_fwd(p, ptrs, ptrs, (ctypes.c_int * 1)(n), 1, 0, 64, 1, None) == rc, n
+        assert lib.mhc_glu_fwd(p, p, p, p, 0, 64, n, 1, None) == rc, n
+
+
 def test_decode_workspace_limits(lib):
     """S is rounded up to tiles in 32 bits: past 2^30 the shape is refused, not planned."""
     for S, ok in ((0, False), (1, True), (1 << 30, True), ((1 << 30) + 1, False), ((1 << 31) - 1, False)):
