@@ -245,14 +245,15 @@ class MHCConnection_Fused(nn.Module):
             out = _ops.post(x_flat, o["h_res"], o["h_post"], f_out, self.n, self.dim,
                             ssq_out=ssq_out).view(B, L, NC)
             return chain.put(out, ssq_out) if chain is not None else out
-        grad = torch.is_grad_enabled()
+        # x's two gradients meet in the pre phase's backward; where x has none there is no sum
+        pass_x = torch.is_grad_enabled() and x_flat.requires_grad
         sublayer_in, h_post, h_res, *passed = _PreSinkhornFn.apply(
             x_flat, self.phi_weight, packed,
             self.alpha_pre, self.bias_pre, self.alpha_post, self.bias_post,
             self.alpha_res, self.bias_res,
             self.post_mult_value, self.pre_eps, self.eps, self.n, self.dim,
-            self.sinkhorn_iters, self.sinkhorn_eps, ssq, grad)
+            self.sinkhorn_iters, self.sinkhorn_eps, ssq, pass_x)
         f_out = sublayer_fn(sublayer_in)
-        out = _PostPhaseFullFn.apply(passed[0] if grad else x_flat, h_res, h_post, f_out, self.n,
+        out = _PostPhaseFullFn.apply(passed[0] if pass_x else x_flat, h_res, h_post, f_out, self.n,
                                      self.dim, ssq_out)
         return chain.put(out, ssq_out) if chain is not None else out

@@ -135,12 +135,13 @@ class MHCConnection_FusedNoHres(nn.Module):
             out = _ops.post(x_flat, None, o["h_post"], f_out, self.n, self.dim,
                             ssq_out=ssq_out).view(B, L, NC)
             return chain.put(out, ssq_out) if chain is not None else out
-        grad = torch.is_grad_enabled()
+        # x's two gradients meet in the pre phase's backward; where x has none there is no sum
+        pass_x = torch.is_grad_enabled() and x_flat.requires_grad
         sublayer_in, _h_pre, h_post, *passed = _PrePhaseFn.apply(
             x_flat, self.phi_weight, self.alpha_pre, self.bias_pre,
             self.alpha_post, self.bias_post,
             self.post_mult_value, self.pre_eps, self.eps, self.n, self.dim, packed, ssq,
-            grad)
+            pass_x)
         f_out = sublayer_fn(sublayer_in)
-        out = _PostPhaseFn.apply(passed[0] if grad else x_flat, h_post, f_out, self.n, self.dim, ssq_out)
+        out = _PostPhaseFn.apply(passed[0] if pass_x else x_flat, h_post, f_out, self.n, self.dim, ssq_out)
         return chain.put(out, ssq_out) if chain is not None else out

@@ -108,3 +108,20 @@ def test_hooks_and_saved_tensor_hooks(dev):
     assert len(seen) == 1 and torch.equal(seen[0], x.grad)
     want, = torch.autograd.grad(_apart(m, x, torch.tanh).float().sum(), x)
     assert torch.equal(x.grad, want)
+
+
+@pytest.mark.parametrize("kind", ["full", "nohres"])
+def test_no_sum_for_a_stream_without_a_gradient(dev, kind, monkeypatch):
+    """A stream that needs no gradient has none to add: the launch reads one stream less."""
+    m = _module(kind, 4, 64, BF, dev)
+    x = torch.randn(1, 6, 256, device=dev).to(BF)
+    added, pre_bwd = [], _ops.pre_bwd
+
+    def spy(*args, g_x_in=None, **kwargs):
+        added.append(g_x_in is not None)
+        return pre_bwd(*args, g_x_in=g_x_in, **kwargs)
+
+    monkeypatch.setattr(_ops, "pre_bwd", spy)
+    for xx in (x, x.clone().requires_grad_()):
+        m(xx, torch.tanh).float().sum().backward()
+    assert added == [False, True]
