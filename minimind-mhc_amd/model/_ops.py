@@ -554,6 +554,8 @@ def pre_bwd(x2, phi, alphas, biases, inv_rms, mixes, n, C, mode, post_mult, pre_
     if g_x_in is not None:
         H.require_device(x2, g_x_in)
         g_x_in = g_x_in.to(x2.dtype).reshape(x2.shape).contiguous()
+        if g_x_in.data_ptr() % 16:  # a caller's view; the MFMA kernels load 16 bytes
+            g_x_in = g_x_in.clone()
     g_x = torch.empty_like(x2)
     if mode == H.MODE_RMS:
         phi_p = phi_dt = None

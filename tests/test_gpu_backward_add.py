@@ -125,3 +125,17 @@ def test_no_sum_for_a_stream_without_a_gradient(dev, kind, monkeypatch):
     for xx in (x, x.clone().requires_grad_()):
         m(xx, torch.tanh).float().sum().backward()
     assert added == [False, True]
+
+
+@pytest.mark.parametrize("kind,n,C,dt", [("nohres", 4, 64, BF), ("nohres", 2, 96, F32), ("full", 4, 64, BF)])
+def test_gradient_off_16_byte_alignment(dev, kind, n, C, dt):
+    """A gradient that arrives at an odd offset (without a residual matrix it is the one
+    that the pre phase adds, as it came) leaves the pre phase on its MFMA kernel."""
+    m = _module(kind, n, C, dt, dev)
+    x = torch.randn(2, 9, n * C, device=dev).to(dt).requires_grad_()
+    buf = torch.randn(x.numel() + 1, device=dev).to(dt)
+    g = buf[1:].view(x.shape)
+    assert g.data_ptr() % 16 and g.is_contiguous()
+    low = (lambda z: z.to(BF)) if dt == F32 else torch.tanh
+    for got, want in zip(_grads(m, m(x, low), x, g), _grads(m, _apart(m, x, low), x, g)):
+        assert torch.equal(got, want)
