@@ -538,6 +538,10 @@ int mhc_linear_fwd(const void* x, const void* const* w, void* const* out, const 
 int mhc_glu_fwd(const void* x, const void* gate_w, const void* up_w, void* out, int64_t M, int K,
                 int N, int dtype, hipStream_t stream);
 
+/* 1 where mhc_linear_fwd (glu: mhc_glu_fwd, whose two weights n then holds) is no
+ * slower than library products of these sizes, 0 where it is or takes them not. */
+int mhc_linear_pays(const int* n, int count, int64_t M, int K, int glu);
+
 #ifdef __cplusplus
 }
 #endif

@@ -774,16 +774,21 @@ int mhc_moe_fwd(const void* x, const void* probs, const void* const* gate_w,
 
 // -------------------------------------------------- linear layers (inference)
 
-static int run_linear(mhc::LinearArgs& a, int dtype, hipStream_t stream, const char* fn) {
+static int check_linear(const mhc::LinearArgs& a, const char* fn) {
   if (a.M < 0 || a.K < 32 || a.K % 32 != 0 || a.K > kMaxProductK)
     return fail(hipErrorInvalidValue, "%s: bad shape (M=%lld K=%d)", fn, (long long)a.M, a.K);
-  if (dtype != mhc::kBF16 && dtype != mhc::kF16) return fail(hipErrorInvalidValue, "%s: dtype must be bf16 or fp16 (got %d)", fn, dtype);
   int64_t cols = 0;
   for (int i = 0; i < a.count; ++i) {
     if (a.n[i] < 4 || a.n[i] % 4 != 0 || a.n[i] > 1 << 30) return fail(hipErrorInvalidValue, "%s: weight %d has %d rows", fn, i, a.n[i]);
     cols += a.n[i];
   }
   if ((a.M / 64 + 1) * (cols / 32 + 3) > kMaxBlocks) return fail(hipErrorInvalidValue, "%s: too large", fn);
+  return 0;
+}
+
+static int run_linear(mhc::LinearArgs& a, int dtype, hipStream_t stream, const char* fn) {
+  if (int rc = check_linear(a, fn)) return rc;
+  if (dtype != mhc::kBF16 && dtype != mhc::kF16) return fail(hipErrorInvalidValue, "%s: dtype must be bf16 or fp16 (got %d)", fn, dtype);
   if (a.M == 0) return 0;
   for (int i = 0; i < a.count; ++i)
     if (!a.w[i] || !aligned16(a.w[i]) || (!(a.glu && i == 1) && (!a.out[i] || !aligned16(a.out[i]))))
@@ -811,6 +816,14 @@ int mhc_glu_fwd(const void* x, const void* gate_w, const void* up_w, void* out, 
   a.x = x; a.w[0] = gate_w; a.w[1] = up_w; a.out[0] = out;
   a.n[0] = a.n[1] = N; a.count = 2; a.M = M; a.K = K; a.glu = true;
   return run_linear(a, dtype, stream, "mhc_glu_fwd");
+}
+
+int mhc_linear_pays(const int* n, int count, int64_t M, int K, int glu) {
+  if (count < 1 || count > 3 || !n || (glu && (count != 2 || n[0] != n[1]))) return 0;
+  mhc::LinearArgs a{};
+  for (int i = 0; i < count; ++i) a.n[i] = n[i];
+  a.count = count; a.M = M; a.K = K; a.glu = glu != 0;
+  return check_linear(a, "mhc_linear_pays") == 0 && M > 0 && mhc::linear_pays(a);
 }
 
 }  // extern "C"

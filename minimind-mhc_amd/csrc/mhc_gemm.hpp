@@ -143,7 +143,7 @@ __device__ __forceinline__ float silu_mul(float z, float u) {
 //     up of 1024 x 2048 (256) 12.0 and 13.3; of 2048 x 2048 (512) 22.6 and 17.4.
 //   64 x 64 while 128 x 64 ones would be fewer than 192: 1024 x 1536 (192) 7.5 us
 //     either way, 512 x 6400 (400) 17.9 and 11.9.
-enum class Tile { k64x64, k128x64, k128x128, k128x192, k256x256 };
+enum class Tile { k16x16, k64x64, k128x64, k128x128, k128x192, k256x256 };  // 16 x 16: linear layers only
 template <typename Rows, typename Cols>
 Tile pick_tile(Rows rows, Cols cols, bool glu) {
   const int64_t cus = device_cus();

@@ -335,5 +335,7 @@ struct LinearArgs {
   bool glu, f16;
 };
 hipError_t launch_linear(const LinearArgs& a, hipStream_t s);
+// Whether that is no slower than the library's products (and elementwise passes).
+bool linear_pays(const LinearArgs& a);
 
 }  // namespace mhc

@@ -137,33 +137,94 @@ hipError_t launch_tiles(const LinearArgs& a, int64_t work, int col_tiles, hipStr
 // slices and stores from the accumulators, the three library products 39.0), GLU 2048
 // columns 52.1 us (990 TFLOP/s; 64.2 before, two library products, silu and the
 // multiplication 83.3).
-template <bool F16, bool GLU>
-hipError_t launch(const LinearArgs& a, hipStream_t s) {
+struct Choice {
+  Tile tile;
+  int64_t work;   // tiles
+  int col_tiles;
+};
+Choice choose(const LinearArgs& a) {
   auto tiles = [&](int width) {
     int t = 0;
-    for (int i = 0; i < (GLU ? 1 : a.count); ++i) t += (a.n[i] + width - 1) / width;
+    for (int i = 0; i < (a.glu ? 1 : a.count); ++i) t += (a.n[i] + width - 1) / width;
     return t;
   };
   auto rows = [&](int height) { return (a.M + height - 1) / height; };
-  if (tiles(16) * rows(16) <= 448) {
-    const dim3 grid((unsigned)tiles(16), (unsigned)rows(16));
-    if (a.K >= 1536) skinny_kernel<F16, 16, GLU><<<grid, 16 * 64, 0, s>>>(a);
-    else skinny_kernel<F16, 8, GLU><<<grid, 8 * 64, 0, s>>>(a);
-    return hipGetLastError();
+  if (tiles(16) * rows(16) <= 448) return {Tile::k16x16, tiles(16) * rows(16), tiles(16)};
+  auto cols = [&](int width) { return tiles(a.glu ? width / 2 : width); };  // GLU: half gate, half up
+  const Tile t = pick_tile(rows, cols, a.glu);
+  switch (t) {
+    case Tile::k256x256: return {t, rows(256) * cols(256), cols(256)};
+    case Tile::k128x192: return {t, rows(128) * cols(192), cols(192)};
+    case Tile::k128x128: return {t, rows(128) * cols(128), cols(128)};
+    case Tile::k128x64: return {t, rows(128) * cols(64), cols(64)};
+    default: return {t, rows(64) * cols(64), cols(64)};
   }
-  auto cols = [&](int width) { return tiles(GLU ? width / 2 : width); };  // GLU: half gate, half up
-  switch (pick_tile(rows, cols, GLU)) {
-    case Tile::k256x256: return launch_tiles<F16, GLU, GemmTile<256, 256, 4, 2, 2>>(a, rows(256) * cols(256), cols(256), s);
+}
+
+template <bool F16, bool GLU>
+hipError_t launch(const LinearArgs& a, hipStream_t s) {
+  const Choice c = choose(a);
+  switch (c.tile) {
+    case Tile::k16x16: {
+      const dim3 grid((unsigned)c.col_tiles, (unsigned)((a.M + 15) / 16));
+      if (a.K >= 1536) skinny_kernel<F16, 16, GLU><<<grid, 16 * 64, 0, s>>>(a);
+      else skinny_kernel<F16, 8, GLU><<<grid, 8 * 64, 0, s>>>(a);
+      return hipGetLastError();
+    }
+    case Tile::k256x256: return launch_tiles<F16, GLU, GemmTile<256, 256, 4, 2, 2>>(a, c.work, c.col_tiles, s);
     case Tile::k128x192:
-      if constexpr (!GLU) return launch_tiles<F16, GLU, GemmTile<128, 192, 4, 2, 2>>(a, rows(128) * cols(192), cols(192), s);
+      if constexpr (!GLU) return launch_tiles<F16, GLU, GemmTile<128, 192, 4, 2, 2>>(a, c.work, c.col_tiles, s);
       [[fallthrough]];
-    case Tile::k128x128: return launch_tiles<F16, GLU, GemmTile<128, 128, 4, 2, 2>>(a, rows(128) * cols(128), cols(128), s);
-    case Tile::k128x64: return launch_tiles<F16, GLU, GemmTile<128, 64, 4, 1, 2>>(a, rows(128) * cols(64), cols(64), s);
-    default: return launch_tiles<F16, GLU, GemmTile<64, 64, 2, 2, 4>>(a, rows(64) * cols(64), cols(64), s);
+    case Tile::k128x128: return launch_tiles<F16, GLU, GemmTile<128, 128, 4, 2, 2>>(a, c.work, c.col_tiles, s);
+    case Tile::k128x64: return launch_tiles<F16, GLU, GemmTile<128, 64, 4, 1, 2>>(a, c.work, c.col_tiles, s);
+    default: return launch_tiles<F16, GLU, GemmTile<64, 64, 2, 2, 4>>(a, c.work, c.col_tiles, s);
   }
 }
 
 }  // namespace
+
+// Where the kernels are no slower than the library's (torch 2.10; GPU times of graph
+// replays over 1907, 202 and 480 sizes, M 1 to 65536, K 256 to 8192; a round fills the
+// chip: two workgroups a CU, one of the 256 x 256 tiles).  The kernels keep K in one
+// workgroup, so a long K makes a long tile; the library's own splits it.
+//   One layer: a kernel's gain is the host's (a call costs 11 us, the library's 20), so
+//     it pays while the host bounds the call: kernels of up to some 13 us.  16 x 16 tiles
+//     to K = 6464 in one tile a CU (M x K x N: 64 x 3264 x 1024 7.9 us against the library's
+//     10.6, 64 x 6464 x 1024 13.2 and 16.4, 128 x 4096 x 64 8.9 and 7.6), 2560 past that
+//     (128 x 2048 x 768 9.1 and 6.0, 128 x 4096 x 768 16.0 and 7.4), 64 x 64 ones to 2048 in one
+//     a CU (512 x 2048 x 2048 12.7 and 10.8), to 1024 past that (512 x 1536 x 2432 15.8 and
+//     11.7), 128 x 64 to K = 768 (512 x 768 x 6400 11.9 and 10.6; at 1024 half the sizes are
+//     9% slower or more, up to 15.0).  Larger tiles pay where they win by themselves:
+//     128 x 128 to K = 512 in one round (8192 x 512 x 1024 12.9 and 15.0; two rounds, 2048 x
+//     512 x 6400, 24.1 and 20.1), 128 x 192 to K = 1024 (8192 x 768 x 768 14.1 and 14.9,
+//     8192 x 1024 x 768 16.8 and 17.9, 12000 x 1536 x 768 32.8 and 28.7).  256 x 256 ones
+//     mostly lose (4096 x 768 x 6400 50 and 42).
+//   q, k, v: two launches less.  128 x 128 and 128 x 192 tiles while rounds x K is up to
+//     4096 (2048 rows, hidden 2048, 30.7 and 42.4; 12000 rows 157 and 141; 2930 x 7488 at K
+//     = 3296, two rounds, 186 and 180), 256 x 256 up to 2560
+//     (16384 rows, hidden 768, 49.1 and 54.4; 65536 rows 187 and 167; 16384 x 3072 at K =
+//     1024, three rounds, 7% slower), the rest to K = 4096 (never slower).
+//   Gate and up: also two passes less.  128 x 128 to K = 1536 (1 to 170% faster, 5400 rows
+//     of 4864 or more columns 3% slower), past that by the same rounds x K (2048 columns,
+//     two rounds 5% faster, three 6% slower); the rest to K = 3072 (2% faster and more).
+bool linear_pays(const LinearArgs& a) {
+  const Choice c = choose(a);
+  const int64_t cus = device_cus(), chip = c.tile == Tile::k256x256 ? cus : 2 * cus;
+  const int64_t rounds = (c.work + chip - 1) / chip;
+  if (a.glu) return c.tile == Tile::k128x128 && a.K > 1536 ? rounds * a.K <= 4096 : a.K <= 3072;
+  if (a.count > 1) {
+    if (c.tile == Tile::k128x128 || c.tile == Tile::k128x192) return rounds * a.K <= 4096;
+    return c.tile == Tile::k256x256 ? rounds * a.K <= 2560 : a.K <= 4096;
+  }
+  switch (c.tile) {
+    case Tile::k16x16: return a.K <= (c.work <= cus ? 6464 : 2560);
+    case Tile::k64x64: return a.K <= (c.work <= cus ? 2048 : 1024);
+    case Tile::k128x64: return a.K <= 768;
+    case Tile::k128x128: return a.K <= 512 && rounds == 1;
+    case Tile::k128x192: return a.K <= 1024;
+    default: return false;
+  }
+}
 
 hipError_t launch_linear(const LinearArgs& a, hipStream_t s) {
   if (a.glu) return a.f16 ? launch<true, true>(a, s) : launch<false, true>(a, s);

@@ -99,6 +99,7 @@ _SIGNATURES = {
     "mhc_sinkhorn_bwd_max_iters": (_I, [_I]),
     "mhc_linear_fwd": (_I, [_P, _P, _P, _P, _I, _I64, _I, _I, _P]),
     "mhc_glu_fwd": (_I, [_P, _P, _P, _P, _I64, _I, _I, _I, _P]),
+    "mhc_linear_pays": (_I, [_P, _I, _I64, _I, _I]),
     "mhc_moe_workspace_bytes": (_I64, [_I64, _I, _I, _I, _I]),
     "mhc_moe_fwd": (_I, [_P, _P, _P, _P, _P, _P, _P,      # x, probs, gate_w, up_w, down_w, out, zero
                          _P, _I64, _I64, _I, _I, _I, _I, _I, _I, _P]),

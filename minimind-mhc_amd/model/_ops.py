@@ -8,6 +8,7 @@ current stream.  Inputs are made contiguous, as the reference's Functions do
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 import weakref
 from typing import Optional
@@ -689,23 +690,38 @@ def plain_tensors(dtype: torch.dtype, dev: torch.device, *ts) -> bool:
                and t.device == dev and t.data_ptr() % 16 == 0 for t in ts)
 
 
-# Multiply-adds up to which one linear layer runs on mhc_linear_fwd.  The library's
-# call costs the host 19 us (MI355X, torch 2.10), the kernel's 7, and up to here the
-# kernel is as fast: 8192 rows, 768 x 768: 14.6 against 15.5 us; 2048 x 768: 30.1
-# against 30.5; 512 rows, 768 x 6400: 11.9 against 11.1.  Past it the library's kernel
-# is the faster one (8192 rows, 768 x 6400: 86 against 97 us).
+# Multiply-adds past which one linear layer is the library's at every K.
 LINEAR_MAX_MACS = 13_000_000_000
 
 
-def _linear_weights(x: torch.Tensor, mods):
-    """The weights of bias-free nn.Linear layers the kernels can apply to x, or None."""
+@functools.lru_cache(maxsize=4096)
+def _linear_pays(M: int, K: int, ns: tuple, glu: bool = False) -> bool:
+    """Whether the kernels are no slower than the library for these sizes."""
+    if M * K * sum(ns) >= 1 << 62 or max(M, K, *ns) >= 1 << 31:
+        return False
+    return bool(H.load().mhc_linear_pays((ctypes.c_int * len(ns))(*ns), len(ns), M, K, int(glu)))
+
+
+def _linear_weights(x: torch.Tensor, mods, glu: bool = False, closely: bool = True):
+    """The weights of bias-free nn.Linear layers the kernels can apply to x, or None; also
+    None where the library is faster (not closely: where it is at every K).  That is asked
+    before what takes longer to look at: a call left to torch waits for this."""
     if not isinstance(x, torch.Tensor):  # an fx Proxy: the torch ops are traced
         return None
-    if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or not plain_call()
-            or not on_current_device(x) or x.dim() < 2 or x.numel() == 0 or not x.is_contiguous()):
+    if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or not plain_call():
+        return None
+    total = x.numel()
+    if x.dim() < 2 or total == 0:
         return None
     K = x.shape[-1]
     if K % 32 != 0 or K > 1 << 22:
+        return None
+    ns = tuple([getattr(m, "out_features", None) for m in mods])
+    if None in ns:
+        return None
+    if not (_linear_pays(total // K, K, ns, glu) if closely else total * ns[0] <= LINEAR_MAX_MACS):
+        return None
+    if not on_current_device(x) or not x.is_contiguous():
         return None
     ws = []
     for m in mods:
@@ -718,37 +734,36 @@ def _linear_weights(x: torch.Tensor, mods):
     return ws if plain_tensors(x.dtype, x.device, x, *ws) else None
 
 
-def linears(x: torch.Tensor, *mods):
-    """[m(x) for m in mods] for one to three bias-free nn.Linear layers in one
-    launch, or None for a call the kernels do not take (or, for a single layer,
-    one that is faster in the library)."""
-    ws = _linear_weights(x, mods)
-    if ws is None:
-        return None
-    K = x.shape[-1]
-    M = x.numel() // K
-    if len(ws) == 1 and M * K * ws[0].shape[0] > LINEAR_MAX_MACS:
-        return None
-    n = len(ws)
+def _launch_linears(x: torch.Tensor, ws):
+    K, n = x.shape[-1], len(ws)
     outs = [x.new_empty(*x.shape[:-1], w.shape[0]) for w in ws]
     H.check(H.load().mhc_linear_fwd(
         x.data_ptr(), (ctypes.c_void_p * n)(*[w.data_ptr() for w in ws]),
         (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs]),
-        (ctypes.c_int * n)(*[w.shape[0] for w in ws]), n, M, K, H.dtype_tag(x),
+        (ctypes.c_int * n)(*[w.shape[0] for w in ws]), n, x.numel() // K, K, H.dtype_tag(x),
         H.stream(x.device)), "mhc_linear_fwd")
     return outs
 
 
+def linears(x: torch.Tensor, *mods):
+    """[m(x) for m in mods] for one to three bias-free nn.Linear layers in one
+    launch, or None for a call the kernels do not take or that is faster in the
+    library (`linear` looks closer at a single layer)."""
+    ws = _linear_weights(x, mods, closely=len(mods) > 1)
+    return None if ws is None else _launch_linears(x, ws)
+
+
 def linear(x: torch.Tensor, m: torch.nn.Module) -> torch.Tensor:
-    """m(x), on mhc_linear_fwd where `linears` takes it."""
-    out = linears(x, m)
-    return m(x) if out is None else out[0]
+    """m(x), on mhc_linear_fwd for a call that it takes and that is not faster in the
+    library."""
+    ws = _linear_weights(x, (m,))
+    return m(x) if ws is None else _launch_linears(x, ws)[0]
 
 
 def glu(x: torch.Tensor, gate: torch.nn.Module, up: torch.nn.Module) -> Optional[torch.Tensor]:
     """silu(gate(x)) * up(x) for bias-free nn.Linear layers in one launch, or None
     for a call the kernels do not take."""
-    ws = _linear_weights(x, (gate, up))
+    ws = _linear_weights(x, (gate, up), glu=True)
     if ws is None or ws[0].shape != ws[1].shape:
         return None
     K, N = x.shape[-1], ws[0].shape[0]

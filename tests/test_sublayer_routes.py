@@ -43,6 +43,7 @@ def _taken(monkeypatch, device, current):
         raise RuntimeError("the library")
 
     monkeypatch.setattr(_ops.H, "load", library)
+    monkeypatch.setattr(_ops, "_linear_pays", lambda *a: True)
     lin = nn.Linear(128, 64, bias=False).to(BF)
     q, kv, pos = _fake((1, 4, 128), device), _fake((1, 4, 64), device), _fake((4, 64), device)
     out = [_ops._linear_weights(q, (lin,)) is not None,
@@ -239,3 +240,71 @@ def test_linear_widths(monkeypatch, n, taken):
     lin = nn.utils.skip_init(nn.Linear, 128, n, bias=False).to(BF)
     with torch.no_grad():
         assert (_ops._linear_weights(_fake((4, 128)), (lin,)) is not None) == taken
+
+
+PRODUCTS = [
+    # (rows, K, outputs, glu), whether the kernels are no slower than the library there
+    # 16 x 16 tiles: one a CU, more
+    ((64, 768, (768,), False), True), ((64, 6464, (1024,), False), True), ((64, 6496, (1024,), False), False),
+    ((64, 2560, (1536,), False), True), ((64, 2592, (1536,), False), False),
+    # 64 x 64 tiles: one a CU, more
+    ((512, 2048, (2048,), False), True), ((512, 2080, (2048,), False), False),
+    ((512, 1024, (2432,), False), True), ((512, 1536, (2432,), False), False),
+    # 128 x 64 tiles
+    ((512, 768, (6400,), False), True), ((2048, 2048, (768,), False), False),
+    # 128 x 128 tiles: one round, two
+    ((8192, 512, (1024,), False), True), ((2048, 512, (6400,), False), False),
+    ((8192, 768, (2048,), False), False), ((2048, 768, (6400,), False), False),
+    # 128 x 192 tiles, 256 x 256 tiles
+    ((8192, 768, (768,), False), True), ((8192, 2048, (768,), False), False),
+    ((4096, 768, (6400,), False), False),
+    # q, k, v
+    ((64, 768, (768, 384, 384), False), True), ((8192, 768, (768, 384, 384), False), True),
+    ((16384, 768, (768, 384, 384), False), True), ((65536, 768, (768, 384, 384), False), False),
+    ((16384, 1024, (1024, 1024, 1024), False), False), ((8192, 2048, (2048, 512, 512), False), False),
+    ((2930, 3296, (2496, 2496, 2496), False), False), ((4225, 768, (768, 384, 384), False), True),
+    ((300, 4096, (4096, 1024, 1024), False), True), ((3000, 4096, (4096, 1024, 1024), False), False),
+    # gate and up
+    ((64, 768, (2048, 2048), True), True), ((8192, 768, (2432, 2432), True), True),
+    ((8192, 2048, (6464, 6464), True), True), ((3000, 2048, (4096, 4096), True), False),
+    ((1024, 4096, (12928, 12928), True), False)]
+
+
+@pytest.mark.parametrize("size,pays", PRODUCTS)
+def test_products_go_where_they_are_faster(monkeypatch, size, pays):
+    M, K, ns, glu = size
+    calls, lib = [], _ops.H.load()
+
+    class Lib:
+        mhc_linear_pays = lib.mhc_linear_pays if hasattr(lib, "mhc_linear_pays") else None
+
+        def __getattr__(self, name):
+            calls.append(name)
+            raise RuntimeError(name)
+
+    class Layer(nn.Linear):  # what plain_module is told is an nn.Linear; the library's call
+        def __init__(self, n):
+            super().__init__(32, 4, bias=False, dtype=BF)
+            self.out_features = n
+            self.weight = nn.Parameter(_fake((n, K)), requires_grad=False)
+
+        def forward(self, x):
+            calls.append("torch")
+            return None
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(_ops, "plain_tensors", lambda *a: True)
+    monkeypatch.setattr(_ops, "plain_module", lambda *a: True)
+    monkeypatch.setattr(_ops.H, "load", lambda: Lib())
+    monkeypatch.setattr(_ops.H, "stream", lambda dev: 0)
+    monkeypatch.setattr(_ops.H, "dtype_tag", lambda t: 1)
+    x, mods = _fake((M, K)), [Layer(n) for n in ns]
+    with torch.no_grad():
+        try:
+            if glu:
+                taken = _ops.glu(x, *mods) is not None
+            else:
+                taken = (_ops.linear(x, mods[0]) if len(ns) == 1 else _ops.linears(x, *mods)) is not None
+        except RuntimeError:
+            taken = True
+    assert taken == pays and (not calls or calls == ["torch"] or pays), (taken, calls)
