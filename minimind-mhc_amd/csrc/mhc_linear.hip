@@ -199,9 +199,10 @@ hipError_t launch(const LinearArgs& a, hipStream_t s) {
 //     512 x 6400, 24.1 and 20.1), 128 x 192 to K = 1024 (8192 x 768 x 768 14.1 and 14.9,
 //     8192 x 1024 x 768 16.8 and 17.9, 12000 x 1536 x 768 32.8 and 28.7).  256 x 256 ones
 //     mostly lose (4096 x 768 x 6400 50 and 42).
-//   q, k, v: two launches less.  128 x 128 and 128 x 192 tiles while rounds x K is up to
-//     4096 (2048 rows, hidden 2048, 30.7 and 42.4; 12000 rows 157 and 141; 2930 x 7488 at K
-//     = 3296, two rounds, 186 and 180), 256 x 256 up to 2560
+//   q, k, v: two launches less.  128 x 128 tiles while rounds x K is up to 4096 (2048
+//     rows, hidden 2048, 30.7 and 42.4; 12000 rows 157 and 141), 128 x 192 up to 3072 (two
+//     rounds: 8192 x 2304 at K = 1536 54 and 71, 2051 x 8064 at K = 1984 84 and 74), 256 x
+//     256 up to 2560
 //     (16384 rows, hidden 768, 49.1 and 54.4; 65536 rows 187 and 167; 16384 x 3072 at K =
 //     1024, three rounds, 7% slower), the rest to K = 4096 (never slower).
 //   Gate and up: also two passes less.  128 x 128 to K = 1536 (1 to 170% faster, 5400 rows
@@ -213,7 +214,8 @@ bool linear_pays(const LinearArgs& a) {
   const int64_t rounds = (c.work + chip - 1) / chip;
   if (a.glu) return c.tile == Tile::k128x128 && a.K > 1536 ? rounds * a.K <= 4096 : a.K <= 3072;
   if (a.count > 1) {
-    if (c.tile == Tile::k128x128 || c.tile == Tile::k128x192) return rounds * a.K <= 4096;
+    if (c.tile == Tile::k128x128) return rounds * a.K <= 4096;
+    if (c.tile == Tile::k128x192) return rounds * a.K <= 3072;
     return c.tile == Tile::k256x256 ? rounds * a.K <= 2560 : a.K <= 4096;
   }
   switch (c.tile) {

@@ -262,7 +262,7 @@ PRODUCTS = [
     ((64, 768, (768, 384, 384), False), True), ((8192, 768, (768, 384, 384), False), True),
     ((16384, 768, (768, 384, 384), False), True), ((65536, 768, (768, 384, 384), False), False),
     ((16384, 1024, (1024, 1024, 1024), False), False), ((8192, 2048, (2048, 512, 512), False), False),
-    ((2930, 3296, (2496, 2496, 2496), False), False), ((4225, 768, (768, 384, 384), False), True),
+    ((2051, 1984, (2688, 2688, 2688), False), False), ((2930, 3296, (2496, 2496, 2496), False), False), ((4225, 768, (768, 384, 384), False), True),
     ((300, 4096, (4096, 1024, 1024), False), True), ((3000, 4096, (4096, 1024, 1024), False), False),
     # gate and up
     ((64, 768, (2048, 2048), True), True), ((8192, 768, (2432, 2432), True), True),
