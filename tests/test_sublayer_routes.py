@@ -308,3 +308,28 @@ def test_products_go_where_they_are_faster(monkeypatch, size, pays):
         except RuntimeError:
             taken = True
     assert taken == pays and (not calls or calls == ["torch"] or pays), (taken, calls)
+
+
+@pytest.mark.parametrize("tokens,hidden,inter,experts,topk,taken", [
+    (8192, 4096, 14336, 4, 1, False), (8188, 4096, 14336, 4, 1, True), (8192, 4096, 8192, 4, 1, True),
+    (8192, 8192, 8192, 4, 1, False), (1, 8192, 8192, 4, 1, True), (65536, 2048, 6464, 4, 2, True)])
+def test_experts_go_where_they_are_faster(monkeypatch, tokens, hidden, inter, experts, topk, taken):
+    """Wide experts with many rows each: the library's products, in the loop."""
+    def proj(n, k):
+        return types.SimpleNamespace(out_features=n, in_features=k, bias=None, weight=_fake((n, k)))
+
+    def library():
+        raise RuntimeError("the library")
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(_ops, "plain_tensors", lambda *a: True)
+    monkeypatch.setattr(_ops, "plain_module", lambda *a: True)
+    monkeypatch.setattr(_ops.H, "load", library)
+    mods = [types.SimpleNamespace(gate_proj=proj(inter, hidden), up_proj=proj(inter, hidden),
+                                  down_proj=proj(hidden, inter)) for _ in range(experts)]
+    with torch.no_grad():
+        try:
+            got = _ops.moe_experts(mods, _fake((tokens, hidden)), _fake((tokens, experts)), topk, True) is not None
+        except RuntimeError:
+            got = True
+    assert got == taken
