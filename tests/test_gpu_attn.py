@@ -58,7 +58,10 @@ def _close(want, got, bar):
 @pytest.mark.parametrize("hd,heads,kv,dtype,B,T", [
     (96, 8, 4, BF, 2, 1), (96, 8, 4, BF, 1, 63), (96, 8, 4, BF, 1, 64), (96, 8, 4, BF, 3, 65),
     (64, 4, 4, BF, 2, 127), (64, 3, 1, F16, 1, 129), (128, 8, 2, BF, 1, 257), (128, 4, 1, F16, 2, 96),
-    (96, 6, 2, BF, 1, 200), (96, 8, 4, F16, 2, 333)])
+    (96, 6, 2, BF, 1, 200), (96, 8, 4, F16, 2, 333),
+    # more workgroups than the 256 CUs: a part-filled second round (which runs backwards)
+    # and a third one, of paired heads and of single ones
+    (96, 8, 4, BF, 5, 1000), (64, 8, 2, BF, 16, 520), (64, 8, 8, BF, 6, 700), (64, 6, 2, F16, 16, 700)])
 def test_prefill(dev, hd, heads, kv, dtype, B, T):
     m = _layer(hd, heads, kv, dtype)
     x, pos = torch.randn(B, T, 128).to(dtype), _pos(hd, 0, T, dtype)
@@ -78,7 +81,9 @@ def test_prefill(dev, hd, heads, kv, dtype, B, T):
     (96, 8, 4, BF, 1, 1, True), (96, 8, 4, BF, 3, 15, True), (96, 8, 4, BF, 2, 16, False),
     (64, 4, 4, BF, 2, 17, True), (128, 8, 2, BF, 1, 1000, True), (64, 3, 1, F16, 5, 47, True),
     (96, 8, 4, F16, 64, 130, True), (128, 4, 1, F16, 1, 333, False), (96, 6, 2, BF, 300, 33, True),
-    (64, 6, 6, BF, 2, 95, True), (96, 3, 3, BF, 1, 129, True)])
+    (64, 6, 6, BF, 2, 95, True), (96, 3, 3, BF, 1, 129, True),
+    # more than 64 partial results a head
+    (96, 8, 4, BF, 1, 4000, True), (64, 3, 1, F16, 1, 2050, False)])
 def test_decode(dev, hd, heads, kv, dtype, B, S, cache):
     m = _layer(hd, heads, kv, dtype)
     x, pos = torch.randn(B, 1, 128).to(dtype), _pos(hd, S, 1, dtype)
