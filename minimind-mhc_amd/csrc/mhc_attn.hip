@@ -265,6 +265,12 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
         *reinterpret_cast<U32x4*>(vo + obase + row * orow + ocol[p]) = vn[p];
       }
     }
+    // rows that are not there: 0 x infinity would be NaN (here and not as a select on vc: 176
+    // registers instead of 160 at head_dim 96 cost the third wave a SIMD, 5 us a launch)
+    if ((t + 1) * rows > a.S)
+#pragma unroll
+      for (int p = 0; p < NC; ++p)
+        if (t * rows + prow[p] >= a.S) *reinterpret_cast<U32x4*>(&vl[buf][lpos[p]]) = U32x4{};
     if (t + 1 < t1) load(t + 1);
     __syncthreads();
     U32x4 kc[NC], vc[NC];
@@ -273,12 +279,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
       kc[c] = *reinterpret_cast<const U32x4*>(&kl[buf][(wave * 16 + r) * LST + 32 * c + 8 * g]);
       vc[c] = *reinterpret_cast<const U32x4*>(&vl[buf][(wave * 16 + r) * LST + 32 * c + 8 * g]);
     }
-    const bool ok = t * rows + sub + r < a.S;
-    if ((t + 1) * rows > a.S && !ok) {  // a row that is not there: 0 x infinity would be NaN
-#pragma unroll
-      for (int c = 0; c < NC; ++c) vc[c] = U32x4{};
-    }
-    step(kc, vc, ok);
+    step(kc, vc, t * rows + sub + r < a.S);
   }
   if (has_new) {  // the new position: one row, in the lanes with r == 0
     U32x4 kc[NC], vc[NC];
@@ -286,7 +287,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
                                a.cos, a.sin, a.k_eps, g, kc);
     const uint16_t* vp = static_cast<const uint16_t*>(a.v) + (b * a.kv_heads + kvh) * HD + 8 * g;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) vc[c] = r == 0 ? ld16(vp + 32 * c) : U32x4{};
+    for (int c = 0; c < NC; ++c) vc[c] = ld16(vp + 32 * c);
     if (ko && r == 0) {
       const int64_t o = obase + a.S * orow + kvh * HD + 8 * g;
 #pragma unroll
@@ -294,6 +295,11 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnDecodeArgs a) {
 #pragma unroll
       for (int c = 0; c < NC; ++c) *reinterpret_cast<U32x4*>(vo + o + 32 * c) = vc[c];
     }
+    const uint32_t keep = r == 0 ? ~0u : 0u;  // the other lanes hold no position
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) vc[c].v[j] &= keep;
     step(kc, vc, r == 0);
   }
   // merge the 16 positions of the row
@@ -445,10 +451,18 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
       const int piece = p * 256 + tid;
       const int row = piece / (HD / 8);
       const int col = (piece % (HD / 8)) * 8;
-      if (s0 + KT > T && s0 + row >= T) vr[p] = U32x4{};  // no such row: 0 x infinity would be NaN
       *reinterpret_cast<U32x4*>(&ks[buf][row * KST + col]) = kr[p];
       *reinterpret_cast<U32x4*>(&vs[buf][row * VST + col]) = vr[p];
     }
+    // rows that are not there: 0 x infinity would be NaN (stores in a uniform branch: as
+    // selects on every tile's registers 1.7% of the layer)
+    if (s0 + KT > T)
+#pragma unroll
+      for (int p = 0; p < PPT; ++p) {
+        const int piece = p * 256 + tid;
+        const int row = piece / (HD / 8);
+        if (s0 + row >= T) *reinterpret_cast<U32x4*>(&vs[buf][row * VST + (piece % (HD / 8)) * 8]) = U32x4{};
+      }
   };
   load(0);
   U32x4 qb[2][NC];
