@@ -649,19 +649,23 @@ def sinkhorn_bwd(m: torch.Tensor, g: torch.Tensor, iters: int, eps: float,
 # transform, no tracing or compiling, no dispatch or function mode, no autocast, and
 # submodules that nobody has hooked or patched.
 
+# torch.cuda.current_device also looks whether torch's GPU side is set up, which a GPU
+# tensor answers: 0.3 us a call.
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+
+
 def on_current_device(t: torch.Tensor) -> bool:
     """Whether t, a GPU tensor, lies on the device the library would launch on.  Its entry points set no
     device, and a device's default stream is handle 0 on every device, so for a tensor
     of another one the launch would go to the wrong GPU; torch ops set the device."""
-    return t.get_device() == torch.cuda.current_device()
+    return t.get_device() == _current_device()
 
 
 def _function_modes() -> bool:
-    """Whether a torch-function mode could see or replace the torch ops.  The one that
-    torch.set_default_device and `with torch.device(...)` leave on the stack only changes
-    factory calls without a device, of which the sublayers make none."""
-    return (_len_torch_function_stack() > 0
-            and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
+    """Whether one of the torch-function modes on the stack could see or replace the torch
+    ops.  The one that torch.set_default_device and `with torch.device(...)` leave there
+    only changes factory calls without a device, of which the sublayers make none."""
+    return any(type(m) is not DeviceContext for m in _get_current_function_mode_stack())
 
 
 def plain_call() -> bool:
@@ -670,7 +674,8 @@ def plain_call() -> bool:
     return not (torch.compiler.is_compiling() or not CAN_TELL
                 or torch.is_grad_enabled() or torch.is_autocast_enabled("cuda")
                 or forward_ad._current_level >= 0
-                or _len_torch_dispatch_stack() > 0 or _function_modes()
+                or _len_torch_dispatch_stack() > 0
+                or (_len_torch_function_stack() > 0 and _function_modes())
                 or peek_interpreter_stack() is not None
                 or torch.jit.is_tracing())
 
@@ -683,11 +688,18 @@ def plain_module(m: torch.nn.Module, kind: type) -> bool:
             and not (_global_forward_hooks or _global_forward_pre_hooks))
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
 def plain_tensors(dtype: torch.dtype, dev: torch.device, *ts) -> bool:
-    """Whether every tensor is a plain one of that dtype on that device, its data
+    """Whether every tensor is a plain one of that dtype on that GPU, its data
     16-byte aligned."""
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == dtype
-               and t.device == dev and t.data_ptr() % 16 == 0 for t in ts)
+    index = dev.index
+    for t in ts:
+        if (type(t) not in _PLAIN or t.dtype != dtype or not t.is_cuda or t.get_device() != index
+                or t.data_ptr() % 16):
+            return False
+    return True
 
 
 # Multiply-adds past which one linear layer is the library's at every K.
@@ -702,13 +714,16 @@ def _linear_pays(M: int, K: int, ns: tuple, glu: bool = False) -> bool:
     return bool(H.load().mhc_linear_pays((ctypes.c_int * len(ns))(*ns), len(ns), M, K, int(glu)))
 
 
+_HALF = (torch.bfloat16, torch.float16)
+
+
 def _linear_weights(x: torch.Tensor, mods, glu: bool = False, closely: bool = True):
     """The weights of bias-free nn.Linear layers the kernels can apply to x, or None; also
     None where the library is faster (not closely: where it is at every K).  That is asked
     before what takes longer to look at: a call left to torch waits for this."""
     if not isinstance(x, torch.Tensor):  # an fx Proxy: the torch ops are traced
         return None
-    if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or not plain_call():
+    if not x.is_cuda or x.dtype not in _HALF or not plain_call():
         return None
     total = x.numel()
     if x.dim() < 2 or total == 0:
@@ -716,8 +731,9 @@ def _linear_weights(x: torch.Tensor, mods, glu: bool = False, closely: bool = Tr
     K = x.shape[-1]
     if K % 32 != 0 or K > 1 << 22:
         return None
-    ns = tuple([getattr(m, "out_features", None) for m in mods])
-    if None in ns:
+    try:
+        ns = tuple([m.out_features for m in mods])
+    except AttributeError:
         return None
     if not (_linear_pays(total // K, K, ns, glu) if closely else total * ns[0] <= LINEAR_MAX_MACS):
         return None
@@ -783,7 +799,7 @@ def attn_route(m, q, k, v, position_embeddings, past) -> Optional[str]:
     projections (q, k, v): "prefill", "decode", or None (the torch ops).
     q [B, T, heads * head_dim]; k, v [B, T, kv_heads * head_dim]."""
     H_, KV, hd = m.n_local_heads, m.n_local_kv_heads, m.head_dim
-    if (not q.is_cuda or q.dtype not in (torch.bfloat16, torch.float16) or hd not in ATTN_HEAD_DIMS
+    if (not q.is_cuda or q.dtype not in _HALF or hd not in ATTN_HEAD_DIMS
             or q.dim() != 3 or H_ % KV != 0 or not plain_call() or not on_current_device(q)):
         return None
     B, T, _ = q.shape
@@ -875,7 +891,7 @@ def moe_experts(experts, x: torch.Tensor, probs: torch.Tensor, topk: int, norm_t
     and down_proj (plain nn.Linear without bias) and SiLU between them; probs
     [M, experts], the router's softmax; zero: a tensor of x's type whose one element
     the last launch sets to 0."""
-    if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or not plain_call()
+    if (not x.is_cuda or x.dtype not in _HALF or not plain_call()
             or not on_current_device(x) or x.dim() != 2 or x.shape[0] == 0 or not x.is_contiguous()
             or probs.shape != (x.shape[0], len(experts)) or not probs.is_contiguous()):
         return None

@@ -33,7 +33,7 @@ def _fake(shape, device="cuda:1"):
 def _taken(monkeypatch, device, current):
     """What the rules say to calls that nothing but the device speaks against; with the
     device right, they get as far as the first look at the data."""
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: current)
+    monkeypatch.setattr(_ops, "_current_device", lambda: current)
     monkeypatch.setattr(_ops, "plain_tensors", lambda *a: True)
     attn, moe = Attention(_cfg()).to(BF).eval(), MOEFeedForward(_cfg()).to(BF).eval()
     seen = []
@@ -76,7 +76,7 @@ def test_another_device_current_runs_torch_ops(dev, monkeypatch):
         for m in (ff, moe, attn):
             m.to(dev).to(BF).eval()
         want = [ff(x), moe(x), attn(x, pos, None, True)[0]]
-        monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+        monkeypatch.setattr(_ops, "_current_device", lambda: 1)
         q, k, v = attn.q_proj(x), attn.k_proj(x), attn.v_proj(x)
         assert _ops.linears(x, attn.q_proj) is None and _ops.glu(x, ff.gate_proj, ff.up_proj) is None
         assert _ops.attn_route(attn, q, k, v, pos, None) is None
@@ -221,7 +221,7 @@ def test_stream_on_a_torch_without_the_raw_handle(monkeypatch):
 
 def test_decode_past_the_librarys_limit_is_torchs(monkeypatch):
     """mhc_attn_decode_fwd takes up to 2^20 sequences x kv heads and raises past that."""
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(_ops, "_current_device", lambda: 1)
     monkeypatch.setattr(_ops, "plain_tensors", lambda *a: True)
     attn = Attention(_cfg()).to(BF).eval()
     pos = _fake((1, 64))
@@ -235,7 +235,7 @@ def test_decode_past_the_librarys_limit_is_torchs(monkeypatch):
 @pytest.mark.parametrize("n,taken", [(0, False), (2, False), (4, True)])
 def test_linear_widths(monkeypatch, n, taken):
     """mhc_linear_fwd takes multiples of four output features, and none of zero."""
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(_ops, "_current_device", lambda: 1)
     monkeypatch.setattr(_ops, "plain_tensors", lambda *a: True)
     lin = nn.utils.skip_init(nn.Linear, 128, n, bias=False).to(BF)
     with torch.no_grad():
@@ -292,7 +292,7 @@ def test_products_go_where_they_are_faster(monkeypatch, size, pays):
             calls.append("torch")
             return None
 
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(_ops, "_current_device", lambda: 1)
     monkeypatch.setattr(_ops, "plain_tensors", lambda *a: True)
     monkeypatch.setattr(_ops, "plain_module", lambda *a: True)
     monkeypatch.setattr(_ops.H, "load", lambda: Lib())
@@ -321,7 +321,7 @@ def test_experts_go_where_they_are_faster(monkeypatch, tokens, hidden, inter, ex
     def library():
         raise RuntimeError("the library")
 
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(_ops, "_current_device", lambda: 1)
     monkeypatch.setattr(_ops, "plain_tensors", lambda *a: True)
     monkeypatch.setattr(_ops, "plain_module", lambda *a: True)
     monkeypatch.setattr(_ops.H, "load", library)
