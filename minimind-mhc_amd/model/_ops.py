@@ -807,6 +807,8 @@ def attn_route(m, q, k, v, position_embeddings, past) -> Optional[str]:
         return None
     if not (plain_module(m.q_norm, torch.nn.RMSNorm) and plain_module(m.k_norm, torch.nn.RMSNorm)):
         return None
+    if m.q_norm.eps is None or m.k_norm.eps is None:  # torch's own choice, which its versions differ in
+        return None
     cos, sin = position_embeddings
     gq, gk = m.q_norm.weight, m.k_norm.weight
     if gq is None or gk is None or not plain_tensors(q.dtype, q.device, q, k, v, gq, gk, cos, sin):
@@ -829,10 +831,6 @@ def attn_route(m, q, k, v, position_embeddings, past) -> Optional[str]:
     return "decode"
 
 
-def _rms_eps(norm, dtype) -> float:
-    return float(norm.eps) if norm.eps is not None else float(torch.finfo(dtype).eps)
-
-
 def attn_prefill(m, q, k, v, position_embeddings):
     """(attention output [B, T, heads * head_dim], normed and rotated k); the
     call is one attn_route calls "prefill"."""
@@ -843,7 +841,7 @@ def attn_prefill(m, q, k, v, position_embeddings):
     H.check(H.load().mhc_attn_prefill_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), m.q_norm.weight.data_ptr(),
         m.k_norm.weight.data_ptr(), cos.data_ptr(), sin.data_ptr(), kr.data_ptr(), out.data_ptr(),
-        B, T, H_, KV, hd, H.dtype_tag(q), _rms_eps(m.q_norm, q.dtype), _rms_eps(m.k_norm, q.dtype),
+        B, T, H_, KV, hd, H.dtype_tag(q), float(m.q_norm.eps), float(m.k_norm.eps),
         H.stream(q.device)), "mhc_attn_prefill_fwd")
     return out, kr
 
@@ -870,7 +868,7 @@ def attn_decode(m, q, k, v, position_embeddings, past, use_cache: bool):
         pk.data_ptr(), *pk.stride()[:3], pv.data_ptr(), *pv.stride()[:3],
         grown[0].data_ptr() if grown else None, grown[1].data_ptr() if grown else None,
         out.data_ptr(), H.ptr(ws), max(nbytes, 0), B, S, H_, KV, hd, H.dtype_tag(q),
-        _rms_eps(m.q_norm, q.dtype), _rms_eps(m.k_norm, q.dtype), H.stream(q.device)),
+        float(m.q_norm.eps), float(m.k_norm.eps), H.stream(q.device)),
         "mhc_attn_decode_fwd")
     return out, grown
 

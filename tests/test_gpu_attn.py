@@ -173,6 +173,25 @@ def test_prefill_infinite_value(dev, hd, heads, kv, dtype, T):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name", ["q_norm", "k_norm"])
+def test_norm_without_eps(dev, name):
+    """nn.RMSNorm(eps=None) takes an epsilon of torch's choosing (2^-23 for bf16 input,
+    not bf16's own 2^-7): inputs small enough to tell give what torch's ops give."""
+    m = _layer(96, 8, 4, BF).to(dev)
+    getattr(m, name).eps = None
+    with torch.no_grad():
+        getattr(m, name[0] + "_proj").weight.mul_(0.01)
+        for T, past in ((70, None), (1, tuple(torch.randn(2, 9, 4, 96, device=dev).to(BF) for _ in range(2)))):
+            x = torch.randn(2, T, 128, device=dev).to(BF)
+            pos = tuple(t.to(dev) for t in _pos(96, 9 if past else 0, T, BF))
+            got = m(x, pos, past, True)
+            with torch.amp.autocast("cuda", enabled=True, dtype=BF):  # not the kernels' call
+                want = m(x, pos, past, True)
+            _close(want[0], got[0], _bar(BF))
+            _close(want[1][0], got[1][0], _bar(BF))
+
+
+@pytest.mark.gpu
 def test_calls_left_to_torch(dev):
     """Calls the kernels do not take, or that would tell: the route is None."""
     m = _layer(96, 8, 4, BF).to(dev)
