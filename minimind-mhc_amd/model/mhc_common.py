@@ -24,20 +24,16 @@ def _is_pow2(n: int) -> bool:
 def fusable_norm(norm, dim: int, x: torch.Tensor) -> bool:
     """True when an nn.RMSNorm over `dim` can run inside a HIP launch for this
     call: grad mode off (torch.no_grad / inference_mode) and an affine norm
-    over exactly (dim,).  With grad mode on the norm stays a separate op even
-    when nothing visible here requires grad: the sublayer F is opaque, and the
-    fused launches record no autograd graph that gradients to F's parameters
-    could flow through."""
-    if not isinstance(norm, nn.RMSNorm) or norm.weight is None:
+    over exactly (dim,) with an eps (None is torch's own choice: 2^-23 for 16-bit
+    inputs here, the type's own epsilon in its documentation).  With grad mode on
+    the norm stays a separate op even when nothing visible here requires grad: the
+    sublayer F is opaque, and the fused launches record no autograd graph that
+    gradients to F's parameters could flow through."""
+    if not isinstance(norm, nn.RMSNorm) or norm.weight is None or norm.eps is None:
         return False
     if tuple(norm.normalized_shape) != (dim,) or not x.is_cuda:
         return False
     return not torch.is_grad_enabled()
-
-
-def norm_eps(norm: nn.RMSNorm, x: torch.Tensor) -> float:
-    """nn.RMSNorm's eps (None means the dtype's machine epsilon, as torch uses)."""
-    return float(norm.eps) if norm.eps is not None else float(torch.finfo(x.dtype).eps)
 
 
 class _StreamExpandFn(_ops.GradAwareFunction):
@@ -74,7 +70,7 @@ class StreamExpand(nn.Module):
         if fusable_norm(in_norm, self.dim, x):
             ssq = (chain.buffer(x, self.n, self.dim, rows=x.numel() // self.dim)
                    if chain is not None and self.n > 1 else None)
-            out = _ops.expand_norm(x, in_norm.weight, norm_eps(in_norm, x), self.n, ssq_out=ssq)
+            out = _ops.expand_norm(x, in_norm.weight, float(in_norm.eps), self.n, ssq_out=ssq)
             return chain.put(out, ssq) if chain is not None else out
         out = self(in_norm(x))
         return chain.put(out, None) if chain is not None else out
@@ -168,7 +164,7 @@ class MHCHead(nn.Module):
                           if self.n > 1 else None)
                 out, _, _ = _ops.head(x_flat, self.phi_weight, packed, self.alpha, self.bias,
                                       self.n, self.dim, self.pre_eps, self.eps,
-                                      norm=(out_norm.weight, norm_eps(out_norm, x_flat)), ssq=ssq)
+                                      norm=(out_norm.weight, float(out_norm.eps)), ssq=ssq)
                 return out.view(*x_flat.shape[:-1], self.dim)
             return out_norm(self(x_flat, chain=chain))
         if self.n == 1:

@@ -22,7 +22,7 @@ import torch.nn as nn
 
 from . import _ops
 from . import _hip as H
-from .mhc_common import fusable_norm, norm_eps
+from .mhc_common import fusable_norm
 
 
 def _is_pow2(n: int) -> bool:
@@ -239,7 +239,7 @@ class MHCConnection_Fused(nn.Module):
                               self.alpha_post, self.bias_post, self.alpha_res, self.bias_res,
                               self.n, self.dim, self.post_mult_value, self.pre_eps, self.eps,
                               self.sinkhorn_iters, self.sinkhorn_eps, ssq=ssq,
-                              norm=(in_norm.weight, norm_eps(in_norm, x_flat)) if fused else None)
+                              norm=(in_norm.weight, float(in_norm.eps)) if fused else None)
             B, L, NC = x_flat.shape
             f_out = sublayer_fn(o["sub_in"].view(B, L, self.dim))
             out = _ops.post(x_flat, o["h_res"], o["h_post"], f_out, self.n, self.dim,

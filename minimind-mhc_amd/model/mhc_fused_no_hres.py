@@ -15,7 +15,7 @@ import torch.nn as nn
 
 from . import _ops
 from . import _hip as H
-from .mhc_common import fusable_norm, norm_eps
+from .mhc_common import fusable_norm
 
 
 def _is_pow2(n: int) -> bool:
@@ -129,7 +129,7 @@ class MHCConnection_FusedNoHres(nn.Module):
             o = _ops.pre_nohres(x_flat, self.phi_weight, packed, self.alpha_pre, self.bias_pre,
                                 self.alpha_post, self.bias_post, self.n, self.dim,
                                 self.post_mult_value, self.pre_eps, self.eps, ssq=ssq,
-                                norm=(in_norm.weight, norm_eps(in_norm, x_flat)) if fused else None)
+                                norm=(in_norm.weight, float(in_norm.eps)) if fused else None)
             B, L, NC = x_flat.shape
             f_out = sublayer_fn(o["sub_in"].view(B, L, self.dim))
             out = _ops.post(x_flat, None, o["h_post"], f_out, self.n, self.dim,

@@ -242,3 +242,25 @@ def test_expand_norm_rejects_wrong_gain(dev):
     x = torch.randn(1, 4, 64, device=dev, dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="norm weight"):
         _ops.expand_norm(x, torch.ones(32, device=dev, dtype=torch.bfloat16), 1e-6, 4)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_norm_without_eps_is_torchs(dev, dtype):
+    """nn.RMSNorm(eps=None) takes an epsilon of torch's choosing: without grad mode each
+    module gives what the norm by itself gives, on streams small enough to tell."""
+    from model.mhc_common import MHCHead, StreamExpand
+    from model.mhc_fused import MHCConnection_Fused
+    from model.mhc_fused_no_hres import MHCConnection_FusedNoHres
+    torch.manual_seed(0)
+    norm = torch.nn.RMSNorm(64, eps=None).to(dev).to(dtype)
+    x = (torch.randn(1, 9, 256, device=dev) * 0.01).to(dtype)
+    with torch.no_grad():
+        for cls in (MHCConnection_Fused, MHCConnection_FusedNoHres):
+            m, seen = cls(4, 64).to(dev).to(dtype), []
+            m(x, lambda z: seen.append(z) or z, in_norm=norm)
+            m(x, lambda z: seen.append(norm(z)) or z)
+            assert torch.equal(*seen)
+        head = MHCHead(4, 64).to(dev).to(dtype)
+        assert torch.equal(head(x, out_norm=norm), norm(head(x)))
+        e, z = StreamExpand(4, 64), x[..., :64].contiguous()
+        assert torch.equal(e.forward_normed(z, norm), e(norm(z)))
