@@ -916,8 +916,11 @@ def moe_experts(experts, x: torch.Tensor, probs: torch.Tensor, topk: int, norm_t
     nbytes = lib.mhc_moe_workspace_bytes(M, D, inter, len(experts), topk)
     if nbytes < 0:
         return None
+    try:  # every expert's rows at once; the loop needs one expert's at a time
+        work = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    except torch.OutOfMemoryError:
+        return None
     out = torch.empty_like(x)
-    work = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     ptrs = [(ctypes.c_void_p * len(w))(*[t.data_ptr() for t in w]) for w in ws]
     H.check(lib.mhc_moe_fwd(x.data_ptr(), probs.data_ptr(), *ptrs, out.data_ptr(), H.ptr(zero),
                             work.data_ptr(), nbytes, M, D, inter, len(experts), topk,

@@ -333,3 +333,24 @@ def test_experts_go_where_they_are_faster(monkeypatch, tokens, hidden, inter, ex
         except RuntimeError:
             got = True
     assert got == taken
+
+
+@pytest.mark.gpu
+def test_experts_without_room_for_all_rows_loop(dev, monkeypatch):
+    """The kernels hold every expert's rows at once: where that does not fit, the loop
+    over the experts, which needs less, runs as it did."""
+    torch.manual_seed(0)
+    moe, x = MOEFeedForward(_cfg()).to(dev).to(BF).eval(), torch.randn(1, 40, 128, device=dev).to(BF)
+    empty = torch.empty
+
+    def full(*args, **kwargs):
+        if kwargs.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no room")
+        return empty(*args, **kwargs)
+
+    with torch.no_grad():
+        want = moe(x)
+        monkeypatch.setattr(torch, "empty", full)
+        got = moe(x)
+    assert float(moe.aux_loss) == 0
+    assert float((want.float() - got.float()).abs().max()) <= 6 * 2.0 ** -9 * float(want.float().abs().max())
