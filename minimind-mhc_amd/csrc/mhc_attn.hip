@@ -121,10 +121,12 @@ __global__ __launch_bounds__(256) void k_norm_rope_kernel(KRopeArgs a) {
 //     32 or 64 positions, loaded (non-temporal: read once) and stored as their bytes
 //     run, whole lines across the workgroup, and regrouped through LDS.  64
 //     sequences, 4 kv heads of 96, S = 2048, grown cache, 403 MB: 72.6 us, 5.55 TB/s
-//     (a large torch copy runs at 4.9).  Each wave loading and storing its own head's
-//     rows 80 us (cached loads 97, non-temporal stores 101), in the operand layout
-//     (16 rows x 64 bytes) 94; here non-temporal stores 85.  The torch ops (cat, two
-//     expanded copies, SDPA, norms and rotary) took 670 us.
+//     (a 1 GiB torch copy runs at 5.07); the same over eight caches in turn (1.6 GB)
+//     and with eight grown ones kept, 85 between the model's other launches.  Each
+//     wave loading and storing its own head's rows 80 us (cached loads 97,
+//     non-temporal stores 101), in the operand layout (16 rows x 64 bytes) 94; here
+//     non-temporal stores 85.  The torch ops (cat, two expanded copies, SDPA, norms
+//     and rotary) took 670 us.
 //   * The maximum is raised (and the sums rescaled) only when some score exceeds
 //     it by more than 2^8 in the exponent; fp32 sums lose nothing by that.
 constexpr float kLazyMax = 8.f;
@@ -395,16 +397,16 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(AttnDecodeArgs a) {
 //     contraction runs over positions 16 (j / 4) + 4 g + j % 4 of each 32).
 //   * V^T is read from the row-major tile by the transposing LDS load
 //     (ds_read_b64_tr_b16: a 16-lane group gets columns of 4 rows x 16).
-//   * Row strides of HD + 8 (K) and HD + 16 (V) elements spread 16 rows over all
-//     64 banks.
+//   * Row strides of HD + 8 (K) and HD + 16 (V) elements spread the 16 rows of a read
+//     over all 64 banks; with the tile's stores, 31% of the LDS cycles are conflicts.
 //   * Tiles above the diagonal are skipped; the workgroups with the longest rows
 //     start first.  The maximum is raised lazily as in the decode step.
 //   * Each wave norms and rotates its own q rows (a pass over q less).
 //   * Only the tiles on the diagonal compare positions (a uniform branch: as selects on
 //     every score 37 us, a fifth of the loop's VALU work).
-// 8 sequences of 1024, 8 query / 4 kv heads of 96: 34 us with the norms and
-// rotary of q, and 6 us for k; torch took 92 us for SDPA (with expanded k, v) and
-// 200 us for the norms, rotary and expanded copies.
+// 8 sequences of 1024, 8 query / 4 kv heads of 96: 34 us with the norms and rotary of
+// q (matrix cores busy 22% of the time, the VALU 48%), and 5 us for k; torch took 92 us
+// for SDPA (with expanded k, v) and 200 us for the norms, rotary and expanded copies.
 template <bool F16, int HD, int HP>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a) {
   constexpr int NC = HD / 32, ND = HD / 16, KT = 64;

@@ -130,10 +130,13 @@ __device__ __forceinline__ float silu_mul(float z, float u) {
   return z * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-kLog2e * z)) * u;
 }
 
-// Which tile a product of that many rows and columns takes: BM x BN of GemmTile.
+// Which tile a product of that many rows and columns takes: BM x BN of GemmTile.  The
+// lines come from these sizes; the counts 192 and (linear layers) 448 are tiles on the
+// 256 CUs they were measured on.
 //   256 x 256: one workgroup a CU, so only for rounds of the chip that are nearly full.
 //     8192 x 6400, K = 768 (800 tiles, 3.1 of 4 rounds): 97 us, 128 x 192 tiles 107;
-//     gate and up of 8192 x 2048 (512 tiles): 52.1, 128 x 128 tiles 61.0; 8192 x 1536
+//     gate and up of 8192 x 2048 (512 tiles): 52.1, 128 x 128 tiles 61.0; of 8 routed
+//     experts (16384 rows x 1024, 544 tiles, 2.1 of 3 rounds): 72.4 and 70.8; 8192 x 1536
 //     (192 tiles, under one round): 26.0 against 22.2 for 128 x 192.
 //   128 x 192: where a tile a CU is left and no column is padding that 128 would not
 //     have.  8192 x 1536: 22.2 us, 128 x 128 tiles 24.7; 8192 x 768 (256 tiles) 14.6

@@ -110,8 +110,11 @@ __global__ __launch_bounds__(kRouteTok) void moe_group_kernel(MoeArgs a) {
 //     in its L2).
 // 8192 tokens, 8 experts, top 2, 768 x 1024: 71 us for gate and up (128 x 128 tiles, 51.5
 // GFLOP, 725 TFLOP/s; 77 with 32-column slices and stores from the accumulators), 41 us
-// for down (128 x 192 tiles, 25.8 GFLOP, 629 TFLOP/s; 47 before).  The dense layer's rows
-// take 56 and 27 us: the rest is the gathered rows and the experts' partly filled tiles.
+// for down (128 x 192 tiles, 25.8 GFLOP, 629 TFLOP/s; 47 before).  As many rows of a dense
+// layer take 56 and 27 us, on 512 whole tiles each.  The experts' part-filled last tiles
+// are 3% of the operations, but they take gate and up just past whole rounds of the chip
+// (2112 tiles, 4.1 rounds of two a CU; 544 of 256 x 256, 2.1 rounds, 72 us); the gathered
+// rows cost no more traffic (113 MB read either way).
 // The layer's loop over experts took 1.6 ms, of which library products were 290 us.
 template <bool F16, typename G, bool GLU>
 __global__ __launch_bounds__(G::THREADS, G::WAVES) void moe_gemm_kernel(MoeArgs a) {
